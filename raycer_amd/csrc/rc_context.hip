@@ -222,9 +222,9 @@ extern "C" int rc_set_tuning(rc_ctx* c, const rc_tuning* t) {
         return rc_host_fail(RC_ERR_INVALID, "rc_set_tuning: spp_per_pass must be 0 (automatic) or in [1, 64]");
     if (t->blocks_per_cu == 0 || t->blocks_per_cu > 64)
         return rc_host_fail(RC_ERR_INVALID, "rc_set_tuning: blocks_per_cu must be in [1, 64]");
-    if (t->stack_limit > uint32_t(rcd::kOnChipStack))
+    if (t->stack_limit > uint32_t(rcd::kStackLimitMax))
         return rc_host_fail(RC_ERR_INVALID, "rc_set_tuning: stack_limit must be 0 (all) or in [1, " +
-                                                std::to_string(rcd::kOnChipStack) + "]");
+                                                std::to_string(rcd::kStackLimitMax) + "]");
     if (t->park_steps > 1024)
         return rc_host_fail(RC_ERR_INVALID, "rc_set_tuning: park_steps must be 0 (never park) or in [1, 1024]");
     c->tuning = *t;
@@ -269,7 +269,8 @@ float round_up(double x) {
 // smallest power of two 2^e with 253 * 2^e >= the node's extent and 2^e >= 8
 // ulps of its largest coordinate; children are quantized one unit outward on
 // each side, so the decoded box origin + q * 2^e contains the exact one with a
-// unit to spare, which covers the traversal's rounding of the decode.
+// unit to spare, which covers the traversal's rounding of the decode (the
+// node's own lower bounds, q = 0, are exact).
 void quantize_node(const NodeRec* r, QNode& q) {
     std::memset(&q, 0, sizeof(q));
     double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -280,8 +281,6 @@ void quantize_node(const NodeRec* r, QNode& q) {
             hi[a] = std::max(hi[a], double(r[k].hi[a]));
         }
     }
-    int ebias[3];
-    double scale[3];
     for (int a = 0; a < 3; ++a) {
         if (!(lo[a] <= hi[a])) lo[a] = hi[a] = 0.0;  // no child: any box
         const double ext = hi[a] - lo[a], mag = std::max(std::fabs(lo[a]), std::fabs(hi[a]));
@@ -290,36 +289,27 @@ void quantize_node(const NodeRec* r, QNode& q) {
         if (mag > 0.0) e = std::max(e, int(std::floor(std::log2(mag))) - 23 + 3);
         while (std::ldexp(253.0, e) < ext) ++e;  // guard log2 rounding
         e = std::min(e, 127);
-        ebias[a] = e + 127;
-        scale[a] = std::ldexp(1.0, e);
+        q.scale[a] = float(std::ldexp(1.0, e));
         q.origin[a] = float(lo[a]);  // lo is a float (a child's bound)
     }
-    q.exps = uint32_t(ebias[0]) | (uint32_t(ebias[1]) << 8) | (uint32_t(ebias[2]) << 16);
     for (int k = 0; k < kWidth; ++k) {
         const NodeRec& c = r[k];
-        uint32_t meta;
-        if (c.count == kEmptyChild) {
-            meta = 0xFFu;
-        } else {
-            meta = c.count;  // 0 interior, else 1..31 triangles
-            for (int a = 0; a < 3; ++a) {
-                double ql = std::floor((double(c.lo[a]) - double(q.origin[a])) / scale[a]) - 1.0;
-                double qh = std::ceil((double(c.hi[a]) - double(q.origin[a])) / scale[a]) + 1.0;
-                ql = std::max(0.0, std::min(255.0, ql));
-                qh = std::max(0.0, std::min(255.0, qh));
-                q.qlo[a] |= uint32_t(ql) << (8 * k);
-                q.qhi[a] |= uint32_t(qh) << (8 * k);
-            }
+        if (c.count == kEmptyChild) {  // a box no ray enters over a leaf of no triangles
+            for (int a = 0; a < 3; ++a) q.qlo[a] |= 255u << (8 * k);
+            q.link[k] = kEmptyLeaf;
+            continue;
         }
-        q.meta |= meta << (8 * k);
-        // the traversal's stack entry: an interior child's node index, a leaf
-        // tagged with its count and first triangle, or kEmptyChild
-        if (c.count == kEmptyChild)
-            q.link[k] = kEmptyChild;
-        else if (c.count == 0)
-            q.link[k] = c.link / kWidth;
-        else
-            q.link[k] = kLeafTag | (c.count << 26) | c.link;
+        for (int a = 0; a < 3; ++a) {
+            double ql = std::floor((double(c.lo[a]) - double(q.origin[a])) / double(q.scale[a])) - 1.0;
+            double qh = std::ceil((double(c.hi[a]) - double(q.origin[a])) / double(q.scale[a])) + 1.0;
+            ql = std::max(0.0, std::min(255.0, ql));
+            qh = std::max(0.0, std::min(255.0, qh));
+            q.qlo[a] |= uint32_t(ql) << (8 * k);
+            q.qhi[a] |= uint32_t(qh) << (8 * k);
+        }
+        // the traversal's stack entry: an interior child's node index, or a
+        // leaf tagged with its count and first triangle
+        q.link[k] = c.count == 0 ? c.link / kWidth : kLeafTag | (c.count << 26) | c.link;
     }
 }
 
@@ -582,7 +572,8 @@ extern "C" int rc_scene_upload(rc_ctx* c, const float* v, size_t ntri, const uin
         recs[p.slot].link = b;
     }
     size_t nrec = recs.size();
-    if (nrec >= 0x7fffffffull) return rc_host_fail(RC_ERR_INVALID, "rc_scene_upload: too many nodes");
+    if (nrec >= 0x7fffffffull || (RC_QNODE && nrec / kWidth > kMaxTriangles))  // the kernels' 32-bit node offsets
+        return rc_host_fail(RC_ERR_INVALID, "rc_scene_upload: too many nodes");
     // depth of the wide tree; links must point forward so traversal terminates
     uint32_t depth = 0;
     {
@@ -673,7 +664,7 @@ extern "C" int rc_scene_upload(rc_ctx* c, const float* v, size_t ntri, const uin
 #if RC_QNODE
     std::vector<QNode> qn(nrec / kWidth);
     for (size_t n = 0; n < qn.size(); ++n) quantize_node(&recs[n * kWidth], qn[n]);
-    if (!qn.empty()) qn[0].pad = RC_LDS_TOP ? ntop : 0u;  // the root carries the size of the LDS top
+    if (RC_LDS_TOP && qn.size() < kTopNodes) qn.resize(kTopNodes);  // the kernels copy as many; no link reaches the rest
     const void* node_src = qn.data();
     const size_t b_nodes = qn.size() * sizeof(QNode);
 #else

@@ -38,19 +38,19 @@ static_assert(sizeof(NodeRec) == 32, "NodeRec must be 32 bytes");
 // the child boxes as 8-bit offsets from the node's origin in units of a power
 // of two per axis, widened by one unit on each side so the decoded boxes
 // contain the exact ones.  Links are node indices.  2.6% faster on the
-// 2M-triangle terrain than the 128-byte records (RC_QNODE = 0).
+// 2M-triangle terrain than the 128-byte records (RC_QNODE = 0).  The scales
+// are stored as floats: a visit takes them as they are (as exponent bytes they
+// cost six more VALU instructions per visit).
 #ifndef RC_QNODE
 #define RC_QNODE 1
 #endif
 struct alignas(64) QNode {
     float origin[3];
-    uint32_t exps;     // biased float exponents of the three scales: ex | ey << 8 | ez << 16
+    float scale[3];    // 2^e per axis: bound = origin + q * scale
     uint32_t qlo[3];   // per axis, child k's lower bound in byte k
     uint32_t qhi[3];
-    uint32_t meta;     // per child, byte k: 0xFF unused, 0 interior, else leaf triangle count (1..31)
-    uint32_t pad;      // the root's: the number of top nodes kept in LDS (nodes [0, pad)); others 0
     uint32_t link[4];  // child k's stack entry: interior, node index; leaf, kLeafTag | count << 26 | first
-                       // triangle; unused, kEmptyChild
+                       // triangle; unused, kEmptyLeaf with the bounds reversed (lo 255, hi 0)
 };
 // RC_LDS_TOP = 1 keeps the first kTopNodes wide nodes (the upload puts the
 // tree's breadth-first top there) in LDS for the traversal kernels.  Off: on
@@ -100,24 +100,29 @@ struct alignas(16) DevMaterial {
 constexpr uint32_t kNoHit = 0x7fffffffu;
 constexpr int kDeepStack = 256;  // stack entries of the overflow kernel (memory part)
 
-// Traversal stack of one lane: the top kRegStack entries in registers, as a
-// shift register (no dynamic register indexing), deeper entries in LDS laid
-// out [depth][lane] so a wave's accesses hit 64 distinct banks.  A pop takes
-// its entry from a register, so the next node fetch never waits on an LDS
-// read; the LDS refill of the bottom register runs off the critical path.
-// A ray whose stack would outgrow kOnChipStack entries is handed to the
-// deep-stack kernel.
+// Traversal stack of one lane: the top kRegStack entries in registers, deeper
+// ones in LDS laid out [depth][lane] so a wave's accesses hit 64 distinct
+// banks.  A pop takes its entry from a register, so the next node fetch never
+// waits on an LDS read; the LDS refill of the bottom register runs off the
+// critical path.  Every push spills the bottom register, so the LDS rows are
+// the stack's capacity; registers start as kEmptyChild, and popping that is
+// the end of the stack (no entry count).  A ray whose stack would outgrow
+// kLdsStack entries is handed to the deep-stack kernel.  One register: each
+// more costs a move per push and pop.  19 rows: with them eight 256-thread
+// blocks of the traversal kernels fill the 160 KB of a CU.
 #ifndef RC_REG_STACK
-#define RC_REG_STACK 4
+#define RC_REG_STACK 1
 #endif
 #ifndef RC_LDS_DEPTH
-#define RC_LDS_DEPTH 16
+#define RC_LDS_DEPTH 19
 #endif
 constexpr int kRegStack = RC_REG_STACK;
 constexpr int kLdsStack = RC_LDS_DEPTH;
-constexpr int kOnChipStack = kRegStack + kLdsStack;
+static_assert(kLdsStack >= 1, "the traversal stack needs an LDS row");
+constexpr int kStackLimitMax = 20;  // the largest rc_tuning.stack_limit (above kLdsStack: all the build holds)
 constexpr int kWidth = 4;        // children per wide node
-constexpr uint32_t kEmptyChild = 0xffffffffu;
+constexpr uint32_t kEmptyChild = 0xffffffffu;  // no entry: an unused child record, the end of a stack
+constexpr uint32_t kEmptyLeaf = 0x80000000u;   // a leaf entry of no triangles: an unused slot of a QNode
 
 // ---------------------------------------------------------------- RNG
 // Philox4x32-10 (Salmon et al., SC'11): 10 rounds of two 32x32->64 products.
@@ -288,18 +293,6 @@ __device__ __forceinline__ float3 safe_inv(float3 d) {
     return make_float3(1.0f / x, 1.0f / y, 1.0f / z);
 }
 
-// Slab test of one child record against [tmin, tmax]; entry distance or +inf.
-// The exit distance is widened by a few ulps so rounding never culls a box the
-// triangle test could still hit.
-__device__ __forceinline__ float slab(float4 r0, float4 r1, float3 o, float3 inv, float tmin, float tmax) {
-    float tx0 = (r0.x - o.x) * inv.x, tx1 = (r0.w - o.x) * inv.x;
-    float ty0 = (r0.y - o.y) * inv.y, ty1 = (r1.x - o.y) * inv.y;
-    float tz0 = (r0.z - o.z) * inv.z, tz1 = (r1.y - o.z) * inv.z;
-    float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), tmin));
-    float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), tmax));
-    return tn <= tf * 1.000002f ? tn : __builtin_inff();
-}
-
 // FP32 Möller–Trumbore with the reference's structure (Triangle.cpp:61-91):
 // double-sided; the determinant test is the scale-free det == 0 instead of
 // |det| < epsilon.  This is a conservative filter: the barycentric bounds are
@@ -307,14 +300,9 @@ __device__ __forceinline__ float slab(float4 r0, float4 r1, float3 o, float3 inv
 // decision (mt_hit64, inclusive bounds) would accept.
 constexpr float kFilterBand = 1e-3f;
 // RC_FAST_RCP 1: the FP32 filter's 1/det is the hardware reciprocal (1 ulp;
-// the filter bands absorb it and FP64 decides).  RC_SLAB_SELECT 1: the four
-// child slab tests run unconditionally and empty slots are masked by a select
-// (no branch).  Together 10% faster on the 2M-triangle terrain.
+// the filter bands absorb it and FP64 decides).
 #ifndef RC_FAST_RCP
 #define RC_FAST_RCP 1
-#endif
-#ifndef RC_SLAB_SELECT
-#define RC_SLAB_SELECT 1
 #endif
 __device__ __forceinline__ bool mt_hit(const TriRec& T, float3 o, float3 d, float& t) {
     float3 v0 = f3(T.v0);
@@ -394,32 +382,58 @@ constexpr float kRefineWindow = 1e-3f;
 // triangle at exactly that distance (an exact tie) is still reached.
 constexpr float kTieWindow = 4.0f / 16777216.0f;
 
-// Stack push of x (false: the stack already holds `limit` entries).  sp
-// counts all entries; the first kRegStack live in reg[0..] (reg[0] the top),
-// entry k >= kRegStack at mem[(k - kRegStack) * stride].
-__device__ __forceinline__ bool stack_push(uint32_t* reg, int& sp, uint32_t x, uint32_t* mem, int stride, int limit) {
-    if (sp >= limit) return false;
-    if (kRegStack == 0) {
-        mem[sp * stride] = x;
-    } else {
-        if (sp >= kRegStack) mem[(sp - kRegStack) * stride] = reg[kRegStack - 1];
-#pragma unroll
-        for (int k = kRegStack - 1; k > 0; --k) reg[k] = reg[k - 1];
-        reg[0] = x;
+// A lane's stack memory: rows of `stride` bytes in an array shared by the
+// lanes, row r of the lane at byte offset base + r * stride (base = 4 * lane <
+// stride).  end is the offset past row `limit` of every lane (uniform), so a
+// lane whose next free row is at p may push m entries exactly when
+// p + m * stride < end.
+struct StackMem {
+    uint32_t* array;
+    int base, stride, end;
+    __device__ __forceinline__ uint32_t& at(int p) const {
+        return *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(array) + uint32_t(p));
     }
-    ++sp;
-    return true;
+};
+__device__ __forceinline__ StackMem stack_mem(uint32_t* array, uint32_t lane, int lanes, int limit) {
+    return StackMem{array, int(4 * lane), 4 * lanes, 4 * lanes * (limit + 1)};
 }
 
-// Stack pop (sp > 0): the top register, the registers shifted up and the
-// bottom one refilled from memory while entries remain there.
-__device__ __forceinline__ uint32_t stack_pop(uint32_t* reg, int& sp, const uint32_t* mem, int stride) {
-    --sp;
-    if (kRegStack == 0) return mem[sp * stride];
-    const uint32_t x = reg[0];
+// The stack's registers and the offset of its next free row.
+struct Stack {
+    int p;
+    uint32_t reg[kRegStack > 0 ? kRegStack : 1];  // top first
+};
+__device__ __forceinline__ void stack_reset(Stack& K, const StackMem& M) {
+    K.p = M.base;
 #pragma unroll
-    for (int k = 0; k < kRegStack - 1; ++k) reg[k] = reg[k + 1];
-    if (sp >= kRegStack) reg[kRegStack - 1] = mem[(sp - kRegStack) * stride];
+    for (int k = 0; k < kRegStack; ++k) K.reg[k] = kEmptyChild;
+    if (kRegStack == 0) {  // the end marker lies in row 0
+        M.at(K.p) = kEmptyChild;
+        K.p += M.stride;
+    }
+}
+// Push without a check: the caller has seen that the rows hold it.
+__device__ __forceinline__ void stack_push(Stack& K, const StackMem& M, uint32_t x) {
+    if (kRegStack == 0) {
+        M.at(K.p) = x;
+    } else {
+        M.at(K.p) = K.reg[kRegStack - 1];
+#pragma unroll
+        for (int k = kRegStack - 1; k > 0; --k) K.reg[k] = K.reg[k - 1];
+        K.reg[0] = x;
+    }
+    K.p += M.stride;
+}
+// The top entry, or kEmptyChild when the stack is empty (then it is not to be
+// popped again).  At the end of the stack row 0 is read, the lane's own; its
+// value is not used.
+__device__ __forceinline__ uint32_t stack_pop(Stack& K, const StackMem& M) {
+    K.p = max(K.p - M.stride, M.base);
+    if (kRegStack == 0) return M.at(K.p);
+    const uint32_t x = K.reg[0];
+#pragma unroll
+    for (int k = 0; k < kRegStack - 1; ++k) K.reg[k] = K.reg[k + 1];
+    K.reg[kRegStack - 1] = M.at(K.p);
     return x;
 }
 
@@ -499,8 +513,8 @@ __device__ __forceinline__ void wave_add(unsigned long long* dst, uint32_t v) {
 // decided in FP64 on the exact FP32 inputs (RC_HIT_FP64); otherwise the FP32
 // test decides (mt_dec32).  Closest hit keeps the smallest t; an exact tie
 // goes to the lower original triangle id, so the answer does not depend on
-// traversal order.  Returns true when an any-hit query is answered (tmax_any:
-// its tmax).
+// traversal order.  Returns true when an any-hit query is answered (its R.t
+// holds tmax until then).
 template <bool DEC64>
 struct BestT {
     using T = float;
@@ -512,10 +526,10 @@ struct BestT<true> {
 
 template <bool ANY, bool COUNT, bool DEC64>
 __device__ __forceinline__ bool test_leaf(const TriRec* __restrict__ tris, uint32_t first, uint32_t count, float3 o,
-                                          float3 d, float tmin, float tmax_any, typename BestT<DEC64>::T& best,
-                                          float& cull, TraceResult& R, uint32_t& n_tri) {
+                                          float3 d, float tmin, typename BestT<DEC64>::T& best, TraceResult& R,
+                                          uint32_t& n_tri) {
     for (uint32_t j = first; j < first + count; ++j) {
-        const float4* q = reinterpret_cast<const float4*>(tris + j);
+        const float4* q = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(tris) + j * 48u);  // < 4 GiB
         TriRec T;
         T.v0 = q[0];
         T.v1 = q[1];
@@ -524,13 +538,13 @@ __device__ __forceinline__ bool test_leaf(const TriRec* __restrict__ tris, uint3
         if (DEC64) {
             float t32;
             if (!mt_hit(T, o, d, t32)) continue;
-            if (t32 > cull || t32 < tmin * (1.0f - kRefineWindow) - 1e-30f) continue;
+            if (t32 > R.t * (1.0f + kRefineWindow) || t32 < tmin * (1.0f - kRefineWindow) - 1e-30f) continue;
             double t64, u64, v64;
             if (!mt_hit64(T, o, d, t64, u64, v64)) continue;
             if (t64 < double(tmin)) continue;
             uint32_t id = __float_as_uint(T.v0.w);
             if (ANY) {
-                if (t64 <= double(tmax_any) && !(__float_as_uint(T.v1.w) & RC_MAT_NON_SHADOWING)) {
+                if (t64 <= double(R.t) && !(__float_as_uint(T.v1.w) & RC_MAT_NON_SHADOWING)) {
                     R.t = float(t64);
                     R.id = id;
                     return true;
@@ -542,62 +556,56 @@ __device__ __forceinline__ bool test_leaf(const TriRec* __restrict__ tris, uint3
                 R.v = float(v64);
                 R.w = 1.0f;
                 R.id = id;
-                cull = R.t * (1.0f + kRefineWindow);
             }
         } else {
             float t, U, V, adet;
             if (!mt_dec32(T, o, d, t, U, V, adet)) continue;
-            if (t < tmin || t > cull) continue;
+            if (t < tmin) continue;
             uint32_t id = __float_as_uint(T.v0.w);
             if (ANY) {
-                if (t <= tmax_any && !(__float_as_uint(T.v1.w) & RC_MAT_NON_SHADOWING)) {
+                if (t <= R.t && !(__float_as_uint(T.v1.w) & RC_MAT_NON_SHADOWING)) {
                     R.t = t;
                     R.id = id;
                     return true;
                 }
-            } else if (t < best || (t == best && id < R.id)) {
-                best = t;
+            } else if (t < R.t || (t == R.t && id < R.id)) {
                 R.t = t;
                 R.u = U;
                 R.v = V;
                 R.w = adet;
                 R.id = id;
-                cull = t * (1.0f + kTieWindow);
             }
         }
     }
     return false;
 }
 
-// Cull distance of a query with no hit yet.
+// How far past a distance the boxes are still entered: a relative window that
+// covers the decision's ties and refinements.
 template <bool DEC64>
-__device__ __forceinline__ float initial_cull(float tmax) {
-    return tmax * (1.0f + (DEC64 ? kRefineWindow : kTieWindow));
+__device__ __forceinline__ float cull_at(float t) {
+    return t * (1.0f + (DEC64 ? kRefineWindow : kTieWindow));
 }
 
-// Compare-exchange of two children (entry distance, stack entry) by distance,
-// as selects (no branch).
-__device__ __forceinline__ void order2(float& ta, uint32_t& ea, float& tb, uint32_t& eb) {
-    const bool sw = tb < ta;
-    const float t0 = sw ? tb : ta, t1 = sw ? ta : tb;
-    const uint32_t e0 = sw ? eb : ea, e1 = sw ? ea : eb;
-    ta = t0; tb = t1;
-    ea = e0; eb = e1;
-}
-
-// The same with the link and count of a child record carried separately.
-__device__ __forceinline__ void order2(float& ta, uint32_t& la, uint32_t& ca, float& tb, uint32_t& lb, uint32_t& cb) {
-    const bool sw = tb < ta;
-    const float t0 = sw ? tb : ta, t1 = sw ? ta : tb;
-    const uint32_t l0 = sw ? lb : la, l1 = sw ? la : lb;
-    const uint32_t c0 = sw ? cb : ca, c1 = sw ? ca : cb;
-    ta = t0; tb = t1;
-    la = l0; lb = l1;
-    ca = c0; cb = c1;
+// Compare-exchange of two children (entry distance in the high word, stack
+// entry in the low one) by distance.  As doubles the words order by the
+// distances' bits (both are non-negative floats, whose bits order as they do
+// and stay below a double's infinity), so one v_min_f64 and one v_max_f64 move
+// the distance and its entry together: 8 cycles of a SIMD against 20 for a
+// compare and four selects (full-rate VALU instructions take 2 cycles per
+// wave on this chip: FMA, add, multiply, and / or / xor, moves; minima,
+// compares, selects, conversions and FP64 take 4).
+__device__ __forceinline__ void order2(double& a, double& b) {
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
 }
 
 // 1: the if-if traversal (leaves postponed onto the stack), 2% faster on the
-// 2M-triangle terrain than testing leaf children at once (0).
+// 2M-triangle terrain than testing leaf children at once (0, with the 128-byte
+// node records).
 #ifndef RC_TRAV_IFIF
 #define RC_TRAV_IFIF 1
 #endif
@@ -617,251 +625,256 @@ __device__ __forceinline__ void order2(float& ta, uint32_t& la, uint32_t& ca, fl
 #define RC_LEAF_POSTPONE_ANY 32
 #endif
 // Stack entries of the if-if traversal: an interior child's record index, or
-// a leaf tagged with kLeafTag, its triangle count (1..31) in bits 26..30 and
+// a leaf tagged with kLeafTag, its triangle count (0..31) in bits 26..30 and
 // its first triangle (< 2^26) below.  The upload guarantees both: scenes hold
-// at most 2^26 triangles and longer leaves are split into wide nodes.
+// at most 2^26 triangles and longer leaves are split into wide nodes.  As
+// signed numbers: interior entries are >= 0, leaves < -1, kEmptyChild is -1.
 constexpr uint32_t kLeafTag = 0x80000000u;
 constexpr uint32_t kMaxLeafRecord = 32;           // leaf records hold fewer triangles
 constexpr size_t kMaxTriangles = size_t(1) << 26;
+__device__ __forceinline__ bool is_node(uint32_t e) { return int32_t(e) >= 0; }
+__device__ __forceinline__ bool is_leaf(uint32_t e) { return int32_t(e) < -1; }
 
-// Ordered, t-culled traversal over 4-wide nodes.  The four child boxes are
-// tested and sorted by entry distance (a 5-comparator network); leaf children
-// are tested in that order at once, the nearest interior child is visited
-// next and the others are pushed far-to-near on the lane's stack (registers,
-// then stack[k * stride]: LDS for the main kernels, global memory for the
-// deep-stack kernel), at most max_depth entries.  ANY: stop at the first
-// triangle (not nonShadowing) with t in [tmin, tmax].
-template <bool ANY, bool COUNT, bool DEC64>
-__device__ __forceinline__ TraceResult traverse_inline(const NodeRec* __restrict__ nodes, const TriRec* __restrict__ tris,
-                                                float3 o, float3 d, float tmin, float tmax, uint32_t* stack,
-                                                int stride, int max_depth, uint32_t& n_rec, uint32_t& n_tri) {
-    const float INF = __builtin_inff();
-    TraceResult R{tmax, 0.0f, 0.0f, kNoHit, false, 1.0f};
-    tmin = fmaxf(tmin, 0.0f);
-    typename BestT<DEC64>::T best = tmax;
-    float cull = initial_cull<DEC64>(tmax);
-    float3 inv = safe_inv(d);
-    uint32_t cur = 0;
-    int sp = 0;
-    uint32_t reg[kRegStack > 0 ? kRegStack : 1];
-    while (true) {
-        const float4* p = reinterpret_cast<const float4*>(nodes + cur);
-        float4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3], q4 = p[4], q5 = p[5], q6 = p[6], q7 = p[7];
-        if (COUNT) n_rec += kWidth;
-        uint32_t l0 = __float_as_uint(q1.z), c0 = __float_as_uint(q1.w);
-        uint32_t l1 = __float_as_uint(q3.z), c1 = __float_as_uint(q3.w);
-        uint32_t l2 = __float_as_uint(q5.z), c2 = __float_as_uint(q5.w);
-        uint32_t l3 = __float_as_uint(q7.z), c3 = __float_as_uint(q7.w);
-        float t0 = c0 == kEmptyChild ? INF : slab(q0, q1, o, inv, tmin, cull);
-        float t1 = c1 == kEmptyChild ? INF : slab(q2, q3, o, inv, tmin, cull);
-        float t2 = c2 == kEmptyChild ? INF : slab(q4, q5, o, inv, tmin, cull);
-        float t3 = c3 == kEmptyChild ? INF : slab(q6, q7, o, inv, tmin, cull);
-        order2(t0, l0, c0, t1, l1, c1);
-        order2(t2, l2, c2, t3, l3, c3);
-        order2(t0, l0, c0, t2, l2, c2);
-        order2(t1, l1, c1, t3, l3, c3);
-        order2(t1, l1, c1, t2, l2, c2);
-        // leaf children, nearest first
-        if (c0 != 0 && t0 != INF && t0 <= cull)
-            if (test_leaf<ANY, COUNT, DEC64>(tris, l0, c0, o, d, tmin, tmax, best, cull, R, n_tri)) return R;
-        if (c1 != 0 && t1 != INF && t1 <= cull)
-            if (test_leaf<ANY, COUNT, DEC64>(tris, l1, c1, o, d, tmin, tmax, best, cull, R, n_tri)) return R;
-        if (c2 != 0 && t2 != INF && t2 <= cull)
-            if (test_leaf<ANY, COUNT, DEC64>(tris, l2, c2, o, d, tmin, tmax, best, cull, R, n_tri)) return R;
-        if (c3 != 0 && t3 != INF && t3 <= cull)
-            if (test_leaf<ANY, COUNT, DEC64>(tris, l3, c3, o, d, tmin, tmax, best, cull, R, n_tri)) return R;
-        // interior children: farthest pushed first, nearest visited next
-        bool have = false;
-        uint32_t next = 0;
-#define RC_INTERIOR(t, l, c)                                            \
-        if (c == 0 && t != INF && t <= cull) {                          \
-            if (have && !stack_push(reg, sp, next, stack, stride, max_depth)) { \
-                R.overflow = true;                                      \
-                return R;                                               \
-            }                                                           \
-            next = l;                                                   \
-            have = true;                                                \
-        }
-        RC_INTERIOR(t3, l3, c3)
-        RC_INTERIOR(t2, l2, c2)
-        RC_INTERIOR(t1, l1, c1)
-        RC_INTERIOR(t0, l0, c0)
-#undef RC_INTERIOR
-        if (have) {
-            cur = next;
-        } else {
-            if (sp == 0) break;
-            cur = stack_pop(reg, sp, stack, stride);
-        }
-    }
-    return R;
-}
-
-// The same traversal with leaves postponed ("if-if"): a node visit pushes its
-// hit children, leaves included, far-to-near and keeps the nearest; each step
-// then does at most one node visit and one leaf, so the lanes of a wave stay
-// in step instead of waiting while one lane tests up to four leaves.  The
-// state is explicit (trav_begin / trav_step).
+// A traversal's state.  The boxes are tested in ray distances scaled by a power
+// of two (so every product and comparison is the unscaled one) that puts the
+// scene's end of the ray, or tmax when that is nearer, below 1: clamping an
+// entry plane's FMA to [0, 1], which is free (a modifier), then takes the place
+// of the maximum with 0, and 1 stays an entry past everything.  The distances
+// reported are the triangle tests', unscaled.
 template <bool DEC64>
 struct Trav {
-    float3 o, d, inv;
-    float tmin, cull;
-    typename BestT<DEC64>::T best;
+    float3 o, d;
+    float3 inv;   // 1 / d, no zero component (safe_inv), scaled
+    float scale;  // the power of two
+    float tmin;
+    bool late;    // wave-uniform: some ray of the wave has a tmin > 0, entries are held against it
+    float cull;   // boxes entered beyond it are skipped (scaled, below 1)
+    typename BestT<DEC64>::T best;  // DEC64: the best hit's FP64 distance; else unused (R.t is it)
     TraceResult R;
     uint32_t cur;
-    int sp;
-    uint32_t reg[kRegStack > 0 ? kRegStack : 1];  // top of the stack
+    Stack stack;
     uint32_t leaf;     // a leaf set aside (leaf postponing), else kEmptyChild
     const uint4* top;  // LDS copy of nodes [0, ntop), or null
     uint32_t ntop;
 };
 
-// Copies the first `ntop` nodes (the root's count) into LDS `top` (four
-// 16-byte words per node); every thread of the block calls it, and it ends in
-// a barrier.  Returns the count (0 with the 128-byte node records).
+// Copies the first kTopNodes nodes into LDS `top` (four 16-byte words per
+// node; the upload pads the array to as many); every thread of the block calls
+// it, and it ends in a barrier.  Returns the count (0 with the 128-byte node
+// records or with RC_LDS_TOP 0).
 template <class N>
 __device__ __forceinline__ uint32_t load_top(const N* __restrict__ nodes, uint4* top) {
-    if constexpr (!RC_LDS_TOP || sizeof(N) != sizeof(QNode)) {
+    if constexpr (!RC_LDS_TOP || sizeof(N) != 64) {
         return 0u;
     } else {
-        const uint32_t ntop = min(reinterpret_cast<const QNode*>(nodes)[0].pad, kTopNodes);
         const uint4* src = reinterpret_cast<const uint4*>(nodes);
-        for (uint32_t w = threadIdx.x; w < 4 * ntop; w += blockDim.x) top[w] = src[w];
+        for (uint32_t w = threadIdx.x; w < 4 * kTopNodes; w += blockDim.x) top[w] = src[w];
         __syncthreads();
-        return ntop;
+        return kTopNodes;
     }
 }
 
+// The cull distance for R.t (the best hit's, or tmax).
 template <bool DEC64>
-__device__ __forceinline__ void trav_begin(Trav<DEC64>& S, float3 o, float3 d, float tmin, float tmax,
-                                           const uint4* top = nullptr, uint32_t ntop = 0) {
+__device__ __forceinline__ void trav_cull(Trav<DEC64>& S) {
+    S.cull = fminf(cull_at<DEC64>(S.R.t) * S.scale, 0.99999994f);
+}
+
+// Distance at which a ray (origin o, 1/d inv) has left the root's box, a hair
+// later; negative when the box lies behind.  Nothing is hit past it.
+__device__ __forceinline__ float scene_exit(const NodeT* __restrict__ nodes, float3 o, float3 inv) {
+#if RC_QNODE
+    // scalar loads; opaque, so a loop over rays reads the root again instead of
+    // keeping its planes in vector registers
+    typedef const __attribute__((address_space(4))) float* scalar_floats;
+    uint64_t root = reinterpret_cast<uint64_t>(nodes);
+    asm volatile("" : "+s"(root));
+    const scalar_floats f = reinterpret_cast<scalar_floats>(root);  // QNode: origin, scale
+    auto far = [](float lo, float scale, float o, float inv) {
+        return ((inv < 0.0f ? lo : fmaf(255.0f, scale, lo)) - o) * inv;
+    };
+    const float t = fminf(fminf(far(f[0], f[3], o.x, inv.x), far(f[1], f[4], o.y, inv.y)), far(f[2], f[5], o.z, inv.z));
+    return t * 1.00001f;
+#else
+    return __builtin_inff();
+#endif
+}
+
+// late: false when every ray's tmin is 0 (the renderer's).
+template <bool DEC64>
+__device__ __forceinline__ void trav_begin(Trav<DEC64>& S, const NodeT* __restrict__ nodes, const StackMem& M,
+                                           float3 o, float3 d, float tmin, float tmax, const uint4* top, uint32_t ntop,
+                                           bool late) {
     S.top = top;
     S.ntop = top ? ntop : 0u;
     S.o = o;
     S.d = d;
-    S.inv = safe_inv(d);
-    S.tmin = fmaxf(tmin, 0.0f);
+    S.tmin = late ? fmaxf(tmin, 0.0f) : 0.0f;
+    S.late = late && __any(S.tmin > 0.0f);
     S.best = tmax;
-    S.cull = initial_cull<DEC64>(tmax);
     S.R = TraceResult{tmax, 0.0f, 0.0f, kNoHit, false, 1.0f};
-    S.cur = 0;  // root: interior record 0
-    S.sp = 0;
+    const float3 inv = safe_inv(d);
+    const float T0 = cull_at<DEC64>(tmax), exit = scene_exit(nodes, o, inv);
+    const float T = fminf(fmaxf(exit < T0 ? exit : T0, 1e-12f), 3e37f);
+    S.scale = __uint_as_float((253u << 23) - (__float_as_uint(T) & 0x7f800000u));  // 2^-k, 2^(k-1) <= T < 2^k
+    S.inv = inv * S.scale;
+    trav_cull(S);
+    S.cur = tmax < S.tmin ? kEmptyChild : 0u;  // root: interior record 0; an empty interval has no hit
     S.leaf = kEmptyChild;
+    stack_reset(S.stack, M);
 }
 
-// One step; true when the traversal has ended (S.R holds the result,
-// S.R.overflow when the stack would have outgrown max_depth entries).
+// a selected where the mask is 0, b where it is ~0 (one full-rate instruction).
+__device__ __forceinline__ uint32_t pick(uint32_t a, uint32_t b, uint32_t mask) {
+    return uint32_t(__builtin_amdgcn_bitop3_b32(int(a), int(b), int(mask), 0xD8));
+}
+__device__ __forceinline__ float clamp01(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); }
+
+// Box tests of one wide node: per child its entry distance in [0, 1] (scaled),
+// whether the ray enters it, and its stack entry.
+struct Hits {
+    float t[kWidth];
+    bool h[kWidth];
+    uint32_t e[kWidth];
+};
+template <bool DEC64>
+__device__ __forceinline__ void node_hits(const Trav<DEC64>& S, const NodeT* __restrict__ nodes, uint32_t cur,
+                                          Hits& H) {
+    // Per axis the entry plane is the lower bound when the direction is
+    // positive and the upper one when it is negative: the planes are picked by
+    // the sign once per node, not by a minimum and a maximum per child.  The
+    // exit is widened by a few ulps so rounding never culls a box the triangle
+    // test could still hit.
+    auto enter = [&](int k, float tnx, float tny, float tnz, float tfx, float tfy, float tfz) {
+        H.t[k] = fmaxf(fmaxf(clamp01(tnx), tny), tnz);
+        if (S.late) H.t[k] = fmaxf(H.t[k], S.tmin * S.scale);
+        H.h[k] = H.t[k] <= fminf(fminf(fminf(tfx, tfy), tfz) * 1.000002f, S.cull);
+    };
+    const uint32_t mx = uint32_t(int32_t(__float_as_uint(S.inv.x)) >> 31);
+    const uint32_t my = uint32_t(int32_t(__float_as_uint(S.inv.y)) >> 31);
+    const uint32_t mz = uint32_t(int32_t(__float_as_uint(S.inv.z)) >> 31);
+#if RC_QNODE
+    uint4 q0, q1, q2, q3;
+    if (RC_LDS_TOP && cur < S.ntop) {  // the top of the tree, from LDS
+        const uint4* t = S.top + 4 * cur;
+        q0 = t[0];
+        q1 = t[1];
+        q2 = t[2];
+        q3 = t[3];
+    } else {
+        // a 32-bit offset from the uniform base: the node array stays within 4 GiB
+        // (fewer than 2^26 wide nodes)
+        const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + cur * 64u);
+        q0 = p[0];
+        q1 = p[1];
+        q2 = p[2];
+        q3 = p[3];
+    }
+    // bound = origin + q * scale; in scaled ray distance q * (scale * inv) + (origin - o) * inv
+    const float ax = __uint_as_float(q0.w) * S.inv.x, bx = (__uint_as_float(q0.x) - S.o.x) * S.inv.x;
+    const float ay = __uint_as_float(q1.x) * S.inv.y, by = (__uint_as_float(q0.y) - S.o.y) * S.inv.y;
+    const float az = __uint_as_float(q1.y) * S.inv.z, bz = (__uint_as_float(q0.z) - S.o.z) * S.inv.z;
+    const uint32_t nx = pick(q1.z, q2.y, mx), fx = pick(q2.y, q1.z, mx);
+    const uint32_t ny = pick(q1.w, q2.z, my), fy = pick(q2.z, q1.w, my);
+    const uint32_t nz = pick(q2.x, q2.w, mz), fz = pick(q2.w, q2.x, mz);
+    auto plane = [](uint32_t w, int k, float a, float b) { return fmaf(float((w >> (8 * k)) & 0xFFu), a, b); };
+#pragma unroll
+    for (int k = 0; k < kWidth; ++k)
+        enter(k, plane(nx, k, ax, bx), plane(ny, k, ay, by), plane(nz, k, az, bz), plane(fx, k, ax, bx),
+              plane(fy, k, ay, by), plane(fz, k, az, bz));
+    H.e[0] = q3.x;
+    H.e[1] = q3.y;
+    H.e[2] = q3.z;
+    H.e[3] = q3.w;
+#else
+    const uint4* p = reinterpret_cast<const uint4*>(nodes + cur);
+    auto plane = [](uint32_t w, float inv, float o) { return (__uint_as_float(w) - o) * inv; };
+#pragma unroll
+    for (int k = 0; k < kWidth; ++k) {
+        const uint4 a = p[2 * k], b = p[2 * k + 1];  // lo.xyz hi.x, hi.yz link count
+        const uint32_t nx = pick(a.x, a.w, mx), fx = pick(a.w, a.x, mx);
+        const uint32_t ny = pick(a.y, b.x, my), fy = pick(b.x, a.y, my);
+        const uint32_t nz = pick(a.z, b.y, mz), fz = pick(b.y, a.z, mz);
+        enter(k, plane(nx, S.inv.x, S.o.x), plane(ny, S.inv.y, S.o.y), plane(nz, S.inv.z, S.o.z),
+              plane(fx, S.inv.x, S.o.x), plane(fy, S.inv.y, S.o.y), plane(fz, S.inv.z, S.o.z));
+        H.h[k] = H.h[k] && b.w != kEmptyChild;
+        H.e[k] = b.w != 0 ? (kLeafTag | (b.w << 26) | b.z) : b.z;
+    }
+#endif
+}
+
+// The children of a visited node in H: the nearest (ANY without RC_ANY_SORT:
+// the first) becomes S.cur, the others go on the stack farthest first; with
+// none S.cur is popped.  False when the stack would outgrow its rows.
+template <bool SORT, bool DEC64>
+__device__ __forceinline__ bool take_children(Trav<DEC64>& S, Hits& H, const StackMem& M) {
+    const bool* h = H.h;
+    uint32_t e0 = H.e[0], e1 = H.e[1], e2 = H.e[2], e3 = H.e[3];
+    const bool a01 = h[0] || h[1], a23 = h[2] || h[3], b01 = h[0] && h[1], b23 = h[2] && h[3];
+    const bool two = b01 || b23 || (a01 && a23);
+    const bool three = (b01 && a23) || (b23 && a01), four = b01 && b23;
+    if (SORT) {
+        // a child not entered sorts last: 2.0f, above every entry distance
+        double k0 = __hiloint2double(h[0] ? __float_as_int(H.t[0]) : 0x40000000, int(e0));
+        double k1 = __hiloint2double(h[1] ? __float_as_int(H.t[1]) : 0x40000000, int(e1));
+        double k2 = __hiloint2double(h[2] ? __float_as_int(H.t[2]) : 0x40000000, int(e2));
+        double k3 = __hiloint2double(h[3] ? __float_as_int(H.t[3]) : 0x40000000, int(e3));
+        order2(k0, k1);
+        order2(k2, k3);
+        order2(k0, k2);
+        order2(k1, k3);
+        order2(k1, k2);
+        e0 = uint32_t(__double2loint(k0));
+        e1 = uint32_t(__double2loint(k1));
+        e2 = uint32_t(__double2loint(k2));
+        e3 = uint32_t(__double2loint(k3));
+    }
+    if (two && S.stack.p + 3 * M.stride >= M.end) {  // rare: count the entries
+        const int m = four ? 3 : three ? 2 : 1;
+        if (S.stack.p + m * M.stride >= M.end) return false;
+    }
+    if (SORT) {
+        if (two) {
+            if (four) stack_push(S.stack, M, e3);
+            if (three) stack_push(S.stack, M, e2);
+            stack_push(S.stack, M, e1);
+        }
+        S.cur = e0;
+    } else {
+        if (two) {
+            if (h[3] && (a01 || h[2])) stack_push(S.stack, M, e3);
+            if (h[2] && a01) stack_push(S.stack, M, e2);
+            if (b01) stack_push(S.stack, M, e1);
+        }
+        S.cur = h[0] ? e0 : h[1] ? e1 : h[2] ? e2 : e3;
+    }
+    if (!(a01 || a23)) S.cur = stack_pop(S.stack, M);
+    return true;
+}
+
+// One step of the ordered, culled traversal over 4-wide nodes with leaves
+// postponed ("if-if"): a node visit pushes the children it enters, leaves
+// included, far-to-near and keeps the nearest; each step does at most one node
+// visit and one leaf, so the lanes of a wave stay in step instead of waiting
+// while one lane tests up to four leaves.  True when the traversal has ended
+// (S.R holds the result, S.R.overflow when the stack would have outgrown its
+// rows).  ANY: stop at the first triangle (not nonShadowing) with t in [tmin,
+// tmax].
+//
+// Bound by VALU issue: before, a visit's 132 instructions took 448 of a SIMD's
+// cycles and the pushes, the pop and the leaf bookkeeping of a step another
+// 270; the kernels kept the VALU busy all the time.
 template <bool ANY, bool COUNT, bool DEC64>
 __device__ __forceinline__ bool trav_step(Trav<DEC64>& S, const NodeT* __restrict__ nodes,
-                                          const TriRec* __restrict__ tris, uint32_t* stack, int stride, int max_depth,
-                                          uint32_t& n_rec, uint32_t& n_tri) {
-    const float INF = __builtin_inff();
-    if (!(S.cur & kLeafTag)) {
-#if RC_QNODE
-        uint4 q0, q1, q2, q3;
-        if (S.cur < S.ntop) {  // the top of the tree, from LDS
-            const uint4* t = S.top + 4 * S.cur;
-            q0 = t[0];
-            q1 = t[1];
-            q2 = t[2];
-            q3 = t[3];
-        } else {
-            const uint4* p = reinterpret_cast<const uint4*>(nodes + S.cur);
-            q0 = p[0];
-            q1 = p[1];
-            q2 = p[2];
-            q3 = p[3];
-        }
+                                          const TriRec* __restrict__ tris, const StackMem& M, uint32_t& n_rec,
+                                          uint32_t& n_tri) {
+    if (is_node(S.cur)) {
         if (COUNT) n_rec += kWidth;
-        // bound = origin + q * 2^e; in ray distance q * (2^e / d) + (origin - o) / d
-        const float ax = __uint_as_float((q0.w & 0xFFu) << 23) * S.inv.x;
-        const float ay = __uint_as_float(((q0.w >> 8) & 0xFFu) << 23) * S.inv.y;
-        const float az = __uint_as_float(((q0.w >> 16) & 0xFFu) << 23) * S.inv.z;
-        const float bx = (__uint_as_float(q0.x) - S.o.x) * S.inv.x;
-        const float by = (__uint_as_float(q0.y) - S.o.y) * S.inv.y;
-        const float bz = (__uint_as_float(q0.z) - S.o.z) * S.inv.z;
-        // Per axis the entry plane is the lower bound when the direction is
-        // positive and the upper one when it is negative (the decode is
-        // monotonic in q): picking the two words by sign once per node takes
-        // the place of a min and a max per axis and child, with the same result.
-        const uint32_t nx = S.inv.x < 0.0f ? q1.w : q1.x, fx = S.inv.x < 0.0f ? q1.x : q1.w;
-        const uint32_t ny = S.inv.y < 0.0f ? q2.x : q1.y, fy = S.inv.y < 0.0f ? q1.y : q2.x;
-        const uint32_t nz = S.inv.z < 0.0f ? q2.y : q1.z, fz = S.inv.z < 0.0f ? q1.z : q2.y;
-#define RC_QSLAB(k, e)                                                                                         \
-        [&]() {                                                                                                \
-            const float tnx = fmaf(float((nx >> (8 * k)) & 0xFFu), ax, bx);                                     \
-            const float tfx = fmaf(float((fx >> (8 * k)) & 0xFFu), ax, bx);                                     \
-            const float tny = fmaf(float((ny >> (8 * k)) & 0xFFu), ay, by);                                     \
-            const float tfy = fmaf(float((fy >> (8 * k)) & 0xFFu), ay, by);                                     \
-            const float tnz = fmaf(float((nz >> (8 * k)) & 0xFFu), az, bz);                                     \
-            const float tfz = fmaf(float((fz >> (8 * k)) & 0xFFu), az, bz);                                     \
-            const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, S.tmin));                                        \
-            const float tf = fminf(fminf(tfx, tfy), fminf(tfz, S.cull));                                        \
-            return tn <= tf * 1.000002f && e != kEmptyChild ? tn : INF;                                        \
-        }()
-        // links are the children's stack entries (kEmptyChild for an unused slot)
-        uint32_t e0 = q3.x, e1 = q3.y, e2 = q3.z, e3 = q3.w;
-        float t0 = RC_QSLAB(0, e0), t1 = RC_QSLAB(1, e1), t2 = RC_QSLAB(2, e2), t3 = RC_QSLAB(3, e3);
-#undef RC_QSLAB
-        if (!ANY || RC_ANY_SORT) {
-            order2(t0, e0, t1, e1);
-            order2(t2, e2, t3, e3);
-            order2(t0, e0, t2, e2);
-            order2(t1, e1, t3, e3);
-            order2(t1, e1, t2, e2);
-        }
-#else
-        const float4* p = reinterpret_cast<const float4*>(nodes + S.cur);
-        float4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3], q4 = p[4], q5 = p[5], q6 = p[6], q7 = p[7];
-        if (COUNT) n_rec += kWidth;
-        uint32_t l0 = __float_as_uint(q1.z), c0 = __float_as_uint(q1.w);
-        uint32_t l1 = __float_as_uint(q3.z), c1 = __float_as_uint(q3.w);
-        uint32_t l2 = __float_as_uint(q5.z), c2 = __float_as_uint(q5.w);
-        uint32_t l3 = __float_as_uint(q7.z), c3 = __float_as_uint(q7.w);
-#if RC_SLAB_SELECT
-        float t0 = slab(q0, q1, S.o, S.inv, S.tmin, S.cull), t1 = slab(q2, q3, S.o, S.inv, S.tmin, S.cull);
-        float t2 = slab(q4, q5, S.o, S.inv, S.tmin, S.cull), t3 = slab(q6, q7, S.o, S.inv, S.tmin, S.cull);
-        t0 = c0 == kEmptyChild ? INF : t0;
-        t1 = c1 == kEmptyChild ? INF : t1;
-        t2 = c2 == kEmptyChild ? INF : t2;
-        t3 = c3 == kEmptyChild ? INF : t3;
-#else
-        float t0 = c0 == kEmptyChild ? INF : slab(q0, q1, S.o, S.inv, S.tmin, S.cull);
-        float t1 = c1 == kEmptyChild ? INF : slab(q2, q3, S.o, S.inv, S.tmin, S.cull);
-        float t2 = c2 == kEmptyChild ? INF : slab(q4, q5, S.o, S.inv, S.tmin, S.cull);
-        float t3 = c3 == kEmptyChild ? INF : slab(q6, q7, S.o, S.inv, S.tmin, S.cull);
-#endif
-        uint32_t e0 = c0 != 0 ? (kLeafTag | (c0 << 26) | l0) : l0, e1 = c1 != 0 ? (kLeafTag | (c1 << 26) | l1) : l1;
-        uint32_t e2 = c2 != 0 ? (kLeafTag | (c2 << 26) | l2) : l2, e3 = c3 != 0 ? (kLeafTag | (c3 << 26) | l3) : l3;
-        order2(t0, e0, t1, e1);
-        order2(t2, e2, t3, e3);
-        order2(t0, e0, t2, e2);
-        order2(t1, e1, t3, e3);
-        order2(t1, e1, t2, e2);
-#endif  // RC_QNODE
-        bool have = false;
-        uint32_t next = 0;
-#define RC_CHILD(t, e)                                                                                         \
-        if (t != INF && t <= S.cull) {                                                                         \
-            if (have && !stack_push(S.reg, S.sp, next, stack, stride, max_depth)) {                            \
-                S.R.overflow = true;                                                                           \
-                return true;                                                                                   \
-            }                                                                                                  \
-            next = e;                                                                                          \
-            have = true;                                                                                       \
-        }
-        RC_CHILD(t3, e3)
-        RC_CHILD(t2, e2)
-        RC_CHILD(t1, e1)
-        RC_CHILD(t0, e0)
-#undef RC_CHILD
-        if (have) {
-            S.cur = next;
-        } else if (S.sp == 0) {
-            if (!RC_LEAF_POSTPONE) return true;
-            S.cur = kEmptyChild;  // nothing left but a leaf set aside
-        } else {
-            S.cur = stack_pop(S.reg, S.sp, stack, stride);
+        Hits H;
+        node_hits<DEC64>(S, nodes, S.cur, H);
+        if (!take_children<!ANY || RC_ANY_SORT>(S, H, M)) {
+            S.R.overflow = true;
+            return true;
         }
     }
 #if RC_LEAF_POSTPONE
@@ -870,157 +883,179 @@ __device__ __forceinline__ bool trav_step(Trav<DEC64>& S, const NodeT* __restric
     // and goes on with its stack; the wave tests the leaves set aside when at
     // least RC_LEAF_POSTPONE / 64 of its lanes hold one, or when no lane has a
     // node left to visit.  A lane whose next entry is a second leaf waits.
-    if (S.cur != kEmptyChild && (S.cur & kLeafTag) && S.leaf == kEmptyChild) {
+    if (is_leaf(S.cur) && S.leaf == kEmptyChild) {
         S.leaf = S.cur;
-        S.cur = S.sp == 0 ? kEmptyChild : stack_pop(S.reg, S.sp, stack, stride);
+        S.cur = stack_pop(S.stack, M);
     }
     {
         const bool held = S.leaf != kEmptyChild;
-        const uint64_t lanes = __ballot(1), visit = __ballot(!(S.cur & kLeafTag)), holding = __ballot(held);
+        const uint64_t lanes = __ballot(1), visit = __ballot(is_node(S.cur)), holding = __ballot(held);
         const bool run = visit == 0 || uint32_t(__popcll(holding)) * 64u >= uint32_t(__popcll(lanes)) * kHold;
         if (held && run) {
             const uint32_t first = S.leaf & ((1u << 26) - 1u), count = (S.leaf >> 26) & 31u;
-            if (test_leaf<ANY, COUNT, DEC64>(tris, first, count, S.o, S.d, S.tmin, S.R.t, S.best, S.cull, S.R, n_tri))
-                return true;
+            const uint32_t id = S.R.id;
+            if (test_leaf<ANY, COUNT, DEC64>(tris, first, count, S.o, S.d, S.tmin, S.best, S.R, n_tri)) return true;
+            if (!ANY && S.R.id != id) trav_cull(S);
             S.leaf = kEmptyChild;
         }
     }
-    return S.cur == kEmptyChild && S.leaf == kEmptyChild;
+    return (S.cur & S.leaf) == kEmptyChild;
 #else
-    if (S.cur & kLeafTag) {
+    if (is_leaf(S.cur)) {
         const uint32_t first = S.cur & ((1u << 26) - 1u), count = (S.cur >> 26) & 31u;
-        // an any-hit query's R.t holds tmax until the query is answered
-        if (test_leaf<ANY, COUNT, DEC64>(tris, first, count, S.o, S.d, S.tmin, S.R.t, S.best, S.cull, S.R, n_tri))
-            return true;
-        if (S.sp == 0) return true;
-        S.cur = stack_pop(S.reg, S.sp, stack, stride);
+        const uint32_t id = S.R.id;
+        if (test_leaf<ANY, COUNT, DEC64>(tris, first, count, S.o, S.d, S.tmin, S.best, S.R, n_tri)) return true;
+        if (!ANY && S.R.id != id) trav_cull(S);
+        S.cur = stack_pop(S.stack, M);
     }
-    return false;
+    return S.cur == kEmptyChild;
 #endif  // RC_LEAF_POSTPONE
 }
 
+// The traversal without postponed leaves (RC_TRAV_IFIF 0 with the 128-byte
+// node records): the leaf children a node visit enters are tested at once, the
+// nearest interior child is visited next and the others are pushed.
+#ifndef RC_SLAB_SELECT
+#define RC_SLAB_SELECT 1  // 0: leaf children not entered are skipped by a branch per child
+#endif
+template <bool ANY, bool COUNT, bool DEC64>
+__device__ __forceinline__ TraceResult traverse_inline(const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
+                                                       float3 o, float3 d, float tmin, float tmax, const StackMem& M,
+                                                       uint32_t& n_rec, uint32_t& n_tri) {
+    Trav<DEC64> S;
+    trav_begin(S, nodes, M, o, d, tmin, tmax, nullptr, 0, true);
+    while (S.cur != kEmptyChild) {
+        if (COUNT) n_rec += kWidth;
+        Hits H;
+        node_hits<DEC64>(S, nodes, S.cur, H);
+        for (int k = 0; k < kWidth; ++k) {
+            if (is_node(H.e[k])) continue;
+            if (!RC_SLAB_SELECT && !H.h[k]) continue;
+            const uint32_t first = H.e[k] & ((1u << 26) - 1u), count = H.h[k] ? (H.e[k] >> 26) & 31u : 0u;
+            const uint32_t id = S.R.id;
+            if (test_leaf<ANY, COUNT, DEC64>(tris, first, count, o, d, S.tmin, S.best, S.R, n_tri)) return S.R;
+            if (!ANY && S.R.id != id) trav_cull(S);
+            H.h[k] = false;
+        }
+        if (!take_children<true>(S, H, M)) {
+            S.R.overflow = true;
+            return S.R;
+        }
+    }
+    return S.R;
+}
+
 // A traversal parked mid-way (the extension kernel's step budget ran out):
-// 32 words per ray, written and read as eight 16-byte vectors.  Words: 0 the
-// queue entry, 1 the current entry, 2 the stack size, 3 the best hit's id,
-// 4..6 its t, u, v, 7 the cull distance, 8..9 the best distance (a double
-// with the FP64 decision, else a float in word 8), 10.. the register stack
-// (top first), then the LDS rows in their order (only the first sp - kRegStack
-// are meaningful); word 30 the best hit's w, word 31 the leaf set aside.
-constexpr int kParkWords = 32;
-constexpr int kParkW = 30;
+// 32 words per ray (36 with more stack registers), written and read as 16-byte
+// vectors.  Words: 0 the
+// queue entry, 1 the current entry, 2 the stack's rows in use, 3 the best hit's
+// id, 4..6 its t, u, v, 7 unused, 8..9 the best distance of the FP64 decision,
+// 10.. the register stack (top first), then the memory rows in their order
+// (only those in use are meaningful); the last two words the best hit's w and the
+// leaf set aside.
+constexpr int kParkWords = RC_REG_STACK > 1 ? 36 : 32;
+constexpr int kParkW = kParkWords - 2;
 static_assert(10 + kRegStack + kLdsStack <= kParkW, "a parked traversal does not fit its record");
 
 // Word w of a parked record (compile-time w after unrolling).
 template <bool DEC64>
-__device__ __forceinline__ uint32_t park_word(const Trav<DEC64>& S, uint32_t entry, const uint32_t* stack, int stride,
-                                              int w) {
+__device__ __forceinline__ uint32_t park_word(const Trav<DEC64>& S, uint32_t entry, const StackMem& M, int w) {
     if (w == 0) return entry;
     if (w == 1) return S.cur;
-    if (w == 2) return uint32_t(S.sp);
+    if (w == 2) return uint32_t(S.stack.p - M.base) / uint32_t(M.stride);
     if (w == 3) return S.R.id;
     if (w == 4) return __float_as_uint(S.R.t);
     if (w == 5) return __float_as_uint(S.R.u);
     if (w == 6) return __float_as_uint(S.R.v);
-    if (w == 7) return __float_as_uint(S.cull);
+    if (w == 7) return 0u;
     if (w == 8 || w == 9) {
         if constexpr (DEC64) {
             const unsigned long long b = __double_as_longlong(S.best);
             return w == 8 ? uint32_t(b) : uint32_t(b >> 32);
         } else {
-            return w == 8 ? __float_as_uint(S.best) : 0u;
+            return 0u;
         }
     }
     if (w == kParkW) return __float_as_uint(S.R.w);
     if (w == kParkW + 1) return S.leaf;
-    if (w < 10 + kRegStack) return S.reg[w - 10];
-    const int j = w - 10 - kRegStack;  // LDS row
-    return j < kLdsStack && j < S.sp - kRegStack ? stack[j * stride] : 0u;
+    if (w < 10 + kRegStack) return S.stack.reg[w - 10];
+    const int j = w - 10 - kRegStack;  // memory row
+    const int p = M.base + j * M.stride;
+    return j < kLdsStack && p < S.stack.p ? M.at(p) : 0u;
 }
 
 template <bool DEC64>
-__device__ __forceinline__ void trav_park(const Trav<DEC64>& S, uint32_t entry, const uint32_t* stack, int stride,
+__device__ __forceinline__ void trav_park(const Trav<DEC64>& S, uint32_t entry, const StackMem& M,
                                           uint32_t* __restrict__ rec) {
     uint4* r = reinterpret_cast<uint4*>(rec);
 #pragma unroll
     for (int q = 0; q < kParkWords / 4; ++q)
-        st_stream(r + q, make_uint4(park_word(S, entry, stack, stride, 4 * q),
-                                    park_word(S, entry, stack, stride, 4 * q + 1),
-                                    park_word(S, entry, stack, stride, 4 * q + 2),
-                                    park_word(S, entry, stack, stride, 4 * q + 3)));
+        st_stream(r + q, make_uint4(park_word(S, entry, M, 4 * q), park_word(S, entry, M, 4 * q + 1),
+                                    park_word(S, entry, M, 4 * q + 2), park_word(S, entry, M, 4 * q + 3)));
 }
 
 template <bool DEC64>
-__device__ __forceinline__ void unpark_word(Trav<DEC64>& S, uint32_t* stack, int stride, int w, uint32_t v,
-                                            uint32_t& best_lo) {
+__device__ __forceinline__ void unpark_word(Trav<DEC64>& S, const StackMem& M, int w, uint32_t v, uint32_t& best_lo) {
     if (w == 1) S.cur = v;
-    else if (w == 2) S.sp = int(v);
+    else if (w == 2) S.stack.p = M.base + int(v) * M.stride;
     else if (w == 3) S.R.id = v;
     else if (w == 4) S.R.t = __uint_as_float(v);
     else if (w == 5) S.R.u = __uint_as_float(v);
     else if (w == 6) S.R.v = __uint_as_float(v);
-    else if (w == 7) S.cull = __uint_as_float(v);
     else if (w == kParkW) S.R.w = __uint_as_float(v);
     else if (w == kParkW + 1) S.leaf = v;
-    else if (w == 8) {
-        best_lo = v;
-        if constexpr (!DEC64) S.best = __uint_as_float(v);
-    } else if (w == 9) {
+    else if (w == 8) best_lo = v;
+    else if (w == 9) {
         if constexpr (DEC64) S.best = __longlong_as_double((long long)(uint64_t(best_lo) | (uint64_t(v) << 32)));
     } else if (w >= 10 && w < 10 + kRegStack) {
-        S.reg[w - 10] = v;
+        S.stack.reg[w - 10] = v;
     } else if (w >= 10 + kRegStack) {
         const int j = w - 10 - kRegStack;
-        if (j < kLdsStack && j < S.sp - kRegStack) stack[j * stride] = v;
+        const int p = M.base + j * M.stride;
+        if (j < kLdsStack && p < S.stack.p) M.at(p) = v;
     }
 }
 
 // Resumes a parked traversal: S must have been begun on the same ray
 // (trav_begin), which restores the ray's own fields; this restores the rest
-// and the lane's LDS rows (word 0, the queue entry, is the caller's).
+// and the lane's stack rows (word 0, the queue entry, is the caller's).
 template <bool DEC64>
-__device__ __forceinline__ void trav_unpark(Trav<DEC64>& S, const uint32_t* __restrict__ rec, uint32_t* stack,
-                                            int stride) {
+__device__ __forceinline__ void trav_unpark(Trav<DEC64>& S, const uint32_t* __restrict__ rec, const StackMem& M) {
     const uint4* r = reinterpret_cast<const uint4*>(rec);
     uint32_t best_lo = 0;
 #pragma unroll
     for (int q = 0; q < kParkWords / 4; ++q) {
         const uint4 v = ld_stream(r + q);
-        unpark_word(S, stack, stride, 4 * q, v.x, best_lo);
-        unpark_word(S, stack, stride, 4 * q + 1, v.y, best_lo);
-        unpark_word(S, stack, stride, 4 * q + 2, v.z, best_lo);
-        unpark_word(S, stack, stride, 4 * q + 3, v.w, best_lo);
+        unpark_word(S, M, 4 * q, v.x, best_lo);
+        unpark_word(S, M, 4 * q + 1, v.y, best_lo);
+        unpark_word(S, M, 4 * q + 2, v.z, best_lo);
+        unpark_word(S, M, 4 * q + 3, v.w, best_lo);
     }
+    if (S.R.id != kNoHit) trav_cull(S);
 }
 
 template <bool ANY, bool COUNT, bool DEC64>
 __device__ __forceinline__ TraceResult traverse_ifif(const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
-                                                     float3 o, float3 d, float tmin, float tmax, uint32_t* stack,
-                                                     int stride, int max_depth, uint32_t& n_rec, uint32_t& n_tri,
-                                                     const uint4* top = nullptr, uint32_t ntop = 0) {
+                                                     float3 o, float3 d, float tmin, float tmax, const StackMem& M,
+                                                     uint32_t& n_rec, uint32_t& n_tri, const uint4* top, uint32_t ntop,
+                                                     bool late) {
     Trav<DEC64> S;
-    trav_begin(S, o, d, tmin, tmax, top, ntop);
-    while (!trav_step<ANY, COUNT, DEC64>(S, nodes, tris, stack, stride, max_depth, n_rec, n_tri)) {
+    trav_begin(S, nodes, M, o, d, tmin, tmax, top, ntop, late);
+    while (!trav_step<ANY, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
     }
     return S.R;
 }
 
-// Closest hit (ANY = false) or any hit of one ray.  stack: the lane's memory
-// part of the stack, entry k at stack[k * stride]; max_depth: entries the
-// stack may hold in all (registers and memory).
+// Closest hit (ANY = false) or any hit of one ray, with the lane's stack
+// memory M.  late: whether rays may have a tmin > 0.
 template <bool ANY, bool COUNT, bool DEC64>
 __device__ __forceinline__ TraceResult traverse(const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
-                                                float3 o, float3 d, float tmin, float tmax, uint32_t* stack,
-                                                int stride, int max_depth, uint32_t& n_rec, uint32_t& n_tri,
-                                                const uint4* top = nullptr, uint32_t ntop = 0) {
-#if RC_QNODE
-    return traverse_ifif<ANY, COUNT, DEC64>(nodes, tris, o, d, tmin, tmax, stack, stride, max_depth, n_rec, n_tri,
-                                            top, ntop);
-#else
-    if (RC_TRAV_IFIF)
-        return traverse_ifif<ANY, COUNT, DEC64>(nodes, tris, o, d, tmin, tmax, stack, stride, max_depth, n_rec,
-                                                n_tri);
-    return traverse_inline<ANY, COUNT, DEC64>(nodes, tris, o, d, tmin, tmax, stack, stride, max_depth, n_rec, n_tri);
-#endif
+                                                float3 o, float3 d, float tmin, float tmax, const StackMem& M,
+                                                uint32_t& n_rec, uint32_t& n_tri, const uint4* top, uint32_t ntop,
+                                                bool late) {
+    if (!RC_QNODE && !RC_TRAV_IFIF)
+        return traverse_inline<ANY, COUNT, DEC64>(nodes, tris, o, d, tmin, tmax, M, n_rec, n_tri);
+    return traverse_ifif<ANY, COUNT, DEC64>(nodes, tris, o, d, tmin, tmax, M, n_rec, n_tri, top, ntop, late);
 }
 
 #if RC_QNODE
@@ -1038,99 +1073,42 @@ __device__ __forceinline__ TraceResult traverse(const NodeT* __restrict__ nodes,
 template <bool COUNT>
 __device__ __forceinline__ TraceResult traverse_packet(const QNode* __restrict__ nodes,
                                                        const TriRec* __restrict__ tris, float3 o, float3 d,
-                                                       float tmin, float tmax, uint32_t* stack, int stride,
-                                                       int max_depth, uint32_t& n_rec, uint32_t& n_tri) {
-    const float INF = __builtin_inff();
-    const float3 inv = safe_inv(d);
-    tmin = fmaxf(tmin, 0.0f);
-    float best = tmax;
-    float cull = initial_cull<false>(tmax);
-    TraceResult R{tmax, 0.0f, 0.0f, kNoHit, false, 1.0f};
-    uint32_t cur = 0;  // root: interior record 0 (wave-uniform, as sp)
-    int sp = 0;
+                                                       float tmin, float tmax, const StackMem& M, uint32_t& n_rec,
+                                                       uint32_t& n_tri) {
+    Trav<false> S;
+    trav_begin(S, nodes, M, o, d, tmin, tmax, nullptr, 0, false);
+    S.cur = 0;  // wave-uniform, as the stack
     for (;;) {
-        if (!(cur & kLeafTag)) {
-            const uint4* p = reinterpret_cast<const uint4*>(nodes + cur);
-            const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
+        if (is_node(S.cur)) {
             if (COUNT) n_rec += kWidth;
-            const float ax = __uint_as_float((q0.w & 0xFFu) << 23) * inv.x;
-            const float ay = __uint_as_float(((q0.w >> 8) & 0xFFu) << 23) * inv.y;
-            const float az = __uint_as_float(((q0.w >> 16) & 0xFFu) << 23) * inv.z;
-            const float bx = (__uint_as_float(q0.x) - o.x) * inv.x;
-            const float by = (__uint_as_float(q0.y) - o.y) * inv.y;
-            const float bz = (__uint_as_float(q0.z) - o.z) * inv.z;
-            const uint32_t nx = inv.x < 0.0f ? q1.w : q1.x, fx = inv.x < 0.0f ? q1.x : q1.w;
-            const uint32_t ny = inv.y < 0.0f ? q2.x : q1.y, fy = inv.y < 0.0f ? q1.y : q2.x;
-            const uint32_t nz = inv.z < 0.0f ? q2.y : q1.z, fz = inv.z < 0.0f ? q1.z : q2.y;
-            auto slab_q = [&](int k, uint32_t e) {
-                const float tnx = fmaf(float((nx >> (8 * k)) & 0xFFu), ax, bx);
-                const float tfx = fmaf(float((fx >> (8 * k)) & 0xFFu), ax, bx);
-                const float tny = fmaf(float((ny >> (8 * k)) & 0xFFu), ay, by);
-                const float tfy = fmaf(float((fy >> (8 * k)) & 0xFFu), ay, by);
-                const float tnz = fmaf(float((nz >> (8 * k)) & 0xFFu), az, bz);
-                const float tfz = fmaf(float((fz >> (8 * k)) & 0xFFu), az, bz);
-                const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin));
-                const float tf = fminf(fminf(tfx, tfy), fminf(tfz, cull));
-                return tn <= tf * 1.000002f && e != kEmptyChild ? tn : INF;
-            };
-            const float t0 = slab_q(0, q3.x), t1 = slab_q(1, q3.y), t2 = slab_q(2, q3.z), t3 = slab_q(3, q3.w);
-            // per child: entered by any lane (m), the first active lane's
-            // distance (r) and the entry (e), all wave-uniform
-            uint32_t m0 = __ballot(t0 < INF) != 0, m1 = __ballot(t1 < INF) != 0;
-            uint32_t m2 = __ballot(t2 < INF) != 0, m3 = __ballot(t3 < INF) != 0;
-            float r0 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t0)));
-            float r1 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t1)));
-            float r2 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t2)));
-            float r3 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t3)));
-            // the entry of an entered child, else kEmptyChild (which sorts
-            // with the misses)
-            uint32_t e0 = m0 ? __builtin_amdgcn_readfirstlane(q3.x) : kEmptyChild;
-            uint32_t e1 = m1 ? __builtin_amdgcn_readfirstlane(q3.y) : kEmptyChild;
-            uint32_t e2 = m2 ? __builtin_amdgcn_readfirstlane(q3.z) : kEmptyChild;
-            uint32_t e3 = m3 ? __builtin_amdgcn_readfirstlane(q3.w) : kEmptyChild;
-            order2(r0, e0, r1, e1);
-            order2(r2, e2, r3, e3);
-            order2(r0, e0, r2, e2);
-            order2(r1, e1, r3, e3);
-            order2(r1, e1, r2, e2);
-            // far to near: the nearest entered child is visited next, the
-            // others pushed farthest first
-            uint32_t next = kEmptyChild;
-            bool overflow = false;
-            auto take = [&](uint32_t e) {
-                if (e == kEmptyChild) return;
-                if (next != kEmptyChild) {
-                    if (sp >= max_depth) {
-                        overflow = true;
-                        return;
-                    }
-                    stack[sp * stride] = next;
-                    ++sp;
-                }
-                next = e;
-            };
-            take(e3);
-            take(e2);
-            take(e1);
-            take(e0);
-            if (overflow) {
-                R.overflow = true;
-                return R;
+            Hits H;
+            node_hits<false>(S, nodes, S.cur, H);
+            // entered by any lane; the first active lane's distance and the
+            // entry, all wave-uniform
+#pragma unroll
+            for (int k = 0; k < kWidth; ++k) {
+                H.h[k] = __ballot(H.h[k]) != 0;
+                H.t[k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(H.t[k])));
+                H.e[k] = __builtin_amdgcn_readfirstlane(H.e[k]);
             }
-            if (next != kEmptyChild) {
-                cur = next;
-                continue;
+            if (!take_children<true>(S, H, M)) {
+                S.R.overflow = true;
+                return S.R;
             }
         } else {
-            // every active lane tests the leaf: a lane whose ray misses the
-            // leaf's box finds no hit there it would not also find through
-            // its own traversal
-            test_leaf<false, COUNT, false>(tris, cur & 0x03FFFFFFu, (cur >> 26) & 0x1Fu, o, d, tmin, 0.0f, best, cull,
-                                           R, n_tri);
+            if (is_leaf(S.cur)) {
+                // every active lane tests the leaf: a lane whose ray misses
+                // the leaf's box finds no hit there it would not also find
+                // through its own traversal
+                const uint32_t id = S.R.id;
+                test_leaf<false, COUNT, false>(tris, S.cur & 0x03FFFFFFu, (S.cur >> 26) & 0x1Fu, o, d, S.tmin, S.best,
+                                               S.R, n_tri);
+                if (S.R.id != id) trav_cull(S);
+            }
+            S.cur = stack_pop(S.stack, M);
         }
-        if (sp == 0) return R;
-        --sp;
-        cur = __builtin_amdgcn_readfirstlane(stack[sp * stride]);
+        S.cur = __builtin_amdgcn_readfirstlane(S.cur);
+        if (S.cur == kEmptyChild) return S.R;
     }
 }
 #endif

@@ -95,7 +95,7 @@ struct rc_ctx {
 
     // traversal stack entries held on chip before a ray goes to the deep-stack kernel
     int stack_depth() const {
-        return tuning.stack_limit ? int(tuning.stack_limit) : rcd::kOnChipStack;
+        return tuning.stack_limit ? std::min(int(tuning.stack_limit), rcd::kLdsStack) : rcd::kLdsStack;
     }
     rc_stats stats{};
     DevCounters* counters = nullptr;  // device
@@ -176,7 +176,7 @@ struct TraceLaunch {
     uint32_t* deep_stack = nullptr;
     DevCounters* ctr = nullptr;
     hipStream_t stream = nullptr;
-    int max_depth = rcd::kOnChipStack;  // on-chip stack entries before the deep-stack kernel
+    int max_depth = rcd::kLdsStack;  // on-chip stack entries before the deep-stack kernel
     uint32_t max_blocks = 1;            // grid limit; the kernel's grid-stride loop covers the rest
     bool counting = false;
     bool dec64 = false;

@@ -37,7 +37,6 @@ constexpr float kPi = 3.14159265358979323846f;
 #endif
 constexpr uint32_t kExtBlockDefault = RC_EXT_BLOCK;
 constexpr uint32_t kShadowBlockDefault = RC_SHADOW_BLOCK;
-constexpr int kLdsRows = kLdsStack > 0 ? kLdsStack : 1;  // LDS stack entries per thread (at least one row)
 // Minimum waves per SIMD the traversal kernels are compiled for, by triangle
 // decision.  FP32: 8, which caps them at 64 VGPRs with no spills (59-62 used;
 // 7 waves at 70 without the cap), 11% faster on the 2M-triangle terrain at
@@ -542,12 +541,13 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
     DevCounters* __restrict__ ctr, uint32_t cin, uint32_t cout, CacheIO CI, float* __restrict__ W,
     rc_ray* __restrict__ cam_rays, float4* __restrict__ cam_st, ParkIO PK) {
     static_assert(!(PARK && CAM), "the camera bounce does not park");
-    __shared__ uint32_t stack[kLdsRows * BLOCK];
+    __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = ctr->queue_count[cin];
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit);
     const uint32_t i = trace_block<BLOCK>(n) * BLOCK + threadIdx.x;
     if (i == 0) atomicAdd(&ctr->ext_rays, (unsigned long long)n);
     uint32_t n_rec = 0, n_tri = 0;
@@ -563,11 +563,10 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
         if (i < n) {
             const float4* rp = reinterpret_cast<const float4*>(rays + i);
             const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-            trav_begin(S, f3(r0), f3(r1), r0.w, r1.w, top, ntop);
+            trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
             uint32_t steps = 0;
             do {
-                done = trav_step<false, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, P.stack_limit,
-                                                      n_rec, n_tri);
+                done = trav_step<false, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
             } while (keep_going<false>(done, ++steps, PK.steps));
         }
         // every thread of the block reserves (one atomic per block)
@@ -575,11 +574,10 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
         bool parked = false;
         if (!done) {
             if (pos < PK.cap) {
-                trav_park(S, i, stack + threadIdx.x, BLOCK, PK.rec + size_t(pos) * kParkWords);
+                trav_park(S, i, M, PK.rec + size_t(pos) * kParkWords);
                 parked = true;
             } else {
-                while (!trav_step<false, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, P.stack_limit,
-                                                       n_rec, n_tri)) {
+                while (!trav_step<false, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
                 }
             }
         }
@@ -609,13 +607,12 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
         TraceResult R;
 #if RC_QNODE && RC_PACKET_CAMERA
         if constexpr (CAM && !DEC64) {  // a wave holds one pixel's samples: one packet
-            R = traverse_packet<COUNT>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, stack + threadIdx.x, BLOCK,
-                                       min(P.stack_limit, kLdsRows), n_rec, n_tri);
+            R = traverse_packet<COUNT>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, M, n_rec, n_tri);
         } else
 #endif
         {
-            R = traverse<false, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, stack + threadIdx.x, BLOCK,
-                                              P.stack_limit, n_rec, n_tri, top, ntop);
+            R = traverse<false, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, M, n_rec, n_tri, top, ntop,
+                                              false);
         }
         if (R.overflow) {
             if (CAM) {  // the deep-stack kernel and k_shade_listed read the entry
@@ -651,13 +648,14 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
     const DevMaterial* __restrict__ mats, rc_ray* __restrict__ rays_out, float4* __restrict__ st_out,
     rc_ray* __restrict__ srays, float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list,
     DevCounters* __restrict__ ctr, uint32_t cout, CacheIO CI, ParkIO in, ParkIO out) {
-    __shared__ uint32_t stack[kLdsRows * BLOCK];
+    __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = min(ctr->park_count[in.which], in.cap);
     if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&ctr->park_total, (unsigned long long)n);
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit);
     const uint32_t q = blockIdx.x * uint32_t(BLOCK) + threadIdx.x;
     uint32_t n_rec = 0, n_tri = 0;
     ShadeOut O;
@@ -673,13 +671,12 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
         {
             const float4* rp = reinterpret_cast<const float4*>(rays + i);
             const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-            trav_begin(S, f3(r0), f3(r1), r0.w, r1.w, top, ntop);
+            trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
         }
-        trav_unpark(S, rec, stack + threadIdx.x, BLOCK);
+        trav_unpark(S, rec, M);
         uint32_t steps = 0;
         do {
-            done = trav_step<false, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, P.stack_limit, n_rec,
-                                                  n_tri);
+            done = trav_step<false, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
         } while (PARK ? keep_going<false>(done, ++steps, out.steps) : !done);
     }
     bool parked = false;
@@ -687,11 +684,10 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
         const uint32_t pos = block_append<BLOCK>(!done, &ctr->park_count[out.which], append_scratch);
         if (!done) {
             if (pos < out.cap) {
-                trav_park(S, i, stack + threadIdx.x, BLOCK, out.rec + size_t(pos) * kParkWords);
+                trav_park(S, i, M, out.rec + size_t(pos) * kParkWords);
                 parked = true;
             } else {
-                while (!trav_step<false, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, P.stack_limit,
-                                                       n_rec, n_tri)) {
+                while (!trav_step<false, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
                 }
             }
         }
@@ -766,11 +762,12 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
                                                        const float4* __restrict__ scontrib, float4* __restrict__ L,
                                                        uint32_t* __restrict__ ovf_list, DevCounters* __restrict__ ctr,
                                                        uint8_t* __restrict__ occ_out, int stack_limit, ParkIO PK) {
-    __shared__ uint32_t stack[kLdsRows * BLOCK];
+    __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = ctr->queue_count[2];
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit);
     const uint32_t i = trace_block<BLOCK>(n) * BLOCK + threadIdx.x;
     if (i == 0) atomicAdd(&ctr->shadow_rays, (unsigned long long)n);
     uint32_t n_rec = 0, n_tri = 0;
@@ -781,22 +778,20 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
         if (i < n) {
             const float4* rp = reinterpret_cast<const float4*>(srays + i);
             const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-            trav_begin(S, f3(r0), f3(r1), r0.w, r1.w, top, ntop);
+            trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
             uint32_t steps = 0;
             do {
-                done = trav_step<true, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, stack_limit, n_rec,
-                                                     n_tri);
+                done = trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
             } while (keep_going<true>(done, ++steps, PK.steps));
         }
         const uint32_t pos = block_append<BLOCK>(!done, &ctr->park_count[PK.which], append_scratch);
         bool parked = false;
         if (!done) {
             if (pos < PK.cap) {
-                trav_park(S, i, stack + threadIdx.x, BLOCK, PK.rec + size_t(pos) * kParkWords);
+                trav_park(S, i, M, PK.rec + size_t(pos) * kParkWords);
                 parked = true;
             } else {
-                while (!trav_step<true, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, stack_limit, n_rec,
-                                                      n_tri)) {
+                while (!trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
                 }
             }
         }
@@ -807,8 +802,9 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
     } else if (i < n) {
         const float4* rp = reinterpret_cast<const float4*>(srays + i);
         float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-        TraceResult R = traverse<true, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, stack + threadIdx.x,
-                                                     BLOCK, stack_limit, n_rec, n_tri, top, ntop);
+        TraceResult R =
+            traverse<true, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, M, n_rec, n_tri, top, ntop,
+                                              false);
         if (R.overflow) ovf_list[atomicAdd(&ctr->ovf_count, 1u)] = i;
         else shadow_result(i, R.id != kNoHit, scontrib, L, occ_out);
     }
@@ -825,13 +821,14 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow_resume(
     const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris, const rc_ray* __restrict__ srays,
     const float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list,
     DevCounters* __restrict__ ctr, uint8_t* __restrict__ occ_out, int stack_limit, ParkIO in, ParkIO out) {
-    __shared__ uint32_t stack[kLdsRows * BLOCK];
+    __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = min(ctr->park_count[in.which], in.cap);
     if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&ctr->park_total, (unsigned long long)n);
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit);
     const uint32_t q = blockIdx.x * uint32_t(BLOCK) + threadIdx.x;
     uint32_t n_rec = 0, n_tri = 0;
     Trav<DEC64> S;
@@ -843,12 +840,12 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow_resume(
         {
             const float4* rp = reinterpret_cast<const float4*>(srays + i);
             const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-            trav_begin(S, f3(r0), f3(r1), r0.w, r1.w, top, ntop);
+            trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
         }
-        trav_unpark(S, rec, stack + threadIdx.x, BLOCK);
+        trav_unpark(S, rec, M);
         uint32_t steps = 0;
         do {
-            done = trav_step<true, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, stack_limit, n_rec, n_tri);
+            done = trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
         } while (PARK ? keep_going<true>(done, ++steps, out.steps) : !done);
     }
     bool parked = false;
@@ -856,11 +853,10 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow_resume(
         const uint32_t pos = block_append<BLOCK>(!done, &ctr->park_count[out.which], append_scratch);
         if (!done) {
             if (pos < out.cap) {
-                trav_park(S, i, stack + threadIdx.x, BLOCK, out.rec + size_t(pos) * kParkWords);
+                trav_park(S, i, M, out.rec + size_t(pos) * kParkWords);
                 parked = true;
             } else {
-                while (!trav_step<true, COUNT, DEC64>(S, nodes, tris, stack + threadIdx.x, BLOCK, stack_limit, n_rec,
-                                                      n_tri)) {
+                while (!trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
                 }
             }
         }

@@ -40,21 +40,22 @@ __device__ __forceinline__ void store_result(bool any, const TraceResult& R, uin
 }
 
 template <bool ANY, bool COUNT, bool DEC64>
-__global__ __launch_bounds__(kBlock) void k_trace(const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
+__global__ __launch_bounds__(kBlock, DEC64 ? 1 : 8) void k_trace(const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
                                                   const rc_ray* __restrict__ rays, const uint32_t* n_dev,
                                                   uint32_t n_host, rc_hit* __restrict__ hits, uint8_t* __restrict__ occ,
                                                   uint32_t* __restrict__ ovf_list, DevCounters* __restrict__ ctr,
                                                   int max_depth) {
-    __shared__ uint32_t stack[(kLdsStack > 0 ? kLdsStack : 1) * kBlock];
+    __shared__ uint32_t stack[kLdsStack * kBlock];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t ntop = load_top(nodes, top);
+    const StackMem M = stack_mem(stack, threadIdx.x, kBlock, max_depth);
     const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
     uint32_t n_rec = 0, n_tri = 0;
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
         float4 r0 = rp[0], r1 = rp[1];
-        TraceResult R = traverse<ANY, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, stack + threadIdx.x,
-                                                    kBlock, max_depth, n_rec, n_tri, top, ntop);
+        TraceResult R = traverse<ANY, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, M, n_rec, n_tri, top, ntop,
+                                                    true);
         if (R.overflow) {
             ovf_list[atomicAdd(&ctr->ovf_count, 1u)] = i;
             continue;
@@ -78,13 +79,14 @@ __global__ __launch_bounds__(64) void k_trace_deep(const NodeT* __restrict__ nod
     const uint32_t n = ctr->ovf_count;
     const uint32_t gtid = blockIdx.x * 64 + threadIdx.x, nthreads = gridDim.x * 64;
     if (gtid == 0 && n) atomicAdd(&ctr->ovf_total, (unsigned long long)n);
+    const StackMem M = stack_mem(gstack, gtid, int(nthreads), kDeepStack);
     uint32_t n_rec = 0, n_tri = 0;
     for (uint32_t k = gtid; k < n; k += nthreads) {
         uint32_t i = ovf_list[k];
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
         float4 r0 = rp[0], r1 = rp[1];
-        TraceResult R = traverse<ANY, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, gstack + gtid, nthreads,
-                                                    kRegStack + kDeepStack, n_rec, n_tri);
+        TraceResult R = traverse<ANY, COUNT, DEC64>(nodes, tris, f3(r0), f3(r1), r0.w, r1.w, M, n_rec, n_tri, nullptr, 0,
+                                                    true);
         if (R.overflow) {
             ctr->error = 1;  // unreachable: the upload rejects trees this deep
             continue;
