@@ -173,10 +173,11 @@ typedef struct rc_point_light {
  * samples per pixel (0, the default: each frame takes as many samples per pass
  * as keep a pass within 2^26 paths, 2^21 for rc_raytrace; else 1..64), grid
  * limit of the ray-query kernels in blocks per CU, the traversal stack
- * entries held on chip (registers and LDS) before a ray is handed to the
- * deep-stack kernel, which walks it again with a stack in global memory
- * (0, the default: all the build holds; 1..that depth: fewer, which sends
- * more rays down the deep-stack path and changes no result), and the
+ * entries held on chip (registers and LDS) before a ray's stack goes on in
+ * global memory: in one of a launch's 2048 spill slots or, when they are
+ * taken or the limit is below 4, by a second walk in the deep-stack kernel
+ * (0, the default: all the build holds, 19; 1..20: fewer, which sends more
+ * rays that way and changes no result), and the
  * traversal steps a path tracer's extension ray takes in the first kernel
  * of a bounce before it is parked and finished by a second kernel whose
  * waves hold only such long traversals (a wave with at least 8 lanes still
@@ -197,7 +198,7 @@ typedef struct rc_stats {
     uint64_t samples;            /* camera samples of the last render */
     uint64_t node_records;       /* 32-byte node records fetched (counting runs only) */
     uint64_t tri_tests;          /* 48-byte triangle records tested (counting runs only) */
-    uint64_t overflow_rays;      /* rays re-walked by the deep-stack kernel, summed over all launches of the call */
+    uint64_t overflow_rays;      /* rays whose stack outgrew the on-chip entries, summed over all launches of the call */
     uint64_t extend_launches;
     double extend_ms;            /* sum of closest-hit kernel durations (profiling on) */
     double shadow_ms;

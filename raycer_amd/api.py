@@ -617,7 +617,7 @@ class Context:
     def set_tuning(self, block=256, spp_per_pass=0, blocks_per_cu=64, stack_limit=0, park_steps=None) -> None:
         """rc_set_tuning; the defaults are the context's own (spp_per_pass 0:
         each frame chooses its pass size; stack_limit 0: the whole on-chip
-        traversal stack before the deep-stack kernel takes a ray over;
+        traversal stack before a ray's stack goes on in global memory;
         park_steps None: the library's default)."""
         t = Tuning(block, spp_per_pass, blocks_per_cu, stack_limit,
                    PARK_STEPS_DEFAULT if park_steps is None else park_steps)

@@ -88,7 +88,7 @@ __global__ void k_batch_zero(DevCounters* ctr) {
     ctr->tri_tests = 0;
     ctr->ext_rays = 0;
     ctr->shadow_rays = 0;
-    ctr->ovf_total = 0;
+    ctr->spill.total = 0;
     ctr->park_total = 0;
     ctr->ovf_count = 0;
     ctr->error = 0;
@@ -244,7 +244,7 @@ int render_batch(rc_ctx* c, const rc_scene* const* scenes, rc_film* const* films
         if (h.error) return rc_host_fail(RC_ERR_HIP, std::string(fn) + ": traversal stack exceeded the deep-stack limit");
         ext += h.ext_rays;
         shadow += h.shadow_rays;
-        ovf += h.ovf_total;
+        ovf += h.spill.total;
         parked += h.park_total;
     }
     c->stats.extension_rays = ext;

@@ -595,6 +595,19 @@ extern "C" int rc_scene_upload(rc_ctx* c, const float* v, size_t ntri, const uin
             }
         }
     }
+    // The most entries a traversal's stack can hold: below a node, all its
+    // children but the one visited, then that one's (children follow their node).
+    std::vector<uint32_t> need(nrec / kWidth, 0u);
+    for (size_t n = need.size(); n-- > 0;) {
+        uint32_t kids = 0, below = 0;
+        for (int k = 0; k < kWidth; ++k) {
+            const NodeRec& x = recs[n * kWidth + k];
+            if (x.count == kEmptyChild) continue;
+            kids += 1;
+            if (x.count == 0) below = std::max(below, need[x.link / kWidth]);
+        }
+        need[n] = (kids ? kids - 1 : 0) + below;
+    }
     // a traversal stack holds at most (kWidth - 1) entries per level
     if (depth * (kWidth - 1) >= uint32_t(kDeepStack))
         return rc_host_fail(RC_ERR_INVALID, "rc_scene_upload: BVH too deep for the traversal stack");
@@ -728,6 +741,7 @@ extern "C" int rc_scene_upload(rc_ctx* c, const float* v, size_t ntri, const uin
     s->ntri = ntri;
     s->nmat = nmat;
     s->depth = depth;
+    s->stack_need = need.empty() ? 0u : need[0];
     if (empty)
         for (int k = 0; k < 3; ++k) bmin[k] = bmax[k] = 0.0f;
     std::memcpy(s->bmin, bmin, sizeof(bmin));

@@ -98,7 +98,8 @@ struct alignas(16) DevMaterial {
 };
 
 constexpr uint32_t kNoHit = 0x7fffffffu;
-constexpr int kDeepStack = 256;  // stack entries of the overflow kernel (memory part)
+constexpr int kDeepStack = 256;  // words of a stack in global memory: a spill slot, a lane of the deep-stack kernel
+constexpr int kDeepThreads = 2048;  // such stacks of a launch
 
 // Traversal stack of one lane: the top kRegStack entries in registers, deeper
 // ones in LDS laid out [depth][lane] so a wave's accesses hit 64 distinct
@@ -107,7 +108,7 @@ constexpr int kDeepStack = 256;  // stack entries of the overflow kernel (memory
 // critical path.  Every push spills the bottom register, so the LDS rows are
 // the stack's capacity; registers start as kEmptyChild, and popping that is
 // the end of the stack (no entry count).  A ray whose stack would outgrow
-// kLdsStack entries is handed to the deep-stack kernel.  One register: each
+// kLdsStack entries moves them to global memory (stack_spill).  One register: each
 // more costs a move per push and pop.  19 rows: with them eight 256-thread
 // blocks of the traversal kernels fill the 160 KB of a CU.
 #ifndef RC_REG_STACK
@@ -386,17 +387,29 @@ constexpr float kTieWindow = 4.0f / 16777216.0f;
 // lanes, row r of the lane at byte offset base + r * stride (base = 4 * lane <
 // stride).  end is the offset past row `limit` of every lane (uniform), so a
 // lane whose next free row is at p may push m entries exactly when
-// p + m * stride < end.
+// p + m * stride < end.  spill: the launch's kDeepThreads stacks in global
+// memory, handed out by count->claimed, for lanes whose rows are full; null:
+// none.
+struct SpillCount {
+    unsigned long long total;  // rays whose stack outgrew its rows
+    uint32_t claimed;          // stacks the launch's rays asked for
+};
 struct StackMem {
     uint32_t* array;
     int base, stride, end;
+    uint32_t* spill;
+    SpillCount* count;
     __device__ __forceinline__ uint32_t& at(int p) const {
         return *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(array) + uint32_t(p));
     }
 };
-__device__ __forceinline__ StackMem stack_mem(uint32_t* array, uint32_t lane, int lanes, int limit) {
-    return StackMem{array, int(4 * lane), 4 * lanes, 4 * lanes * (limit + 1)};
+__device__ __forceinline__ StackMem stack_mem(uint32_t* array, uint32_t lane, int lanes, int limit,
+                                              uint32_t* spill = nullptr, SpillCount* count = nullptr) {
+    return StackMem{array, int(4 * lane), 4 * lanes, 4 * lanes * (limit + 1), spill, count};
 }
+// Rows the three entries of a node visit need above a stack just spilled: with
+// fewer nothing is spilled.
+constexpr int kSpillRows = 4;
 
 // The stack's registers and the offset of its next free row.
 struct Stack {
@@ -645,7 +658,7 @@ template <bool DEC64>
 struct Trav {
     float3 o, d;
     float3 inv;   // 1 / d, no zero component (safe_inv), scaled
-    float scale;  // the power of two
+    uint32_t scale_spill;  // bits of the power of two (trav_scale); its mantissa's: the spilled stack (stack_spill)
     float tmin;
     bool late;    // wave-uniform: some ray of the wave has a tmin > 0, entries are held against it
     float cull;   // boxes entered beyond it are skipped (scaled, below 1)
@@ -674,10 +687,70 @@ __device__ __forceinline__ uint32_t load_top(const N* __restrict__ nodes, uint4*
     }
 }
 
+constexpr uint32_t kSpillMask = 0x007fffffu;
+template <bool DEC64>
+__device__ __forceinline__ float trav_scale(const Trav<DEC64>& S) {
+    return __uint_as_float(S.scale_spill & ~kSpillMask);
+}
+
 // The cull distance for R.t (the best hit's, or tmax).
 template <bool DEC64>
 __device__ __forceinline__ void trav_cull(Trav<DEC64>& S) {
-    S.cull = fminf(cull_at<DEC64>(S.R.t) * S.scale, 0.99999994f);
+    S.cull = fminf(cull_at<DEC64>(S.R.t) * trav_scale(S), 0.99999994f);
+}
+
+// A stack whose rows are full: they move to a slot of global memory and the
+// lane goes on with empty rows; when those are used up the rows come back
+// (stack_reload).  The word in scale_spill: 1 + the slot in bits 9.., the
+// slot's words in use below (each block of rows is followed by its length);
+// 0 while nothing was spilled.  False when the launch's slots are all taken,
+// the slot is full or the rows are too few: then the deep-stack kernel walks
+// the ray again.  Before, it walked all of them: the few rays that outgrow the
+// rows are a launch's longest, and walked twice, the second time alone on the
+// chip.  An any-hit query over 777,777 segments in 200,000 random triangles
+// takes 446 us against 514; the loop itself pays nothing (the word lies in
+// unused bits and is looked at where a traversal ends or finds no room).
+template <bool DEC64>
+__device__ __forceinline__ bool stack_spill(Trav<DEC64>& S, const StackMem& M) {
+    if (!M.spill || M.end < (kSpillRows + 1) * M.stride) return false;
+    uint32_t w = S.scale_spill & kSpillMask;
+    if (w == 0) {
+        const uint32_t slot = atomicAdd(&M.count->claimed, 1u);
+        if (slot >= uint32_t(kDeepThreads)) return false;
+        atomicAdd(&M.count->total, 1ull);
+        w = (slot + 1u) << 9;
+    }
+    const uint32_t rows = uint32_t(S.stack.p - M.base) / uint32_t(M.stride);
+    uint32_t used = w & 511u;
+    if (used + rows + 1u > uint32_t(kDeepStack)) {
+        atomicAdd(&M.count->total, ~0ull);  // the deep-stack kernel counts it
+        return false;
+    }
+    uint32_t* q = M.spill + ((w >> 9) - 1u) * uint32_t(kDeepStack) + used;
+    for (int p = M.base; p < S.stack.p; p += M.stride) *q++ = M.at(p);
+    *q = rows;
+    S.scale_spill = (S.scale_spill & ~kSpillMask) | (w + rows + 1u);
+    M.at(M.base) = kEmptyChild;  // below the register entries
+    S.stack.p = M.base + M.stride;
+    return true;
+}
+
+// The rows spilled last, back into the used-up stack, and its top entry into
+// S.cur; false when there are none.
+template <bool DEC64>
+__device__ __forceinline__ bool stack_reload(Trav<DEC64>& S, const StackMem& M) {
+    const uint32_t w = S.scale_spill & kSpillMask;
+    if ((w & 511u) == 0) return false;
+    const uint32_t* q = M.spill + ((w >> 9) - 1u) * uint32_t(kDeepStack) + (w & 511u) - 1u;
+    const uint32_t rows = *q;
+    q -= rows;
+    S.stack.p = M.base;
+    for (uint32_t r = 0; r < rows; ++r, S.stack.p += M.stride) M.at(S.stack.p) = q[r];
+    S.scale_spill -= rows + 1u;
+#pragma unroll
+    for (int k = 0; k < kRegStack; ++k) stack_pop(S.stack, M);  // refills the registers
+    S.cur = stack_pop(S.stack, M);
+    return true;
 }
 
 // Distance at which a ray (origin o, 1/d inv) has left the root's box, a hair
@@ -716,8 +789,8 @@ __device__ __forceinline__ void trav_begin(Trav<DEC64>& S, const NodeT* __restri
     const float3 inv = safe_inv(d);
     const float T0 = cull_at<DEC64>(tmax), exit = scene_exit(nodes, o, inv);
     const float T = fminf(fmaxf(exit < T0 ? exit : T0, 1e-12f), 3e37f);
-    S.scale = __uint_as_float((253u << 23) - (__float_as_uint(T) & 0x7f800000u));  // 2^-k, 2^(k-1) <= T < 2^k
-    S.inv = inv * S.scale;
+    S.scale_spill = (253u << 23) - (__float_as_uint(T) & 0x7f800000u);  // 2^-k, 2^(k-1) <= T < 2^k
+    S.inv = inv * trav_scale(S);
     trav_cull(S);
     S.cur = tmax < S.tmin ? kEmptyChild : 0u;  // root: interior record 0; an empty interval has no hit
     S.leaf = kEmptyChild;
@@ -747,7 +820,7 @@ __device__ __forceinline__ void node_hits(const Trav<DEC64>& S, const NodeT* __r
     // test could still hit.
     auto enter = [&](int k, float tnx, float tny, float tnz, float tfx, float tfy, float tfz) {
         H.t[k] = fmaxf(fmaxf(clamp01(tnx), tny), tnz);
-        if (S.late) H.t[k] = fmaxf(H.t[k], S.tmin * S.scale);
+        if (S.late) H.t[k] = fmaxf(H.t[k], S.tmin * trav_scale(S));
         H.h[k] = H.t[k] <= fminf(fminf(fminf(tfx, tfy), tfz) * 1.000002f, S.cull);
     };
     const uint32_t mx = uint32_t(int32_t(__float_as_uint(S.inv.x)) >> 31);
@@ -805,8 +878,9 @@ __device__ __forceinline__ void node_hits(const Trav<DEC64>& S, const NodeT* __r
 
 // The children of a visited node in H: the nearest (ANY without RC_ANY_SORT:
 // the first) becomes S.cur, the others go on the stack farthest first; with
-// none S.cur is popped.  False when the stack would outgrow its rows.
-template <bool SORT, bool DEC64>
+// none S.cur is popped.  False when the stack would outgrow its rows (SPILL:
+// and they cannot be spilled).
+template <bool SORT, bool SPILL, bool DEC64>
 __device__ __forceinline__ bool take_children(Trav<DEC64>& S, Hits& H, const StackMem& M) {
     const bool* h = H.h;
     uint32_t e0 = H.e[0], e1 = H.e[1], e2 = H.e[2], e3 = H.e[3];
@@ -831,7 +905,7 @@ __device__ __forceinline__ bool take_children(Trav<DEC64>& S, Hits& H, const Sta
     }
     if (two && S.stack.p + 3 * M.stride >= M.end) {  // rare: count the entries
         const int m = four ? 3 : three ? 2 : 1;
-        if (S.stack.p + m * M.stride >= M.end) return false;
+        if (S.stack.p + m * M.stride >= M.end && !(SPILL && stack_spill(S, M))) return false;
     }
     if (SORT) {
         if (two) {
@@ -872,7 +946,7 @@ __device__ __forceinline__ bool trav_step(Trav<DEC64>& S, const NodeT* __restric
         if (COUNT) n_rec += kWidth;
         Hits H;
         node_hits<DEC64>(S, nodes, S.cur, H);
-        if (!take_children<!ANY || RC_ANY_SORT>(S, H, M)) {
+        if (!take_children<!ANY || RC_ANY_SORT, true>(S, H, M)) {
             S.R.overflow = true;
             return true;
         }
@@ -899,7 +973,7 @@ __device__ __forceinline__ bool trav_step(Trav<DEC64>& S, const NodeT* __restric
             S.leaf = kEmptyChild;
         }
     }
-    return (S.cur & S.leaf) == kEmptyChild;
+    return (S.cur & S.leaf) == kEmptyChild && !stack_reload(S, M);
 #else
     if (is_leaf(S.cur)) {
         const uint32_t first = S.cur & ((1u << 26) - 1u), count = (S.cur >> 26) & 31u;
@@ -908,7 +982,7 @@ __device__ __forceinline__ bool trav_step(Trav<DEC64>& S, const NodeT* __restric
         if (!ANY && S.R.id != id) trav_cull(S);
         S.cur = stack_pop(S.stack, M);
     }
-    return S.cur == kEmptyChild;
+    return S.cur == kEmptyChild && !stack_reload(S, M);
 #endif  // RC_LEAF_POSTPONE
 }
 
@@ -937,7 +1011,7 @@ __device__ __forceinline__ TraceResult traverse_inline(const NodeT* __restrict__
             if (!ANY && S.R.id != id) trav_cull(S);
             H.h[k] = false;
         }
-        if (!take_children<true>(S, H, M)) {
+        if (!take_children<true, false>(S, H, M)) {
             S.R.overflow = true;
             return S.R;
         }
@@ -949,7 +1023,7 @@ __device__ __forceinline__ TraceResult traverse_inline(const NodeT* __restrict__
 // 32 words per ray (36 with more stack registers), written and read as 16-byte
 // vectors.  Words: 0 the
 // queue entry, 1 the current entry, 2 the stack's rows in use, 3 the best hit's
-// id, 4..6 its t, u, v, 7 unused, 8..9 the best distance of the FP64 decision,
+// id, 4..6 its t, u, v, 7 the spilled stack, 8..9 the best distance of the FP64 decision,
 // 10.. the register stack (top first), then the memory rows in their order
 // (only those in use are meaningful); the last two words the best hit's w and the
 // leaf set aside.
@@ -967,7 +1041,7 @@ __device__ __forceinline__ uint32_t park_word(const Trav<DEC64>& S, uint32_t ent
     if (w == 4) return __float_as_uint(S.R.t);
     if (w == 5) return __float_as_uint(S.R.u);
     if (w == 6) return __float_as_uint(S.R.v);
-    if (w == 7) return 0u;
+    if (w == 7) return S.scale_spill & kSpillMask;
     if (w == 8 || w == 9) {
         if constexpr (DEC64) {
             const unsigned long long b = __double_as_longlong(S.best);
@@ -1002,6 +1076,7 @@ __device__ __forceinline__ void unpark_word(Trav<DEC64>& S, const StackMem& M, i
     else if (w == 4) S.R.t = __uint_as_float(v);
     else if (w == 5) S.R.u = __uint_as_float(v);
     else if (w == 6) S.R.v = __uint_as_float(v);
+    else if (w == 7) S.scale_spill |= v;
     else if (w == kParkW) S.R.w = __uint_as_float(v);
     else if (w == kParkW + 1) S.leaf = v;
     else if (w == 8) best_lo = v;
@@ -1091,7 +1166,7 @@ __device__ __forceinline__ TraceResult traverse_packet(const QNode* __restrict__
                 H.t[k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(H.t[k])));
                 H.e[k] = __builtin_amdgcn_readfirstlane(H.e[k]);
             }
-            if (!take_children<true>(S, H, M)) {
+            if (!take_children<true, false>(S, H, M)) {
                 S.R.overflow = true;
                 return S.R;
             }

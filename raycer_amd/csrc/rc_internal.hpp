@@ -40,7 +40,7 @@ struct DevCounters {
     unsigned long long tri_tests;
     unsigned long long ext_rays;
     unsigned long long shadow_rays;
-    unsigned long long ovf_total;  // rays the deep-stack kernel walked, over every launch since the last reset
+    rcd::SpillCount spill;         // its total: rays whose stack outgrew its rows, over every launch since the last reset
     unsigned long long park_total; // traversals parked for the resume kernel since the last reset
     uint32_t ovf_count;            // rays listed for the next deep-stack launch
     uint32_t queue_count[4];   // wavefront queue sizes (ping, pong, shadow, scratch)
@@ -65,7 +65,7 @@ inline uint32_t pass_samples(const rc_tuning& t, uint32_t npix, uint32_t spp, si
 }
 
 // Device buffers of one frame's wavefront passes (path and shadow queues,
-// slot radiance and weights, the cold path's overflow list and deep stack)
+// slot radiance and weights, the overflow list and the stacks in global memory)
 // and its counters.  The context owns one set (fb, whose counters are the
 // context's); a batch owns one more per concurrent branch.
 struct FrameBuffers {
@@ -93,7 +93,7 @@ struct rc_ctx {
     bool hit_fp64 = false;  // RC_HIT_FP64: FP32 filter, FP64 decision of triangle hits
     rc_tuning tuning{256, 0, 64, 0, RC_PARK_STEPS_DEFAULT};  // samples per pass chosen per frame, the whole on-chip stack
 
-    // traversal stack entries held on chip before a ray goes to the deep-stack kernel
+    // traversal stack entries held on chip before a ray's stack goes to global memory
     int stack_depth() const {
         return tuning.stack_limit ? std::min(int(tuning.stack_limit), rcd::kLdsStack) : rcd::kLdsStack;
     }
@@ -135,8 +135,27 @@ struct rc_scene {
     size_t nmat = 0;
     float bmin[3], bmax[3];
     uint32_t depth = 0;
+    uint32_t stack_need = 0;  // the most entries a traversal's stack can hold
     size_t bytes = 0;
 };
+
+// Whether a ray's stack may outgrow `rows` rows.
+inline bool rc_may_spill(const rc_scene* s, int rows) {
+    return int(s->stack_need) > rows - (rcd::kRegStack == 0 ? 1 : 0);  // row 0: the end marker
+}
+
+// Whether a launch over at most `rays` rays may list some for the deep-stack
+// kernel: one whose rays may outgrow their rows, unless each finds a spill slot
+// and its whole stack fits in it (a block of at least rows - 2 rows, end
+// markers among them, adds its length).  An empty launch costs about 5 us: it
+// and what follows it are left out of queries of few rays and of small scenes.
+inline bool rc_may_list(const rc_scene* s, int rows, size_t rays) {
+    if (!rc_may_spill(s, rows)) return false;
+    const int marks = std::max(1, rcd::kRegStack), held = rows - 2 - marks;
+    if (rays > size_t(rcd::kDeepThreads) || rows < rcd::kSpillRows || held < 1) return true;
+    const uint32_t need = s->stack_need, blocks = (need + uint32_t(held) - 1) / uint32_t(held);
+    return need + blocks * uint32_t(marks + 1) > uint32_t(rcd::kDeepStack);
+}
 
 // The triangle records a traversal with the given decision reads.
 template <bool DEC64>
@@ -154,12 +173,11 @@ struct rc_film {
 };
 
 // Launches the closest-hit (ANY = false) or any-hit traversal over a device
-// ray array, then the deep-stack kernel over the rays whose stack outgrew the
-// on-chip depth.  n_dev (may be null) is a device count read by the kernel;
+// ray array, then the deep-stack kernel over the rays whose stack outgrew
+// both its rows and the spill slots.  n_dev (may be null) is a device count read by the kernel;
 // n_bound bounds it and sizes the grid.
 int rc_launch_trace(rc_ctx* ctx, const rc_scene* s, bool any, const rc_ray* rays, const uint32_t* n_dev,
                     uint32_t n_bound, rc_hit* hits, uint8_t* occ);
-int rc_launch_deep(rc_ctx* ctx, const rc_scene* s, bool any, const rc_ray* rays, rc_hit* hits, uint8_t* occ);
 
 // One traversal launch with its scratch given explicitly: the overflow list
 // (n_bound entries), the deep-stack kernel's stack (rc_deep_stack_bytes())
@@ -176,7 +194,7 @@ struct TraceLaunch {
     uint32_t* deep_stack = nullptr;
     DevCounters* ctr = nullptr;
     hipStream_t stream = nullptr;
-    int max_depth = rcd::kLdsStack;  // on-chip stack entries before the deep-stack kernel
+    int max_depth = rcd::kLdsStack;  // on-chip stack entries
     uint32_t max_blocks = 1;            // grid limit; the kernel's grid-stride loop covers the rest
     bool counting = false;
     bool dec64 = false;
@@ -184,7 +202,8 @@ struct TraceLaunch {
 size_t rc_deep_stack_bytes();
 // Clears the overflow count and launches the traversal kernel.
 int rc_launch_trace_with(const TraceLaunch& L);
-// The deep-stack kernel over the rays the last traversal launch listed.
+// The deep-stack kernel over the rays the last traversal launch (of at most
+// L.n_bound rays) listed; nothing when it can have listed none (rc_may_list).
 int rc_launch_deep_with(const TraceLaunch& L);
 // Camera rays of one pass of Tracer::generateMultiSamples (slot = j * npix + q
 // for sample sample0 + j of the pixel at position q of the tiled order): ray,

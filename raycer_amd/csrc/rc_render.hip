@@ -537,7 +537,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
     PassParams P, uint32_t k, const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
     const rc_ray* __restrict__ rays, const float4* __restrict__ st, const float4* __restrict__ shade,
     const DevMaterial* __restrict__ mats, rc_ray* __restrict__ rays_out, float4* __restrict__ st_out,
-    rc_ray* __restrict__ srays, float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list,
+    rc_ray* __restrict__ srays, float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list, uint32_t* __restrict__ gstack,
     DevCounters* __restrict__ ctr, uint32_t cin, uint32_t cout, CacheIO CI, float* __restrict__ W,
     rc_ray* __restrict__ cam_rays, float4* __restrict__ cam_st, ParkIO PK) {
     static_assert(!(PARK && CAM), "the camera bounce does not park");
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
     const uint32_t n = ctr->queue_count[cin];
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
-    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit, gstack, &ctr->spill);
     const uint32_t i = trace_block<BLOCK>(n) * BLOCK + threadIdx.x;
     if (i == 0) atomicAdd(&ctr->ext_rays, (unsigned long long)n);
     uint32_t n_rec = 0, n_tri = 0;
@@ -646,7 +646,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
     PassParams P, uint32_t k, const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
     const rc_ray* __restrict__ rays, const float4* __restrict__ st, const float4* __restrict__ shade,
     const DevMaterial* __restrict__ mats, rc_ray* __restrict__ rays_out, float4* __restrict__ st_out,
-    rc_ray* __restrict__ srays, float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list,
+    rc_ray* __restrict__ srays, float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list, uint32_t* __restrict__ gstack,
     DevCounters* __restrict__ ctr, uint32_t cout, CacheIO CI, ParkIO in, ParkIO out) {
     __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
     if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&ctr->park_total, (unsigned long long)n);
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
-    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit, gstack, &ctr->spill);
     const uint32_t q = blockIdx.x * uint32_t(BLOCK) + threadIdx.x;
     uint32_t n_rec = 0, n_tri = 0;
     ShadeOut O;
@@ -760,14 +760,15 @@ template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
 __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT* __restrict__ nodes,
                                                        const TriRec* __restrict__ tris, const rc_ray* __restrict__ srays,
                                                        const float4* __restrict__ scontrib, float4* __restrict__ L,
-                                                       uint32_t* __restrict__ ovf_list, DevCounters* __restrict__ ctr,
+                                                       uint32_t* __restrict__ ovf_list,
+    uint32_t* __restrict__ gstack, DevCounters* __restrict__ ctr,
                                                        uint8_t* __restrict__ occ_out, int stack_limit, ParkIO PK) {
     __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = ctr->queue_count[2];
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
-    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit, gstack, &ctr->spill);
     const uint32_t i = trace_block<BLOCK>(n) * BLOCK + threadIdx.x;
     if (i == 0) atomicAdd(&ctr->shadow_rays, (unsigned long long)n);
     uint32_t n_rec = 0, n_tri = 0;
@@ -819,7 +820,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
 template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
 __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow_resume(
     const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris, const rc_ray* __restrict__ srays,
-    const float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list,
+    const float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list, uint32_t* __restrict__ gstack,
     DevCounters* __restrict__ ctr, uint8_t* __restrict__ occ_out, int stack_limit, ParkIO in, ParkIO out) {
     __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
@@ -828,7 +829,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow_resume(
     if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&ctr->park_total, (unsigned long long)n);
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
-    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit);
+    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit, gstack, &ctr->spill);
     const uint32_t q = blockIdx.x * uint32_t(BLOCK) + threadIdx.x;
     uint32_t n_rec = 0, n_tri = 0;
     Trav<DEC64> S;
@@ -940,14 +941,15 @@ __global__ void k_prep(DevCounters* ctr, uint32_t cout) {
     ctr->queue_count[cout] = 0;
     ctr->queue_count[2] = 0;
     ctr->ovf_count = 0;
+    ctr->spill.claimed = 0;
     ctr->park_count[0] = 0;
     ctr->park_count[1] = 0;
 }
 
-__global__ void k_reset_ovf(DevCounters* ctr) { ctr->ovf_count = 0; }
 // Before a shadow pass: the overflow list and both park regions are free.
 __global__ void k_reset_shadow(DevCounters* ctr) {
     ctr->ovf_count = 0;
+    ctr->spill.claimed = 0;
     ctr->park_count[0] = 0;
     ctr->park_count[1] = 0;
 }
@@ -1052,7 +1054,7 @@ struct ExtendArgs {
     rc_ray* srays;
     float4* scontrib;
     float4* L;
-    uint32_t* ovf;
+    uint32_t *ovf, *gstack;
     DevCounters* ctr;
     uint32_t cin, cout;
     CacheIO CI;
@@ -1064,7 +1066,7 @@ template <bool COUNT, bool CAM, bool DEC64, int BLOCK, bool PARK>
 void extend_t(const ExtendArgs& a, uint32_t n, hipStream_t st) {
     k_extend_shade<COUNT, CAM, DEC64, BLOCK, PARK><<<(n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(
         a.P, a.k, a.s->nodes, tri_array<DEC64>(a.s), a.rin, a.sin, a.s->shade, a.s->mats, a.rout, a.sout, a.srays, a.scontrib, a.L,
-        a.ovf, a.ctr, a.cin, a.cout, a.CI, a.W, a.rin, a.sin, a.PK);
+        a.ovf, a.gstack, a.ctr, a.cin, a.cout, a.CI, a.W, a.rin, a.sin, a.PK);
 }
 
 template <bool COUNT, bool CAM, bool DEC64>
@@ -1101,7 +1103,7 @@ template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
 void resume_t(const ExtendArgs& a, const ParkIO& in, const ParkIO& out, hipStream_t st) {
     k_extend_resume<COUNT, DEC64, BLOCK, PARK><<<std::max(1u, (in.cap + BLOCK - 1) / BLOCK), BLOCK, 0, st>>>(
         a.P, a.k, a.s->nodes, tri_array<DEC64>(a.s), a.rin, a.sin, a.s->shade, a.s->mats, a.rout, a.sout, a.srays, a.scontrib, a.L,
-        a.ovf, a.ctr, a.cout, a.CI, in, out);
+        a.ovf, a.gstack, a.ctr, a.cout, a.CI, in, out);
 }
 
 template <bool COUNT, bool DEC64, bool PARK>
@@ -1134,7 +1136,7 @@ struct ShadowArgs {
     const rc_ray* srays;
     const float4* scontrib;
     float4* L;
-    uint32_t* ovf;
+    uint32_t *ovf, *gstack;
     DevCounters* ctr;
     uint8_t* occ_out;
     int stack_limit;
@@ -1144,7 +1146,7 @@ struct ShadowArgs {
 template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
 void shadow_t(const ShadowArgs& a, uint32_t n, hipStream_t st) {
     k_shadow<COUNT, DEC64, BLOCK, PARK><<<(n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(
-        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.ctr, a.occ_out, a.stack_limit, a.PK);
+        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit, a.PK);
 }
 
 template <bool COUNT, bool DEC64, bool PARK>
@@ -1166,7 +1168,7 @@ void launch_shadow(const ShadowArgs& a, uint32_t n, hipStream_t st, bool count, 
 template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
 void shadow_resume_t(const ShadowArgs& a, const ParkIO& in, const ParkIO& out, hipStream_t st) {
     k_shadow_resume<COUNT, DEC64, BLOCK, PARK><<<std::max(1u, (in.cap + BLOCK - 1) / BLOCK), BLOCK, 0, st>>>(
-        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.ctr, a.occ_out, a.stack_limit, in, out);
+        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit, in, out);
 }
 
 template <bool COUNT, bool DEC64, bool PARK>
@@ -1207,7 +1209,7 @@ __global__ void k_zero_counters(DevCounters* ctr) {
     ctr->tri_tests = 0;
     ctr->ext_rays = 0;
     ctr->shadow_rays = 0;
-    ctr->ovf_total = 0;
+    ctr->spill.total = 0;
     ctr->park_total = 0;
     ctr->ovf_count = 0;
     ctr->error = 0;
@@ -1397,6 +1399,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
     deep.stream = st;
     deep.counting = c->counting;
     deep.dec64 = c->hit_fp64;
+    deep.max_depth = P.stack_limit;
     for (uint32_t s0 = 0; s0 < cfg->spp; s0 += spp_pass) {
         if (progress) {
             RC_TRY_HIP(hipStreamSynchronize(st));
@@ -1408,6 +1411,8 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
         P.sample0 = s0;
         const uint32_t n = npix * this_pass;
         const uint32_t grid_n = (n + kBlock - 1) / kBlock;
+        deep.n_bound = n;
+        const bool listed = rc_may_list(s, P.stack_limit, n);
         hipEvent_t ev = nullptr;
         if (CI.cache_vertex) k_cache_reset<<<1, 1, 0, st>>>(CI.counters, 0);
         if (RC_FUSED_CAMERA) {
@@ -1428,20 +1433,21 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
             const bool camb = RC_FUSED_CAMERA && k == 0;
             ParkIO PK = regions[0];
             PK.steps = camb ? 0u : c->tuning.park_steps;
-            ExtendArgs ea{P, k, s, rin, sin_, rout, sout, srays, scontrib, L, ovf, ctr, cin, cout, CI, W, PK};
+            ExtendArgs ea{P, k, s, rin, sin_, rout, sout, srays, scontrib, L, ovf, deep.deep_stack, ctr, cin, cout, CI, W, PK};
             launch_extend(ea, n, st, c->counting, camb, c->hit_fp64, shape.ext_block);
             if (PK.steps)
                 launch_resumes(ea, regions, RC_PARK_PHASES, RC_PARK_STEPS2, st, c->counting, c->hit_fp64,
                                shape.ext_block);
             if (timed) RC_TRY(c->prof_end(ev, PK_EXTEND));
-            // cold path: rays whose stack outgrew the on-chip depth
+            // cold path: rays whose stack outgrew the on-chip depth and found no spill slot
             deep.any = false;
             deep.rays = rin;
             deep.hits = B.hits.as<rc_hit>();
             deep.occ = nullptr;
             RC_TRY(rc_launch_deep_with(deep));
-            k_shade_listed<<<grid_small, kBlock, 0, st>>>(P, k, rin, sin_, B.hits.as<rc_hit>(), s->shade, s->mats, rout,
-                                                          sout, srays, scontrib, L, ovf, ctr, cout, CI);
+            if (listed)
+                k_shade_listed<<<grid_small, kBlock, 0, st>>>(P, k, rin, sin_, B.hits.as<rc_hit>(), s->shade, s->mats,
+                                                              rout, sout, srays, scontrib, L, ovf, ctr, cout, CI);
             if (P.has_sun && k + 1 < cfg->max_path_length) {
                 // at the cache vertex the shadow results are kept for the training records
                 const bool nee_fix = CI.cache_vertex && k == CI.cache_vertex;
@@ -1450,7 +1456,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
                 if (timed) RC_TRY(c->prof_begin(&ev));
                 ParkIO SPK = regions[0];
                 SPK.steps = c->tuning.park_steps ? uint32_t(RC_SHADOW_PARK_STEPS) : 0u;
-                ShadowArgs sa_{s, srays, scontrib, L, ovf, ctr, occ_out, P.stack_limit, SPK};
+                ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit, SPK};
                 launch_shadow(sa_, n, st, c->counting, c->hit_fp64, shape.shadow_block);
                 if (SPK.steps)
                     launch_shadow_resumes(sa_, regions, RC_SHADOW_PARK_PHASES, RC_PARK_STEPS2, st, c->counting,
@@ -1461,7 +1467,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
                 deep.hits = nullptr;
                 deep.occ = socc;
                 RC_TRY(rc_launch_deep_with(deep));
-                k_shadow_apply_listed<<<grid_small, kBlock, 0, st>>>(scontrib, socc, ovf, L, ctr);
+                if (listed) k_shadow_apply_listed<<<grid_small, kBlock, 0, st>>>(scontrib, socc, ovf, L, ctr);
                 if (nee_fix)
                     k_cache_nee_fix<<<grid_small, kBlock, 0, st>>>(CI.records, CI.counters, CI.cap, scontrib, socc);
             }
@@ -1555,7 +1561,7 @@ int render_frame(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_camera* cam,
     c->stats.samples = uint64_t(cfg->width) * cfg->height * cfg->spp;
     c->stats.node_records = h.node_records;
     c->stats.tri_tests = h.tri_tests;
-    c->stats.overflow_rays = h.ovf_total;
+    c->stats.overflow_rays = h.spill.total;
     c->stats.parked_rays = h.park_total;
     if (cache) {
         c->stats.cache_queries = cache_counts[0];

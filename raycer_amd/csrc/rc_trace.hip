@@ -4,8 +4,9 @@
 //
 // k_trace: persistent grid-stride loop, one ray per lane, the top of the
 // traversal stack in registers and the rest in LDS laid out [depth][lane] so a
-// wave's pushes and pops hit 64 distinct banks.  A ray whose stack would
-// exceed the on-chip depth is queued for k_trace_deep, which walks it again
+// wave's pushes and pops hit 64 distinct banks.  A ray whose stack outgrows its
+// rows moves them to one of the launch's spill slots in global memory and goes
+// on; when those are taken it is queued for k_trace_deep, which walks it again
 // with the memory part of its stack in global memory, as deep as the deepest
 // BVH the upload accepts.  The node/triangle counting variant is a
 // separate instantiation so the timed kernels carry no counters.
@@ -23,7 +24,6 @@ namespace {
 #define RC_TRACE_BLOCK 256
 #endif
 constexpr int kBlock = RC_TRACE_BLOCK;
-constexpr int kDeepThreads = 2048;
 
 __device__ __forceinline__ void store_result(bool any, const TraceResult& R, uint32_t i, rc_hit* hits, uint8_t* occ) {
     bool hit = R.id != kNoHit;
@@ -43,12 +43,12 @@ template <bool ANY, bool COUNT, bool DEC64>
 __global__ __launch_bounds__(kBlock, DEC64 ? 1 : 8) void k_trace(const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris,
                                                   const rc_ray* __restrict__ rays, const uint32_t* n_dev,
                                                   uint32_t n_host, rc_hit* __restrict__ hits, uint8_t* __restrict__ occ,
-                                                  uint32_t* __restrict__ ovf_list, DevCounters* __restrict__ ctr,
-                                                  int max_depth) {
+                                                  uint32_t* __restrict__ ovf_list, uint32_t* __restrict__ gstack,
+                                                  DevCounters* __restrict__ ctr, int max_depth) {
     __shared__ uint32_t stack[kLdsStack * kBlock];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t ntop = load_top(nodes, top);
-    const StackMem M = stack_mem(stack, threadIdx.x, kBlock, max_depth);
+    const StackMem M = stack_mem(stack, threadIdx.x, kBlock, max_depth, gstack, &ctr->spill);
     const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
     uint32_t n_rec = 0, n_tri = 0;
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64) void k_trace_deep(const NodeT* __restrict__ nod
                                                    uint32_t* __restrict__ gstack, DevCounters* __restrict__ ctr) {
     const uint32_t n = ctr->ovf_count;
     const uint32_t gtid = blockIdx.x * 64 + threadIdx.x, nthreads = gridDim.x * 64;
-    if (gtid == 0 && n) atomicAdd(&ctr->ovf_total, (unsigned long long)n);
+    if (gtid == 0 && n) atomicAdd(&ctr->spill.total, (unsigned long long)n);
     const StackMem M = stack_mem(gstack, gtid, int(nthreads), kDeepStack);
     uint32_t n_rec = 0, n_tri = 0;
     for (uint32_t k = gtid; k < n; k += nthreads) {
@@ -99,13 +99,16 @@ __global__ __launch_bounds__(64) void k_trace_deep(const NodeT* __restrict__ nod
     }
 }
 
-__global__ void k_reset_overflow(DevCounters* ctr) { ctr->ovf_count = 0; }
+__global__ void k_reset_overflow(DevCounters* ctr) {
+    ctr->ovf_count = 0;
+    ctr->spill.claimed = 0;
+}
 
 template <bool ANY, bool COUNT, bool DEC64>
 void launch_pair(const TraceLaunch& L, uint32_t blocks) {
     k_trace<ANY, COUNT, DEC64><<<blocks, kBlock, 0, L.stream>>>(L.scene->nodes, tri_array<DEC64>(L.scene), L.rays, L.n_dev,
-                                                                L.n_bound, L.hits, L.occ, L.ovf_list, L.ctr,
-                                                                L.max_depth);
+                                                                L.n_bound, L.hits, L.occ, L.ovf_list, L.deep_stack,
+                                                                L.ctr, L.max_depth);
 }
 
 template <bool ANY, bool COUNT, bool DEC64>
@@ -134,7 +137,7 @@ size_t rc_deep_stack_bytes() { return size_t(kDeepThreads) * kDeepStack * sizeof
 int rc_launch_trace_with(const TraceLaunch& L) {
     if (L.n_bound == 0) return RC_OK;
     const uint32_t blocks = std::max(1u, std::min((L.n_bound + kBlock - 1) / kBlock, L.max_blocks));
-    k_reset_overflow<<<1, 1, 0, L.stream>>>(L.ctr);
+    if (rc_may_spill(L.scene, L.max_depth)) k_reset_overflow<<<1, 1, 0, L.stream>>>(L.ctr);
     if (L.counting) {
         if (L.dec64) dispatch_trace<true, true>(L, blocks);
         else dispatch_trace<true, false>(L, blocks);
@@ -146,6 +149,7 @@ int rc_launch_trace_with(const TraceLaunch& L) {
 }
 
 int rc_launch_deep_with(const TraceLaunch& L) {
+    if (!rc_may_list(L.scene, L.max_depth, L.n_bound)) return RC_OK;
     if (L.counting) {
         if (L.dec64) dispatch_deep<true, true>(L);
         else dispatch_deep<true, false>(L);
@@ -191,17 +195,8 @@ int rc_launch_trace(rc_ctx* c, const rc_scene* s, bool any, const rc_ray* rays, 
     RC_TRY(c->prof_begin(&ev));
     RC_TRY(rc_launch_trace_with(L));
     RC_TRY(c->prof_end(ev, any ? PK_SHADOW : PK_EXTEND));
-    // rays whose stack outgrew the on-chip depth are walked again with the deep stack
+    // rays whose stack found no more room are walked again
     RC_TRY(rc_launch_deep_with(L));
-    RC_TRY_HIP(hipGetLastError());
-    return RC_OK;
-}
-
-// Deep-stack traversal of the rays listed in the overflow list (count in the
-// device counters); hits (closest) or occluded flags (any) are written at the
-// listed ray indices.
-int rc_launch_deep(rc_ctx* c, const rc_scene* s, bool any, const rc_ray* rays, rc_hit* hits, uint8_t* occ) {
-    RC_TRY(rc_launch_deep_with(context_launch(c, s, any, rays, nullptr, 0, hits, occ)));
     RC_TRY_HIP(hipGetLastError());
     return RC_OK;
 }
@@ -240,7 +235,7 @@ int trace_host(rc_ctx* c, const rc_scene* s, bool any, const rc_ray* rays, size_
     RC_TRY(c->prof_collect());
     c->stats.node_records = h.node_records;
     c->stats.tri_tests = h.tri_tests;
-    c->stats.overflow_rays = h.ovf_total;
+    c->stats.overflow_rays = h.spill.total;
     if (any) c->stats.shadow_rays = n; else c->stats.extension_rays = n;
     return RC_OK;
 }

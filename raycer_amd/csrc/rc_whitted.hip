@@ -887,7 +887,7 @@ extern "C" int rc_raytrace(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_ca
     c->stats.extension_rays = run.ext_rays;
     c->stats.shadow_rays = run.shadow_rays;
     c->stats.samples = uint64_t(P.npix) * cfg->spp;
-    c->stats.overflow_rays = h.ovf_total;
+    c->stats.overflow_rays = h.spill.total;
     c->stats.render_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return RC_OK;
 }
