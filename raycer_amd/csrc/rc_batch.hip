@@ -188,6 +188,8 @@ int render_batch(rc_ctx* c, const rc_scene* const* scenes, rc_film* const* films
     for (size_t i = 0; i < n; ++i) {
         put(key, scenes[i]->nodes);
         put(key, scenes[i]->tris);
+        put(key, scenes[i]->tris_exact);
+        put(key, scenes[i]->stack_need);  // which kernels are launched
         put(key, scenes[i]->shade);
         put(key, scenes[i]->mats);
         put(key, films[i]->sum);
