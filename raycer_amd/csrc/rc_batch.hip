@@ -113,6 +113,7 @@ int capture(rc_ctx* c, const rc_scene* const* scenes, rc_film* const* films, con
             shape.spp_pass = plans[i].spp_per_pass;
             shape.ext_block = plans[i].ext_block;
             shape.shadow_block = plans[i].shadow_block;
+            shape.concurrent = nb > 1;
             rc = rc_enqueue_frame(c, branch_buffers(c, b), branch_stream(c, b), scenes[i], films[i], &cams[i],
                                   &cfgs[i], shape, nullptr, nullptr);
             if (rc != RC_OK) break;

@@ -81,6 +81,7 @@ struct FrameShape {
     uint32_t spp_pass = 1;
     uint32_t ext_block = 256;     // extension kernel: 128 or 256
     uint32_t shadow_block = 128;  // shadow kernel: 64, 128 or 256
+    bool concurrent = false;      // other frames run beside it
 };
 
 struct rc_ctx {

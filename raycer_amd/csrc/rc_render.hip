@@ -59,15 +59,6 @@ constexpr uint32_t kShadowBlockDefault = RC_SHADOW_BLOCK;
 #define RC_PARK_STEPS2 20
 #endif
 static_assert(RC_PARK_PHASES >= 2, "a parking extension launch needs a resume kernel");
-// Shadow rays (any hit) park after RC_SHADOW_PARK_STEPS iterations when
-// parking is on (0: they never park), over RC_SHADOW_PARK_PHASES kernels.
-#ifndef RC_SHADOW_PARK_STEPS
-#define RC_SHADOW_PARK_STEPS 32
-#endif
-#ifndef RC_SHADOW_PARK_PHASES
-#define RC_SHADOW_PARK_PHASES 3
-#endif
-static_assert(RC_SHADOW_PARK_PHASES >= 2, "a parking shadow launch needs a resume kernel");
 #ifndef RC_MIN_WAVES_FP64
 #define RC_MIN_WAVES_FP64 1
 #endif
@@ -274,14 +265,9 @@ __global__ void k_pass_start(DevCounters* ctr, uint32_t n) {
 #ifndef RC_PARK_KEEP
 #define RC_PARK_KEEP 8
 #endif
-#ifndef RC_PARK_KEEP_ANY
-#define RC_PARK_KEEP_ANY 0
-#endif
-// Whether a parking traversal (ANY: a shadow ray's) goes on after `steps`
-// iterations of `budget`.
-template <bool ANY>
+// Whether a parking traversal goes on after `steps` iterations of `budget`.
 __device__ __forceinline__ bool keep_going(bool done, uint32_t steps, uint32_t budget) {
-    constexpr uint32_t keep = ANY ? RC_PARK_KEEP_ANY : RC_PARK_KEEP;
+    constexpr uint32_t keep = RC_PARK_KEEP;
     if (keep == 0) return !done && steps < budget;
     const uint32_t busy = uint32_t(__popcll(__ballot(!done)));
     return !done && (steps < budget || (steps < 2 * budget && busy >= keep));
@@ -530,7 +516,20 @@ struct ParkIO {
     uint32_t cap;    // records of the region
     uint32_t steps;  // budget of the kernel writing the region (0: no parking)
     uint32_t which;  // the region's counter: DevCounters::park_count[which]
+    uint32_t min_rays;  // a launch of fewer rays does not park
 };
+
+// With the default budget a bounce parks from kParkRays rays on: the two
+// resume kernels each end with their longest traversals, some 100 us of a
+// nearly idle chip, which only a large bounce earns back.  A 499x373 frame of
+// 100,000 random triangles (9 samples, FP64 decision) takes 3.71 ms without
+// parking, 3.90 with it; frames of 262,144 paths in scenes of 300 to 131,000
+// triangles 1.1 to 1.4 times as long with it; the 64-sample 1080p frame of
+// 2,093,058 triangles 63.9 ms without, 60.3 with (all bounces 60.6).  The
+// frames of a batch run beside each other, so one's tail is filled by the
+// rest: eight soups take 12.7 ms with bounces parking from 2^20 rays on, 13.5
+// from 6 * 2^20.
+constexpr uint32_t kParkRays = 6u << 20, kParkRaysConcurrent = 1u << 20;
 
 template <bool COUNT, bool CAM, bool DEC64, int BLOCK, bool PARK>
 __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
@@ -564,10 +563,11 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
             const float4* rp = reinterpret_cast<const float4*>(rays + i);
             const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
             trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
+            const uint32_t budget = n >= PK.min_rays ? PK.steps : 0xffffffffu;
             uint32_t steps = 0;
             do {
                 done = trav_step<false, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
-            } while (keep_going<false>(done, ++steps, PK.steps));
+            } while (keep_going(done, ++steps, budget));
         }
         // every thread of the block reserves (one atomic per block)
         const uint32_t pos = block_append<BLOCK>(!done, &ctr->park_count[PK.which], append_scratch);
@@ -677,7 +677,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
         uint32_t steps = 0;
         do {
             done = trav_step<false, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
-        } while (PARK ? keep_going<false>(done, ++steps, out.steps) : !done);
+        } while (PARK ? keep_going(done, ++steps, out.steps) : !done);
     }
     bool parked = false;
     if constexpr (PARK) {
@@ -754,15 +754,18 @@ __device__ __forceinline__ void shadow_result(uint32_t i, bool occluded, const f
 
 // Any hit of a shadow ray; an unoccluded ray adds its contribution to its
 // slot.  Overflowing rays are listed for the deep-stack kernel and applied by
-// k_shadow_apply_listed.  PARK: as the extension kernel, a ray still
-// traversing after PK.steps iterations is parked for k_shadow_resume.
-template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
+// k_shadow_apply_listed.  Shadow rays do not park: they end at their first
+// hit, and the kernels that resumed them ended with their longest ray, alone
+// on the chip, three times over (the 64-sample 1080p frame of 2,093,058
+// triangles takes 60.6 ms without against 61.6, a 499x373 frame of 100,000
+// with 9 samples 3.90 against 4.12).
+template <bool COUNT, bool DEC64, int BLOCK>
 __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT* __restrict__ nodes,
                                                        const TriRec* __restrict__ tris, const rc_ray* __restrict__ srays,
                                                        const float4* __restrict__ scontrib, float4* __restrict__ L,
                                                        uint32_t* __restrict__ ovf_list,
     uint32_t* __restrict__ gstack, DevCounters* __restrict__ ctr,
-                                                       uint8_t* __restrict__ occ_out, int stack_limit, ParkIO PK) {
+                                                       uint8_t* __restrict__ occ_out, int stack_limit) {
     __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = ctr->queue_count[2];
@@ -772,35 +775,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
     const uint32_t i = trace_block<BLOCK>(n) * BLOCK + threadIdx.x;
     if (i == 0) atomicAdd(&ctr->shadow_rays, (unsigned long long)n);
     uint32_t n_rec = 0, n_tri = 0;
-    if constexpr (PARK) {
-        __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
-        Trav<DEC64> S;
-        bool done = true;
-        if (i < n) {
-            const float4* rp = reinterpret_cast<const float4*>(srays + i);
-            const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-            trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
-            uint32_t steps = 0;
-            do {
-                done = trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
-            } while (keep_going<true>(done, ++steps, PK.steps));
-        }
-        const uint32_t pos = block_append<BLOCK>(!done, &ctr->park_count[PK.which], append_scratch);
-        bool parked = false;
-        if (!done) {
-            if (pos < PK.cap) {
-                trav_park(S, i, M, PK.rec + size_t(pos) * kParkWords);
-                parked = true;
-            } else {
-                while (!trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
-                }
-            }
-        }
-        if (i < n && !parked) {
-            if (S.R.overflow) ovf_list[atomicAdd(&ctr->ovf_count, 1u)] = i;
-            else shadow_result(i, S.R.id != kNoHit, scontrib, L, occ_out);
-        }
-    } else if (i < n) {
+    if (i < n) {
         const float4* rp = reinterpret_cast<const float4*>(srays + i);
         float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
         TraceResult R =
@@ -808,63 +783,6 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
                                               false);
         if (R.overflow) ovf_list[atomicAdd(&ctr->ovf_count, 1u)] = i;
         else shadow_result(i, R.id != kNoHit, scontrib, L, occ_out);
-    }
-    if (COUNT) {
-        wave_add(&ctr->node_records, n_rec);
-        wave_add(&ctr->tri_tests, n_tri);
-    }
-}
-
-// The parked shadow traversals of region `in`, continued (and with PARK
-// parked again in region `out` after out.steps iterations) and applied.
-template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
-__global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow_resume(
-    const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris, const rc_ray* __restrict__ srays,
-    const float4* __restrict__ scontrib, float4* __restrict__ L, uint32_t* __restrict__ ovf_list, uint32_t* __restrict__ gstack,
-    DevCounters* __restrict__ ctr, uint8_t* __restrict__ occ_out, int stack_limit, ParkIO in, ParkIO out) {
-    __shared__ uint32_t stack[kLdsStack * BLOCK];
-    __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
-    __shared__ uint4 top[4 * kTopNodes];
-    const uint32_t n = min(ctr->park_count[in.which], in.cap);
-    if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&ctr->park_total, (unsigned long long)n);
-    if (blockIdx.x * uint32_t(BLOCK) >= n) return;
-    const uint32_t ntop = load_top(nodes, top);
-    const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit, gstack, &ctr->spill);
-    const uint32_t q = blockIdx.x * uint32_t(BLOCK) + threadIdx.x;
-    uint32_t n_rec = 0, n_tri = 0;
-    Trav<DEC64> S;
-    uint32_t i = 0;
-    bool done = true;
-    if (q < n) {
-        const uint32_t* rec = in.rec + size_t(q) * kParkWords;
-        i = rec[0];
-        {
-            const float4* rp = reinterpret_cast<const float4*>(srays + i);
-            const float4 r0 = ld_stream(rp), r1 = ld_stream(rp + 1);
-            trav_begin(S, nodes, M, f3(r0), f3(r1), r0.w, r1.w, top, ntop, false);
-        }
-        trav_unpark(S, rec, M);
-        uint32_t steps = 0;
-        do {
-            done = trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri);
-        } while (PARK ? keep_going<true>(done, ++steps, out.steps) : !done);
-    }
-    bool parked = false;
-    if constexpr (PARK) {
-        const uint32_t pos = block_append<BLOCK>(!done, &ctr->park_count[out.which], append_scratch);
-        if (!done) {
-            if (pos < out.cap) {
-                trav_park(S, i, M, out.rec + size_t(pos) * kParkWords);
-                parked = true;
-            } else {
-                while (!trav_step<true, COUNT, DEC64>(S, nodes, tris, M, n_rec, n_tri)) {
-                }
-            }
-        }
-    }
-    if (q < n && !parked) {
-        if (S.R.overflow) ovf_list[atomicAdd(&ctr->ovf_count, 1u)] = i;
-        else shadow_result(i, S.R.id != kNoHit, scontrib, L, occ_out);
     }
     if (COUNT) {
         wave_add(&ctr->node_records, n_rec);
@@ -946,12 +864,10 @@ __global__ void k_prep(DevCounters* ctr, uint32_t cout) {
     ctr->park_count[1] = 0;
 }
 
-// Before a shadow pass: the overflow list and both park regions are free.
+// Before a shadow pass: the overflow list and the spill slots are free.
 __global__ void k_reset_shadow(DevCounters* ctr) {
     ctr->ovf_count = 0;
     ctr->spill.claimed = 0;
-    ctr->park_count[0] = 0;
-    ctr->park_count[1] = 0;
 }
 
 __device__ __forceinline__ void kahan(float& s, float& c, float v) {
@@ -1140,61 +1056,28 @@ struct ShadowArgs {
     DevCounters* ctr;
     uint8_t* occ_out;
     int stack_limit;
-    ParkIO PK;  // PK.steps > 0: long traversals are parked
 };
 
-template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
+template <bool COUNT, bool DEC64, int BLOCK>
 void shadow_t(const ShadowArgs& a, uint32_t n, hipStream_t st) {
-    k_shadow<COUNT, DEC64, BLOCK, PARK><<<(n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(
-        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit, a.PK);
+    k_shadow<COUNT, DEC64, BLOCK><<<(n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(
+        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit);
 }
 
-template <bool COUNT, bool DEC64, bool PARK>
+template <bool COUNT, bool DEC64>
 void shadow_b(const ShadowArgs& a, uint32_t n, hipStream_t st, uint32_t block) {
     if constexpr (!COUNT) {
-        if (block == 64) return shadow_t<COUNT, DEC64, 64, PARK>(a, n, st);
-        if (block == 256) return shadow_t<COUNT, DEC64, 256, PARK>(a, n, st);
+        if (block == 64) return shadow_t<COUNT, DEC64, 64>(a, n, st);
+        if (block == 256) return shadow_t<COUNT, DEC64, 256>(a, n, st);
     }
-    shadow_t<COUNT, DEC64, 128, PARK>(a, n, st);
+    shadow_t<COUNT, DEC64, 128>(a, n, st);
 }
 
 void launch_shadow(const ShadowArgs& a, uint32_t n, hipStream_t st, bool count, bool dec64, uint32_t block) {
-#define RC_SHD(C, D) (a.PK.steps ? shadow_b<C, D, true>(a, n, st, block) : shadow_b<C, D, false>(a, n, st, block))
+#define RC_SHD(C, D) shadow_b<C, D>(a, n, st, block)
     if (count) { if (dec64) RC_SHD(true, true); else RC_SHD(true, false); }
     else { if (dec64) RC_SHD(false, true); else RC_SHD(false, false); }
 #undef RC_SHD
-}
-
-template <bool COUNT, bool DEC64, int BLOCK, bool PARK>
-void shadow_resume_t(const ShadowArgs& a, const ParkIO& in, const ParkIO& out, hipStream_t st) {
-    k_shadow_resume<COUNT, DEC64, BLOCK, PARK><<<std::max(1u, (in.cap + BLOCK - 1) / BLOCK), BLOCK, 0, st>>>(
-        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit, in, out);
-}
-
-template <bool COUNT, bool DEC64, bool PARK>
-void shadow_resume_b(const ShadowArgs& a, const ParkIO& in, const ParkIO& out, hipStream_t st, uint32_t block) {
-    if constexpr (!COUNT) {
-        if (block == 64) return shadow_resume_t<COUNT, DEC64, 64, PARK>(a, in, out, st);
-        if (block == 256) return shadow_resume_t<COUNT, DEC64, 256, PARK>(a, in, out, st);
-    }
-    shadow_resume_t<COUNT, DEC64, 128, PARK>(a, in, out, st);
-}
-
-// The resume kernels of a shadow launch that parked into region 0, as
-// launch_resumes for the extension kernel.
-void launch_shadow_resumes(const ShadowArgs& a, const ParkIO regions[2], uint32_t phases, uint32_t steps2,
-                           hipStream_t st, bool count, bool dec64, uint32_t block) {
-    for (uint32_t ph = 1; ph < phases; ++ph) {
-        ParkIO in = regions[(ph - 1) & 1u], out = regions[ph & 1u];
-        const bool park = ph + 1 < phases;
-        out.steps = park ? steps2 : 0u;
-        if (park && ph > 1) k_zero_park<<<1, 1, 0, st>>>(a.ctr, out.which);
-#define RC_SRES(C, D) \
-    (park ? shadow_resume_b<C, D, true>(a, in, out, st, block) : shadow_resume_b<C, D, false>(a, in, out, st, block))
-        if (count) { if (dec64) RC_SRES(true, true); else RC_SRES(true, false); }
-        else { if (dec64) RC_SRES(false, true); else RC_SRES(false, false); }
-#undef RC_SRES
-    }
 }
 
 uint32_t isqrt_exact(uint32_t v) {
@@ -1374,8 +1257,11 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
     if (c->tuning.park_steps && park_recs < 4)
         return rc_host_fail(RC_ERR_INVALID, "rc_render: no park records for the extension kernel");
     const uint32_t park_cap0 = park_recs / 4 * 3;
-    const ParkIO regions[2] = {{B.park.as<uint32_t>(), park_cap0, 0u, 0u},
-                               {B.park.as<uint32_t>() + size_t(park_cap0) * kParkWords, park_recs - park_cap0, 0u, 1u}};
+    const uint32_t min_rays = c->tuning.park_steps != RC_PARK_STEPS_DEFAULT ? 0u
+                              : !shape.concurrent                             ? kParkRays
+                                                                          : kParkRaysConcurrent;
+    const ParkIO regions[2] = {{B.park.as<uint32_t>(), park_cap0, 0u, 0u, min_rays},
+                               {B.park.as<uint32_t>() + size_t(park_cap0) * kParkWords, park_recs - park_cap0, 0u, 1u, min_rays}};
     const bool timed = st == c->stream;  // profiling events live on the context stream
     PassParams P = base_params(cam, cfg);
     P.stack_limit = c->stack_depth();
@@ -1432,7 +1318,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
             if (timed) RC_TRY(c->prof_begin(&ev));
             const bool camb = RC_FUSED_CAMERA && k == 0;
             ParkIO PK = regions[0];
-            PK.steps = camb ? 0u : c->tuning.park_steps;
+            PK.steps = camb || n < min_rays ? 0u : c->tuning.park_steps;
             ExtendArgs ea{P, k, s, rin, sin_, rout, sout, srays, scontrib, L, ovf, deep.deep_stack, ctr, cin, cout, CI, W, PK};
             launch_extend(ea, n, st, c->counting, camb, c->hit_fp64, shape.ext_block);
             if (PK.steps)
@@ -1454,13 +1340,8 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
                 uint8_t* occ_out = nee_fix ? socc : nullptr;
                 k_reset_shadow<<<1, 1, 0, st>>>(ctr);
                 if (timed) RC_TRY(c->prof_begin(&ev));
-                ParkIO SPK = regions[0];
-                SPK.steps = c->tuning.park_steps ? uint32_t(RC_SHADOW_PARK_STEPS) : 0u;
-                ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit, SPK};
+                ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit};
                 launch_shadow(sa_, n, st, c->counting, c->hit_fp64, shape.shadow_block);
-                if (SPK.steps)
-                    launch_shadow_resumes(sa_, regions, RC_SHADOW_PARK_PHASES, RC_PARK_STEPS2, st, c->counting,
-                                          c->hit_fp64, shape.shadow_block);
                 if (timed) RC_TRY(c->prof_end(ev, PK_SHADOW));
                 deep.any = true;
                 deep.rays = srays;
