@@ -350,15 +350,31 @@ __device__ __forceinline__ bool training_path(const PassParams& P, uint32_t slot
     return h % stride == 0u;
 }
 
+// Where a path's radiance is summed: its slot's word in memory, or the lane's
+// registers.  add: thr * e more.
+struct SlotSum {
+    float4* __restrict__ L;
+    __device__ __forceinline__ void add(uint32_t slot, float3 thr, float3 e) const {
+        const float4 l = ld_stream(&L[slot]);
+        st_stream(&L[slot], make_float4(l.x + thr.x * e.x, l.y + thr.y * e.y, l.z + thr.z * e.z, l.w));
+    }
+};
+struct LaneSum {
+    float3& l;
+    __device__ __forceinline__ void add(uint32_t, float3 thr, float3 e) const {
+        l = make_float3(l.x + thr.x * e.x, l.y + thr.y * e.y, l.z + thr.z * e.z);
+    }
+};
+
 // One path vertex: PathTracer::traceRecursive (PathTracer.cpp:25-75) for the
 // hit (t, tri) of ray (r0, r1), plus sky on a miss, sun next-event estimation
-// and Russian roulette.  Radiance goes to L[slot]; the continuation and the
-// shadow ray are returned for the caller to append.  CACHE false: the caller
-// is the camera bounce, whose vertex is never the cache vertex.
-template <bool CACHE = true>
+// and Russian roulette.  Radiance goes to the path's sum; the continuation and the
+// shadow ray are returned for the caller to append.  CACHE false: the vertex
+// is never the cache vertex (the camera bounce's, k_paths').
+template <bool CACHE = true, class Sum>
 __device__ __forceinline__ ShadeOut shade_vertex(const PassParams& P, uint32_t k, float4 r0, float4 r1, float4 s,
                                                  float t, int tri, const float4* __restrict__ shade,
-                                                 const DevMaterial* __restrict__ mats, float4* __restrict__ L,
+                                                 const DevMaterial* __restrict__ mats, const Sum& sum,
                                                  const CacheIO& CI) {
     ShadeOut O;
     O.alive = O.shadow = O.query = O.train = false;
@@ -367,17 +383,14 @@ __device__ __forceinline__ ShadeOut shade_vertex(const PassParams& P, uint32_t k
     uint32_t slot = __float_as_uint(s.w);
     float3 thr = f3(s);
     if (tri < 0) {
-        float4 l = ld_stream(&L[slot]);
-        st_stream(&L[slot], make_float4(l.x + thr.x * P.sky.x, l.y + thr.y * P.sky.y, l.z + thr.z * P.sky.z, l.w));
+        sum.add(slot, thr, P.sky);
         return O;
     }
     float4 sh = shade[tri];
     const DevMaterial& m = mats[__float_as_uint(sh.w)];
     float4 dif = m.diffuse;
     if (__float_as_uint(dif.w) & RC_MAT_EMISSIVE) {
-        float4 e = m.emittance;
-        float4 l = ld_stream(&L[slot]);
-        st_stream(&L[slot], make_float4(l.x + thr.x * e.x, l.y + thr.y * e.y, l.z + thr.z * e.z, l.w));
+        sum.add(slot, thr, f3(m.emittance));
         return O;
     }
     float3 nrm = f3(sh);
@@ -588,7 +601,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
                 const float4 s = ld_stream(&st[i]);
                 slot = __float_as_uint(s.w);
                 O = shade_vertex(P, k, make_float4(S.o.x, S.o.y, S.o.z, 0.0f), make_float4(S.d.x, S.d.y, S.d.z, 0.0f),
-                                 s, S.R.t, S.R.id == kNoHit ? -1 : int(S.R.id), shade, mats, L, CI);
+                                 s, S.R.t, S.R.id == kNoHit ? -1 : int(S.R.id), shade, mats, SlotSum{L}, CI);
             }
         }
     } else if (i < n) {
@@ -623,7 +636,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
             }
             ovf_list[atomicAdd(&ctr->ovf_count, 1u)] = i;
         } else {
-            O = shade_vertex<!CAM>(P, k, r0, r1, s, R.t, R.id == kNoHit ? -1 : int(R.id), shade, mats, L, CI);
+            O = shade_vertex<!CAM>(P, k, r0, r1, s, R.t, R.id == kNoHit ? -1 : int(R.id), shade, mats, SlotSum{L}, CI);
         }
     }
     emit_vertex<BLOCK, !CAM>(P, k, O, slot, rays_out, st_out, srays, scontrib, ctr, cout, CI, shade, mats, L,
@@ -699,7 +712,7 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_resume(
             const float4 s = ld_stream(&st[i]);
             slot = __float_as_uint(s.w);
             O = shade_vertex(P, k, make_float4(S.o.x, S.o.y, S.o.z, 0.0f), make_float4(S.d.x, S.d.y, S.d.z, 0.0f), s,
-                             S.R.t, S.R.id == kNoHit ? -1 : int(S.R.id), shade, mats, L, CI);
+                             S.R.t, S.R.id == kNoHit ? -1 : int(S.R.id), shade, mats, SlotSum{L}, CI);
         }
     }
     emit_vertex<BLOCK>(P, k, O, slot, rays_out, st_out, srays, scontrib, ctr, cout, CI, shade, mats, L, append_scratch);
@@ -733,7 +746,7 @@ __global__ __launch_bounds__(kBlock) void k_shade_listed(PassParams P, uint32_t 
             float4 s = ld_stream(&st[i]);
             float4 h = reinterpret_cast<const float4*>(hits)[i];
             slot = __float_as_uint(s.w);
-            O = shade_vertex(P, k, rp[0], rp[1], s, h.x, __float_as_int(h.w), shade, mats, L, CI);
+            O = shade_vertex(P, k, rp[0], rp[1], s, h.x, __float_as_int(h.w), shade, mats, SlotSum{L}, CI);
         }
         emit_vertex<0>(P, k, O, slot, rays_out, st_out, srays, scontrib, ctr, cout, CI, shade, mats, L);
     }
@@ -805,6 +818,100 @@ __global__ __launch_bounds__(kBlock) void k_shadow_apply_listed(const float4* __
     }
 }
 
+// A sum rounded by itself: never fused with a product before it.
+__device__ __forceinline__ float add_alone(float a, float b) {
+#pragma clang fp contract(off)
+    return a + b;
+}
+
+// Whole paths, one per lane: the camera ray, then the extension, shading and
+// shadow ray of vertex after vertex, the radiance summed in registers in the
+// order the queues' kernels add it, so a slot holds the same bits.  A path
+// with a stack that outgrows its rows and finds no spill slot is listed and
+// traced again by the DEEP kernel, whose lanes' stacks lie in global memory.
+//
+// For passes that fit on the chip at once (kPathsPerCu): there the queues'
+// kernels, two to four per vertex, are bound by their launches and each by its
+// longest ray, while the compaction they are for saves nothing.  262,144 paths
+// of up to 6 vertices, queues against this: the box 218 and 153 us, terrains
+// of 512, 131,072 and 2,093,058 triangles 285 and 183, 832 and 399, 1142 and
+// 618, 200,000 random triangles 1863 and 1216; 12,288 paths 178 and 117, 251
+// and 143, 620 and 305, 926 and 446, 1575 and 889.  At twice the size the
+// lanes of ended paths begin to cost more than the launches: the box 269 and
+// 246, 20,000 random triangles 1322 and 1405.
+// One wave per block, so that few paths spread over all compute units (12,288
+// paths over 2,093,058 triangles: 446 us, in blocks of 256 515).  Compiled for
+// four waves per SIMD, the 128 registers a path's state and traversal need.
+constexpr int kPathBlock = 64, kPathWaves = 4;
+constexpr size_t kPathsPerCu = size_t(kPathWaves) * 4 * 64;  // lanes of a compute unit
+template <bool DEC64, bool DEEP>
+__global__ __launch_bounds__(kPathBlock, DEC64 || DEEP ? 1 : kPathWaves) void k_paths(
+    PassParams P, const NodeT* __restrict__ nodes, const TriRec* __restrict__ tris, const float4* __restrict__ shade,
+    const DevMaterial* __restrict__ mats, float4* __restrict__ L, float* __restrict__ W, uint32_t* __restrict__ list,
+    uint32_t* __restrict__ gstack, DevCounters* __restrict__ ctr) {
+    __shared__ uint32_t stack[DEEP ? 1 : kLdsStack * kPathBlock];
+    __shared__ uint4 top[4 * kTopNodes];
+    const uint32_t ntop = load_top(nodes, top);
+    const uint32_t thread = blockIdx.x * kPathBlock + threadIdx.x;
+    const StackMem M = DEEP ? stack_mem(gstack, thread, kDeepThreads, kDeepStack)
+                            : stack_mem(stack, threadIdx.x, kPathBlock, P.stack_limit, gstack, &ctr->spill);
+    const uint32_t n = DEEP ? ctr->ovf_count : P.npix * P.spp_pass;
+    if (DEEP && thread == 0 && n) atomicAdd(&ctr->spill.total, (unsigned long long)n);
+    uint32_t ext = 0, shadow = 0, n_rec = 0, n_tri = 0;
+    for (uint32_t i = thread; i < n; i += DEEP ? uint32_t(kDeepThreads) : n) {
+        const uint32_t slot = DEEP ? list[i] : i;
+        float4 r0, r1, s = make_float4(1.0f, 1.0f, 1.0f, __uint_as_float(slot));
+        const float weight = camera_ray(P, slot, r0, r1);
+        float3 sum = make_float3(0.0f, 0.0f, 0.0f);
+        uint32_t path_ext = 0, path_shadow = 0;
+        bool alive = true, listed = false;
+        for (uint32_t k = 0; alive; ++k) {
+            const TraceResult R = traverse<false, false, DEC64>(nodes, tris, f3(r0), f3(r1), 0.0f, __builtin_inff(), M,
+                                                                n_rec, n_tri, top, ntop, false);
+            path_ext += 1;
+            listed = R.overflow;
+            if (listed) break;
+            const ShadeOut O = shade_vertex<false>(P, k, r0, r1, s, R.t, R.id == kNoHit ? -1 : int(R.id), shade, mats,
+                                                   LaneSum{sum}, CacheIO{});
+            if (O.shadow) {
+                path_shadow += 1;
+                const TraceResult H = traverse<true, false, DEC64>(nodes, tris, O.so, P.sun, 0.0f, __builtin_inff(), M,
+                                                                   n_rec, n_tri, top, ntop, false);
+                listed = H.overflow;
+                if (listed) break;
+                if (H.id == kNoHit)
+                    sum = make_float3(add_alone(sum.x, O.contrib.x), add_alone(sum.y, O.contrib.y),
+                                      add_alone(sum.z, O.contrib.z));
+            }
+            alive = O.alive;
+            r0 = make_float4(O.newo.x, O.newo.y, O.newo.z, 0.0f);
+            r1 = make_float4(O.newd.x, O.newd.y, O.newd.z, 0.0f);
+            s = make_float4(O.thr.x, O.thr.y, O.thr.z, s.w);
+        }
+        if (listed) {
+            if (DEEP) ctr->error = 1;  // unreachable: the upload rejects trees this deep
+            else list[atomicAdd(&ctr->ovf_count, 1u)] = slot;
+            continue;
+        }
+        W[slot] = weight;
+        st_stream(&L[slot], make_float4(sum.x, sum.y, sum.z, 0.0f));
+        ext += path_ext;
+        shadow += path_shadow;
+    }
+    wave_add(&ctr->ext_rays, ext);
+    wave_add(&ctr->shadow_rays, shadow);
+}
+
+template <bool DEC64>
+void launch_paths(const PassParams& P, const rc_scene* s, float4* L, float* W, uint32_t* list, uint32_t* gstack,
+                  DevCounters* ctr, uint32_t n, bool deep, hipStream_t st) {
+    k_paths<DEC64, false><<<(n + kPathBlock - 1) / kPathBlock, kPathBlock, 0, st>>>(
+        P, s->nodes, tri_array<DEC64>(s), s->shade, s->mats, L, W, list, gstack, ctr);
+    if (deep)
+        k_paths<DEC64, true><<<kDeepThreads / kPathBlock, kPathBlock, 0, st>>>(P, s->nodes, tri_array<DEC64>(s), s->shade, s->mats, L,
+                                                               W, list, gstack, ctr);
+}
+
 // Training samples of a pass: query + target (L_final - L_before) / T for the
 // recorded training vertices, appended to the frame's batch (capped); also
 // adds the pass's query count to the frame total (kCcFrameQueries).
@@ -864,8 +971,9 @@ __global__ void k_prep(DevCounters* ctr, uint32_t cout) {
     ctr->park_count[1] = 0;
 }
 
-// Before a shadow pass: the overflow list and the spill slots are free.
-__global__ void k_reset_shadow(DevCounters* ctr) {
+// Before a shadow pass, or whole paths: the overflow list and the spill slots
+// are free.
+__global__ void k_reset_ovf(DevCounters* ctr) {
     ctr->ovf_count = 0;
     ctr->spill.claimed = 0;
 }
@@ -1286,6 +1394,12 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
     deep.counting = c->counting;
     deep.dec64 = c->hit_fp64;
     deep.max_depth = P.stack_limit;
+    // whole paths in one kernel: node and triangle counts stay those of the
+    // queues' kernels, and a budget other than the default asks for parking;
+    // frames beside each other fill the gaps and the tails with queues (eight
+    // soups in one graph take 12.7 ms, 13.1 with whole paths in the smaller)
+    const bool whole_paths = !shape.concurrent && npaths <= size_t(c->cu_count) * kPathsPerCu && !c->counting && !CI.cache_vertex &&
+                             (c->tuning.park_steps == 0 || c->tuning.park_steps == RC_PARK_STEPS_DEFAULT);
     for (uint32_t s0 = 0; s0 < cfg->spp; s0 += spp_pass) {
         if (progress) {
             RC_TRY_HIP(hipStreamSynchronize(st));
@@ -1300,6 +1414,17 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
         deep.n_bound = n;
         const bool listed = rc_may_list(s, P.stack_limit, n);
         hipEvent_t ev = nullptr;
+        if (whole_paths) {
+            if (rc_may_spill(s, P.stack_limit)) k_reset_ovf<<<1, 1, 0, st>>>(ctr);
+            if (timed) RC_TRY(c->prof_begin(&ev));
+            (c->hit_fp64 ? launch_paths<true> : launch_paths<false>)(P, s, L, W, ovf, deep.deep_stack, ctr, n, listed, st);
+            if (timed) RC_TRY(c->prof_end(ev, PK_EXTEND));
+            if (timed) RC_TRY(c->prof_begin(&ev));
+            launch_film_add(st, P.order, npix, this_pass, L, W, f->sum, f->comp);
+            if (timed) RC_TRY(c->prof_end(ev, PK_OTHER));
+            RC_TRY_HIP(hipGetLastError());
+            continue;
+        }
         if (CI.cache_vertex) k_cache_reset<<<1, 1, 0, st>>>(CI.counters, 0);
         if (RC_FUSED_CAMERA) {
             k_pass_start<<<1, 1, 0, st>>>(ctr, n);
@@ -1338,7 +1463,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
                 // at the cache vertex the shadow results are kept for the training records
                 const bool nee_fix = CI.cache_vertex && k == CI.cache_vertex;
                 uint8_t* occ_out = nee_fix ? socc : nullptr;
-                k_reset_shadow<<<1, 1, 0, st>>>(ctr);
+                k_reset_ovf<<<1, 1, 0, st>>>(ctr);
                 if (timed) RC_TRY(c->prof_begin(&ev));
                 ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit};
                 launch_shadow(sa_, n, st, c->counting, c->hit_fp64, shape.shadow_block);
