@@ -10,6 +10,7 @@
 #include <cstring>
 #include <new>
 
+#include "host/rc_stream_copy.hpp"
 #include "rc_internal.hpp"
 
 // 1: the FlatBVH is collapsed into 4-wide nodes by the SAH-optimal dynamic
@@ -108,6 +109,75 @@ int rc_ctx::prof_collect() {
     return RC_OK;
 }
 
+namespace {
+void stage_release(rc_ctx* c) {
+    for (hipEvent_t e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->stage) (void)hipHostFree(c->stage);
+}
+
+// Whether the runtime knows the memory at p (page-locked, or a device's own):
+// then it copies from or to it as it is.
+bool known_memory(const void* p) {
+    hipPointerAttribute_t a;
+    const bool known = hipPointerGetAttributes(&a, p) == hipSuccess && a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();  // an unknown pointer is an error to it
+    return known;
+}
+}  // namespace
+
+int rc_upload(rc_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (bytes == 0) return RC_OK;
+    if (!src) return rc_host_fail(RC_ERR_INVALID, "copy to the device: null array");
+    if (bytes > kStageUpload || known_memory(src)) {
+        RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        return RC_OK;
+    }
+    RC_TRY_HIP(hipEventSynchronize(c->stage_ev[0]));
+    std::memcpy(c->stage, src, bytes);
+    RC_TRY_HIP(hipMemcpyAsync(dst, c->stage, bytes, hipMemcpyHostToDevice, c->stream));
+    RC_TRY_HIP(hipEventRecord(c->stage_ev[0], c->stream));
+    return RC_OK;
+}
+
+namespace {
+void host_copy(void* dst, const void* src, size_t bytes) { std::memcpy(dst, src, bytes); }
+}  // namespace
+
+int rc_download(rc_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (bytes == 0) return RC_OK;
+    if (!dst) return rc_host_fail(RC_ERR_INVALID, "copy from the device: null array");
+    if (known_memory(dst)) {
+        RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        RC_TRY_HIP(hipStreamSynchronize(c->stream));
+        return RC_OK;
+    }
+    uint8_t* d = static_cast<uint8_t*>(dst);
+    const uint8_t* s = static_cast<const uint8_t*>(src);
+    auto queue = [&](size_t off, int q) {
+        RC_TRY_HIP(hipMemcpyAsync(c->stage + size_t(q) * kStageChunk, s + off, std::min(kStageChunk, bytes - off),
+                                  hipMemcpyDeviceToHost, c->stream));
+        RC_TRY_HIP(hipEventRecord(c->stage_ev[q], c->stream));
+        return int(RC_OK);
+    };
+    RC_TRY(queue(0, 0));
+    int q = 0;
+    for (size_t off = 0; off < bytes; off += kStageChunk, q ^= 1) {
+        if (off + kStageChunk < bytes) RC_TRY(queue(off + kStageChunk, q ^ 1));
+        RC_TRY_HIP(hipEventSynchronize(c->stage_ev[q]));
+        (bytes > kStageChunk ? rc_stream_copy : host_copy)(d + off, c->stage + size_t(q) * kStageChunk,
+                                                           std::min(kStageChunk, bytes - off));
+    }
+    return RC_OK;
+}
+
+int rc_small(rc_ctx* c, hipStream_t st, SmallResult which, const void* src, size_t bytes, const void** host) {
+    uint8_t* p = c->stage + 2 * kStageChunk + size_t(which) * kSmallBytes;
+    RC_TRY_HIP(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, st));
+    *host = p;
+    return RC_OK;
+}
+
 extern "C" int rc_create(int device, rc_ctx** out) {
     if (!out) return rc_host_fail(RC_ERR_INVALID, "rc_create: null out");
     *out = nullptr;
@@ -140,8 +210,19 @@ extern "C" int rc_create(int device, rc_ctx** out) {
     }
     (void)hipMemset(c->counters, 0, sizeof(DevCounters));
     c->fb.counters = c->counters;  // not owned by the frame buffers
+    if (hipHostMalloc(reinterpret_cast<void**>(&c->stage), 2 * kStageChunk + SMALL_RESULTS * kSmallBytes,
+                      hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&c->stage_ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->stage_ev[1], hipEventDisableTiming) != hipSuccess) {
+        stage_release(c);
+        (void)hipFree(c->counters);
+        (void)hipStreamDestroy(c->stream);
+        delete c;
+        return rc_host_fail(RC_ERR_ALLOC, "rc_create: page-locked memory");
+    }
     int se2 = rc_noalloc_setup(device);  // this device's copy of the allocation-free scratch
     if (se2 != RC_OK) {
+        stage_release(c);
         (void)hipFree(c->counters);
         (void)hipStreamDestroy(c->stream);
         delete c;
@@ -168,6 +249,7 @@ extern "C" int rc_destroy(rc_ctx* c) {
     for (hipStream_t b : c->branch_streams) (void)hipStreamDestroy(b);
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
     if (c->copy_ev) (void)hipEventDestroy(c->copy_ev);
+    stage_release(c);
     c->branch_streams.clear();
     for (hipEvent_t e : c->branch_events) (void)hipEventDestroy(e);
     c->branch_events.clear();
@@ -833,15 +915,13 @@ extern "C" int rc_host_free(rc_ctx* c, void* p) {
 }
 extern "C" int rc_memcpy_h2d(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     RC_TRY(rc_check_ctx(c, "rc_memcpy_h2d"));
-    RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+    RC_TRY(rc_upload(c, dst, src, bytes));
     RC_TRY_HIP(hipStreamSynchronize(c->stream));
     return RC_OK;
 }
 extern "C" int rc_memcpy_d2h(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     RC_TRY(rc_check_ctx(c, "rc_memcpy_d2h"));
-    RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    return RC_OK;
+    return rc_download(c, dst, src, bytes);
 }
 
 // ---------------------------------------------------------------- bandwidth probes

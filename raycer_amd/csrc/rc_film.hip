@@ -243,9 +243,7 @@ extern "C" int rc_film_download_linear(rc_ctx* c, const rc_film* f, float* rgba)
     RC_TRY(mf->linear.ensure(size_t(npix) * sizeof(float4)));
     k_film_linear<<<(npix + kBlock - 1) / kBlock, kBlock, 0, c->stream>>>(f->sum, f->comp, npix, mf->linear.as<float4>());
     RC_TRY_HIP(hipGetLastError());
-    RC_TRY_HIP(hipMemcpyAsync(rgba, mf->linear.p, size_t(npix) * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    return RC_OK;
+    return rc_download(c, rgba, mf->linear.p, size_t(npix) * sizeof(float4));
 }
 
 extern "C" int rc_film_download_sums(rc_ctx* c, const rc_film* f, float* sums) {
@@ -256,9 +254,7 @@ extern "C" int rc_film_download_sums(rc_ctx* c, const rc_film* f, float* sums) {
     RC_TRY(mf->linear.ensure(size_t(npix) * sizeof(float4)));
     k_film_sums<<<(npix + kBlock - 1) / kBlock, kBlock, 0, c->stream>>>(f->sum, f->comp, npix, mf->linear.as<float4>());
     RC_TRY_HIP(hipGetLastError());
-    RC_TRY_HIP(hipMemcpyAsync(sums, mf->linear.p, size_t(npix) * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    return RC_OK;
+    return rc_download(c, sums, mf->linear.p, size_t(npix) * sizeof(float4));
 }
 
 extern "C" int rc_film_tonemap(rc_ctx* c, const rc_film* f, const rc_tonemap* tm, float* rgba, double* log_avg,
@@ -298,10 +294,10 @@ extern "C" int rc_film_tonemap(rc_ctx* c, const rc_film* f, const rc_tonemap* tm
     }
     k_tone_map<<<grid, kBlock, 0, c->stream>>>(lin, npix, part, nparts, M, outd);
     RC_TRY_HIP(hipGetLastError());
-    RC_TRY_HIP(hipMemcpyAsync(rgba, outd, size_t(npix) * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    double2 st = make_double2(0.0, 0.0);
-    if (reinhard) RC_TRY_HIP(hipMemcpyAsync(&st, part + nparts, sizeof(double2), hipMemcpyDeviceToHost, c->stream));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
+    const void* st_host = nullptr;
+    if (reinhard) RC_TRY(rc_small(c, c->stream, SMALL_TONEMAP, part + nparts, sizeof(double2), &st_host));
+    RC_TRY(rc_download(c, rgba, outd, size_t(npix) * sizeof(float4)));  // behind it on the stream
+    const double2 st = reinhard ? *static_cast<const double2*>(st_host) : make_double2(0.0, 0.0);
     if (averaging) mf->max_lum_average = st.y;
     if (log_avg) *log_avg = st.x;
     if (max_lum) *max_lum = st.y;

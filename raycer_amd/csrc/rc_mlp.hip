@@ -665,8 +665,8 @@ rc_ctx* rc_cache_owner(const rc_cache* k) { return k->ctx; }
 
 int rc_cache_frame_end(rc_ctx* c, hipStream_t st, rc_cache* k, uint32_t steps, uint32_t counts[2]) {
     k_cache_frame_end<<<1, 1, 0, st>>>(k->counters, k->cfg.max_batch, k->cfg.train_stride == 0 ? 1u : 0u);
-    uint32_t h[2];  // training samples, cache queries of the frame
-    RC_TRY_HIP(hipMemcpyAsync(h, k->counters + kCcSamples, sizeof(h), hipMemcpyDeviceToHost, st));
+    const void* host = nullptr;  // training samples, cache queries of the frame
+    RC_TRY(rc_small(c, st, SMALL_CACHE, k->counters + kCcSamples, 2 * sizeof(uint32_t), &host));
     k->last_steps = steps;
     if (steps > 0) {
         // the optimizer steps wait for the frame's samples on the cache's stream
@@ -685,6 +685,7 @@ int rc_cache_frame_end(rc_ctx* c, hipStream_t st, rc_cache* k, uint32_t steps, u
         c->train_ev1 = k->ev_trained;
     }
     RC_TRY_HIP(hipStreamSynchronize(st));
+    const uint32_t* h = static_cast<const uint32_t*>(host);
     counts[0] = h[1];
     counts[1] = std::min(h[0], k->cfg.max_batch);
     return RC_OK;
@@ -804,10 +805,10 @@ extern "C" int rc_cache_get_params(rc_cache* k, float* params) {
 namespace {
 int stage(rc_ctx* c, rc_cache* k, const float* q, const float* t, size_t n) {
     RC_TRY(k->queries.ensure(n * 12 * 4));
-    RC_TRY_HIP(hipMemcpyAsync(k->queries.p, q, n * 12 * 4, hipMemcpyHostToDevice, c->stream));
+    RC_TRY(rc_upload(c, k->queries.p, q, n * 12 * 4));
     if (t) {
         RC_TRY(k->targets.ensure(n * 3 * 4));
-        RC_TRY_HIP(hipMemcpyAsync(k->targets.p, t, n * 3 * 4, hipMemcpyHostToDevice, c->stream));
+        RC_TRY(rc_upload(c, k->targets.p, t, n * 3 * 4));
     }
     return RC_OK;
 }
@@ -826,9 +827,7 @@ extern "C" int rc_cache_infer(rc_ctx* c, rc_cache* k, const float* q, size_t n, 
                                                                         k->queries.as<float>(), uint32_t(n), nullptr,
                                                                         k->out.as<float>());
     RC_TRY_HIP(hipGetLastError());
-    RC_TRY_HIP(hipMemcpyAsync(out, k->out.p, n * 3 * 4, hipMemcpyDeviceToHost, c->stream));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    return RC_OK;
+    return rc_download(c, out, k->out.p, n * 3 * 4);
 }
 
 extern "C" int rc_cache_gradient(rc_ctx* c, rc_cache* k, const float* q, const float* t, size_t n, float* grad,
@@ -840,11 +839,11 @@ extern "C" int rc_cache_gradient(rc_ctx* c, rc_cache* k, const float* q, const f
     RC_TRY(stage(c, k, q, t, n));
     k_zero_f<<<1, kThreads, 0, c->stream>>>(k->loss, 1);
     RC_TRY(grad_device(c, c->stream, k, k->queries.as<float>(), k->targets.as<float>(), uint32_t(n), nullptr, 1, 0));
-    if (grad) RC_TRY_HIP(hipMemcpyAsync(grad, k->grad, kParams * 4, hipMemcpyDeviceToHost, c->stream));
-    float l = 0.0f;
-    RC_TRY_HIP(hipMemcpyAsync(&l, k->loss, 4, hipMemcpyDeviceToHost, c->stream));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    if (loss) *loss = l;
+    const void* l = nullptr;
+    RC_TRY(rc_small(c, c->stream, SMALL_LOSS, k->loss, 4, &l));
+    if (grad) RC_TRY(rc_download(c, grad, k->grad, kParams * 4));  // behind it on the stream
+    else RC_TRY_HIP(hipStreamSynchronize(c->stream));
+    if (loss) *loss = *static_cast<const float*>(l);
     return RC_OK;
 }
 

@@ -1555,10 +1555,11 @@ int render_frame(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_camera* cam,
                               cache);
     uint32_t cache_counts[2] = {0, 0};
     if (rc == RC_OK && cache) rc = rc_cache_frame_end(c, c->stream, cache, train, cache_counts);
+    const void* host = nullptr;
+    if (rc == RC_OK) rc = rc_small(c, c->stream, SMALL_COUNTERS, c->counters, sizeof(DevCounters), &host);
     RC_TRY_HIP(hipStreamSynchronize(c->stream));
     if (rc != RC_OK) return rc;
-    DevCounters h;
-    RC_TRY_HIP(hipMemcpy(&h, c->counters, sizeof(DevCounters), hipMemcpyDeviceToHost));
+    const DevCounters& h = *static_cast<const DevCounters*>(host);
     if (h.error) return rc_host_fail(RC_ERR_HIP, "rc_render: traversal stack exceeded the deep-stack limit");
     c->stats.render_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     RC_TRY(c->prof_collect());

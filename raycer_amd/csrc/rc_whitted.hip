@@ -670,8 +670,10 @@ struct Run {
             k_wt_total<<<1, 1, 0, c->stream>>>(cnt[q], off[q], base + n - 1, dev + q);
         }
         RC_TRY_HIP(hipGetLastError());
-        RC_TRY_HIP(hipMemcpyAsync(out, dev, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+        const void* host = nullptr;
+        RC_TRY(rc_small(c, c->stream, SMALL_TOTALS, dev, 3 * sizeof(uint32_t), &host));
         RC_TRY_HIP(hipStreamSynchronize(c->stream));
+        std::memcpy(out, host, 3 * sizeof(uint32_t));
         return RC_OK;
     }
 
@@ -879,9 +881,10 @@ extern "C" int rc_raytrace(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_ca
         RC_TRY(run.process(0, 0, n0));
         RC_TRY(rc_launch_film_add(c, f, cfg, this_pass, run.L, c->fb.slotW.as<float>()));
     }
+    const void* host = nullptr;
+    RC_TRY(rc_small(c, c->stream, SMALL_COUNTERS, c->counters, sizeof(DevCounters), &host));
     RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    DevCounters h;
-    RC_TRY_HIP(hipMemcpy(&h, c->counters, sizeof(DevCounters), hipMemcpyDeviceToHost));
+    const DevCounters& h = *static_cast<const DevCounters*>(host);
     if (h.error) return rc_host_fail(RC_ERR_HIP, "rc_raytrace: traversal stack exceeded the deep-stack limit");
     c->stats = rc_stats{};
     c->stats.extension_rays = run.ext_rays;
