@@ -116,20 +116,30 @@ void stage_release(rc_ctx* c) {
     if (c->stage) (void)hipHostFree(c->stage);
 }
 
-// Whether the runtime knows the memory at p (page-locked, or a device's own):
-// then it copies from or to it as it is.
-bool known_memory(const void* p) {
+}  // namespace
+
+bool rc_known_memory(const void* p) {
     hipPointerAttribute_t a;
     const bool known = hipPointerGetAttributes(&a, p) == hipSuccess && a.type != hipMemoryTypeUnregistered;
     (void)hipGetLastError();  // an unknown pointer is an error to it
     return known;
 }
-}  // namespace
+
+void* rc_mapped(void* p, size_t bytes, size_t align) {
+    hipPointerAttribute_t a, b;
+    const bool mapped = p && hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeHost &&
+                        hipPointerGetAttributes(&b, static_cast<uint8_t*>(p) + bytes - 1) == hipSuccess &&
+                        b.type == hipMemoryTypeHost && a.devicePointer &&
+                        b.devicePointer == static_cast<uint8_t*>(a.devicePointer) + bytes - 1 &&
+                        reinterpret_cast<uintptr_t>(a.devicePointer) % align == 0;
+    (void)hipGetLastError();
+    return mapped ? a.devicePointer : nullptr;
+}
 
 int rc_upload(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     if (bytes == 0) return RC_OK;
     if (!src) return rc_host_fail(RC_ERR_INVALID, "copy to the device: null array");
-    if (bytes > kStageUpload || known_memory(src)) {
+    if (bytes > kStageUpload || rc_known_memory(src)) {
         RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
         return RC_OK;
     }
@@ -147,7 +157,7 @@ void host_copy(void* dst, const void* src, size_t bytes) { std::memcpy(dst, src,
 int rc_download(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     if (bytes == 0) return RC_OK;
     if (!dst) return rc_host_fail(RC_ERR_INVALID, "copy from the device: null array");
-    if (known_memory(dst)) {
+    if (rc_known_memory(dst)) {
         RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
         RC_TRY_HIP(hipStreamSynchronize(c->stream));
         return RC_OK;
@@ -247,8 +257,6 @@ extern "C" int rc_destroy(rc_ctx* c) {
     }
     c->branches.clear();
     for (hipStream_t b : c->branch_streams) (void)hipStreamDestroy(b);
-    if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
-    if (c->copy_ev) (void)hipEventDestroy(c->copy_ev);
     stage_release(c);
     c->branch_streams.clear();
     for (hipEvent_t e : c->branch_events) (void)hipEventDestroy(e);
@@ -908,7 +916,6 @@ extern "C" int rc_host_free(rc_ctx* c, void* p) {
     RC_TRY(rc_check_ctx(c, "rc_host_free"));
     if (p) {
         RC_TRY_HIP(hipStreamSynchronize(c->stream));
-        if (c->copy_stream) RC_TRY_HIP(hipStreamSynchronize(c->copy_stream));
         RC_TRY_HIP(hipHostFree(p));
     }
     return RC_OK;

@@ -114,8 +114,6 @@ struct rc_ctx {
     std::vector<uint8_t> batch_key;           // every value the cached batch graph's kernels were captured with
     std::vector<FrameBuffers*> branches;      // a batch's concurrent branches beyond the first (which uses fb)
     std::vector<hipStream_t> branch_streams;
-    hipStream_t copy_stream = nullptr;  // device-to-host copies that overlap the main stream's kernels
-    hipEvent_t copy_ev = nullptr;
     uint8_t* stage = nullptr;  // page-locked: two chunks that copies go through, then small results (rc_small)
     hipEvent_t stage_ev[2] = {nullptr, nullptr};  // the last copy that used each chunk
     std::vector<hipEvent_t> branch_events;    // fork / join of the branches under capture
@@ -247,6 +245,12 @@ struct CacheIO {
     uint32_t cap;           // record / query capacity of a pass
 };
 
+// Whether the runtime knows the memory at p (page-locked, or a device's own):
+// then it copies from or to it as it is.
+bool rc_known_memory(const void* p);
+// The device's address of page-locked host memory [p, p + bytes); null when p
+// is null, other memory or not aligned to `align`.
+void* rc_mapped(void* p, size_t bytes, size_t align);
 // Copies between host arrays and the device, ordered on the context's stream,
 // through the context's page-locked chunks unless the array is page-locked (or
 // device memory) itself.  The upload returns when src may be changed (page-locked: when the

@@ -1607,83 +1607,119 @@ extern "C" int rc_render_cached(rc_ctx* c, const rc_scene* s, rc_film* f, const 
 // ---------------------------------------------------------------- Phong raycast
 namespace {
 
-__global__ __launch_bounds__(kBlock) void k_cast_camera(CamBasis cam, uint32_t width, uint32_t npix, uint64_t seed,
-                                                        rc_ray* __restrict__ rays) {
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= npix) return;
-    float4 u = draw4(seed, p, 0, 0, kCamDim);
-    float3 d = cam_dir(cam, float(p % width) + u.x, float(p / width) + u.y);
-    float4* r = reinterpret_cast<float4*>(rays + p);
-    r[0] = make_float4(cam.pos.x, cam.pos.y, cam.pos.z, 0.0f);
-    r[1] = make_float4(d.x, d.y, d.z, __builtin_inff());
-}
-
+constexpr int kPhongWaves = 6;  // the FP32 kernel's waves per SIMD
 struct LightParams {
     float3 pos, color, ambient;
     float max_d, att, offset;
 };
 
-// Raytracer::calculateLightColor for one point light + calculatePhongShadingColor
-// (Raytracer.cpp:312-407); the shadow ray of calculateShadowAmount (:524-551)
-// starts rayStartOffset along the light direction and ends at the light.
-__global__ __launch_bounds__(kBlock) void k_phong_prepare(uint32_t npix, LightParams Lp, const rc_ray* __restrict__ rays,
-                                                          const rc_hit* __restrict__ hits,
-                                                          const float4* __restrict__ shade,
-                                                          const DevMaterial* __restrict__ mats,
-                                                          rc_ray* __restrict__ srays, float4* __restrict__ direct,
-                                                          float4* __restrict__ rgba, int32_t* __restrict__ ids,
-                                                          float* __restrict__ hit_t) {
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= npix) return;
-    float4 h = reinterpret_cast<const float4*>(hits)[p];
-    int tri = __float_as_int(h.w);
-    if (ids) ids[p] = tri;
-    if (hit_t) hit_t[p] = h.x;
-    float4* sr = reinterpret_cast<float4*>(srays + p);
-    if (tri < 0) {
-        sr[0] = make_float4(0.0f, 0.0f, 0.0f, 1.0f);  // empty interval: never occluded
-        sr[1] = make_float4(0.0f, 1.0f, 0.0f, 0.0f);
-        direct[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        rgba[p] = make_float4(0.0f, 0.0f, 0.0f, 1.0f);
-        return;
-    }
-    const float4* rp = reinterpret_cast<const float4*>(rays + p);
-    float3 o = f3(rp[0]), d = f3(rp[1]);
-    float3 pos = o + (h.x * d);
-    float4 sh = shade[tri];
-    const DevMaterial& m = mats[__float_as_uint(sh.w)];
-    float3 n = f3(sh), kd = f3(m.diffuse), ka = f3(m.ambient), ks = f3(m.specular);
-    float shin = m.emittance.w;
-    float3 col = mul3(Lp.ambient, ka);
-    float3 tl = Lp.pos - pos;
-    float dist = sqrtf(dot3(tl, tl));
-    float3 l = normalize3(tl);
-    float3 ph = make_float3(0.0f, 0.0f, 0.0f);
-    float diff = dot3(l, n);
-    if (diff > 0.0f) {
-        ph = mul3(Lp.color * diff, kd);
-        if (!(ks.x == 0.0f && ks.y == 0.0f && ks.z == 0.0f)) {
-            float3 refl = normalize3((2.0f * diff * n) - l);
-            float sa = dot3(refl, make_float3(-d.x, -d.y, -d.z));
-            if (sa > 0.0f) ph = ph + mul3(Lp.color * powf(sa, shin), ks);
+// A pixel's primary ray, its hit, Raytracer::calculateLightColor for one point
+// light + calculatePhongShadingColor (Raytracer.cpp:312-407) and the shadow ray
+// of calculateShadowAmount (:524-551), which starts rayStartOffset along the
+// light direction and ends at the light: all of it in the pixel's lane, so
+// nothing but the results reaches memory.  A wave is an 8x8 tile; its block's
+// four lie side by side and write rows of 32 pixels through LDS, since the
+// results may go straight to the caller's page-locked arrays, over the bus.
+// Pixels with a stack that outgrows its rows and finds no spill slot are
+// listed and done by the DEEP kernel, whose lanes' stacks lie in global memory.
+//
+// Bound by the bus: 1080p results are 49.8 MB, 0.94 ms at the 53 GB/s it
+// carries, and the call takes 1.10 ms (1.28 in five kernels, rays and hits in
+// memory between them, rows of 64 pixels to a wave, and copies; this kernel
+// alone 0.45, those 0.85).  Rows of 8 pixels from each wave instead of the
+// block's 32: 1.15 ms; bands of rows copied beside the next one's kernel 1.28,
+// each ending with its longest rays.  5, 6 and 8 waves per SIMD: 1.104, 1.106
+// and 1.118.
+template <bool DEC64, bool DEEP>
+__global__ __launch_bounds__(DEEP ? 64 : kBlock, DEEP ? 1 : DEC64 ? RC_MIN_WAVES_FP64 : kPhongWaves) void k_phong(
+    CamBasis cam, uint32_t width, uint32_t height, uint64_t seed, LightParams Lp, const NodeT* __restrict__ nodes,
+    const TriRec* __restrict__ tris, const float4* __restrict__ shade, const DevMaterial* __restrict__ mats,
+    float4* __restrict__ rgba, int32_t* __restrict__ ids,
+    float* __restrict__ hit_t, uint32_t* __restrict__ list, uint32_t* __restrict__ gstack,
+    DevCounters* __restrict__ ctr, int stack_limit) {
+    __shared__ __align__(16) uint32_t stack[DEEP ? 1 : kLdsStack * kBlock];  // then the block's results
+    __shared__ uint4 top[4 * kTopNodes];
+    static_assert(kBlock == 256 && kLdsStack * kBlock >= 6 * kBlock, "a block is 32x8 pixels, six words each");
+    const uint32_t ntop = load_top(nodes, top);
+    const uint32_t thread = blockIdx.x * 64 + threadIdx.x;  // DEEP
+    const StackMem M = DEEP ? stack_mem(gstack, thread, kDeepThreads, kDeepStack)
+                            : stack_mem(stack, threadIdx.x, kBlock, stack_limit, gstack, &ctr->spill);
+    const uint32_t across = (width + 31) / 32, n = DEEP ? ctr->ovf_count : across * ((height + 7) / 8);
+    uint32_t n_rec = 0, n_tri = 0;
+    for (uint32_t b = DEEP ? thread : blockIdx.x; b < n; b += DEEP ? uint32_t(kDeepThreads) : gridDim.x) {
+        const uint32_t bx = (b % across) * 32, by = (b / across) * 8;
+        const uint32_t col0 = (threadIdx.x >> 6) * 8 + (threadIdx.x & 7u), row0 = (threadIdx.x >> 3) & 7u;
+        int32_t id = -1;
+        float dist_t = __builtin_inff();
+        float3 col = make_float3(0.0f, 0.0f, 0.0f);
+        if (DEEP || (bx + col0 < width && by + row0 < height)) {
+            const uint32_t p = DEEP ? list[b] : (by + row0) * width + bx + col0;
+            const float4 u = draw4(seed, p, 0, 0, kCamDim);
+            const float3 d = cam_dir(cam, float(p % width) + u.x, float(p / width) + u.y);
+            const TraceResult R = traverse<false, false, DEC64>(nodes, tris, cam.pos, d, 0.0f, __builtin_inff(), M, n_rec,
+                                                                n_tri, top, ntop, false);
+            bool listed = R.overflow;
+            const bool hit = !listed && R.id != kNoHit;
+            id = hit ? int32_t(R.id) : -1;
+            dist_t = hit ? R.t : __builtin_inff();
+            col = make_float3(0.0f, 0.0f, 0.0f);
+            if (hit) {
+                const float3 pos = cam.pos + (R.t * d);
+                const float4 sh = shade[R.id];
+                const DevMaterial& m = mats[__float_as_uint(sh.w)];
+                const float3 nrm = f3(sh), kd = f3(m.diffuse), ka = f3(m.ambient), ks = f3(m.specular);
+                const float shin = m.emittance.w;
+                col = mul3(Lp.ambient, ka);
+                const float3 tl = Lp.pos - pos;
+                const float dist = sqrtf(dot3(tl, tl));
+                const float3 l = normalize3(tl);
+                float3 ph = make_float3(0.0f, 0.0f, 0.0f);
+                const float diff = dot3(l, nrm);
+                if (diff > 0.0f) {
+                    ph = mul3(Lp.color * diff, kd);
+                    if (!(ks.x == 0.0f && ks.y == 0.0f && ks.z == 0.0f)) {
+                        const float3 refl = normalize3((2.0f * diff * nrm) - l);
+                        const float sa = dot3(refl, make_float3(-d.x, -d.y, -d.z));
+                        if (sa > 0.0f) ph = ph + mul3(Lp.color * powf(sa, shin), ks);
+                    }
+                }
+                float da = fminf(1.0f, dist / Lp.max_d);
+                da = 1.0f - powf(da, Lp.att);
+                const float3 so = pos + l * Lp.offset;
+                const TraceResult H = traverse<true, false, DEC64>(nodes, tris, so, l, 0.0f, dist, M, n_rec, n_tri, top,
+                                                                   ntop, false);
+                listed = H.overflow;
+                if (!listed && H.id == kNoHit)
+                    col = make_float3(add_alone(col.x, ph.x * da), add_alone(col.y, ph.y * da),
+                                      add_alone(col.z, ph.z * da));
+            }
+            if (listed) {
+                if (DEEP) ctr->error = 1;  // unreachable: the upload rejects trees this deep
+                else list[atomicAdd(&ctr->ovf_count, 1u)] = p;  // its results are written over
+            } else if (DEEP) {
+                if (ids) ids[p] = id;
+                if (hit_t) hit_t[p] = dist_t;
+                if (rgba) rgba[p] = make_float4(col.x, col.y, col.z, 1.0f);
+            }
+        }
+        if constexpr (!DEEP) {
+            __syncthreads();  // the stacks are done with
+            float4* out = reinterpret_cast<float4*>(stack);
+            uint32_t* word = stack + 4 * kBlock;
+            const uint32_t cell = row0 * 32 + col0;
+            out[cell] = make_float4(col.x, col.y, col.z, 1.0f);
+            word[cell] = uint32_t(id);
+            word[kBlock + cell] = __float_as_uint(dist_t);
+            __syncthreads();
+            const uint32_t x = bx + (threadIdx.x & 31u), y = by + (threadIdx.x >> 5), p = y * width + x;
+            if (x < width && y < height) {
+                if (ids) ids[p] = int32_t(word[threadIdx.x]);
+                if (hit_t) hit_t[p] = __uint_as_float(word[kBlock + threadIdx.x]);
+                if (rgba) rgba[p] = out[threadIdx.x];
+            }
+            __syncthreads();
         }
     }
-    float da = fminf(1.0f, dist / Lp.max_d);
-    da = 1.0f - powf(da, Lp.att);
-    float3 so = pos + l * Lp.offset;
-    sr[0] = make_float4(so.x, so.y, so.z, 0.0f);
-    sr[1] = make_float4(l.x, l.y, l.z, dist);
-    direct[p] = make_float4(ph.x * da, ph.y * da, ph.z * da, 0.0f);
-    rgba[p] = make_float4(col.x, col.y, col.z, 1.0f);
-}
-
-// Adds the unoccluded direct light.
-__global__ __launch_bounds__(kBlock) void k_phong_finish(uint32_t npix, const uint8_t* __restrict__ occ,
-                                                         const float4* __restrict__ direct, float4* __restrict__ rgba) {
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= npix || occ[p]) return;
-    float4 c = rgba[p], dd = direct[p];
-    rgba[p] = make_float4(c.x + dd.x, c.y + dd.y, c.z + dd.z, 1.0f);
 }
 
 }  // namespace
@@ -1710,49 +1746,38 @@ extern "C" int rc_raycast_phong(rc_ctx* c, const rc_scene* s, const rc_camera* c
     Lp.max_d = light->max_distance;
     Lp.att = light->attenuation;
     Lp.offset = offset;
-    const uint32_t grid = (npix + kBlock - 1) / kBlock;
     k_zero_counters<<<1, 1, 0, c->stream>>>(c->counters);
+    FrameBuffers& FB = c->fb;
+    // page-locked arrays take the results as they are written; the others get
+    // them from the queues' buffers
+    int32_t* ids_d = static_cast<int32_t*>(rc_mapped(hit_ids, npix * sizeof(int32_t), sizeof(int32_t)));
+    float* t_d = static_cast<float*>(rc_mapped(t, npix * sizeof(float), sizeof(float)));
+    float4* rgba_d = static_cast<float4*>(rc_mapped(rgba, npix * sizeof(float4), sizeof(float4)));
+    const bool ids_copy = hit_ids && !ids_d, t_copy = t && !t_d, rgba_copy = rgba && !rgba_d;
+    if (ids_copy) ids_d = FB.st_a.as<int32_t>();
+    if (t_copy) t_d = FB.st_b.as<float>();
+    if (rgba_copy) rgba_d = FB.slotL.as<float4>();
+    const int rows = c->stack_depth();
+    if (rc_may_spill(s, rows)) k_reset_ovf<<<1, 1, 0, c->stream>>>(c->counters);
     hipEvent_t ev;
     RC_TRY(c->prof_begin(&ev));
-    k_cast_camera<<<grid, kBlock, 0, c->stream>>>(B, w, npix, seed, c->fb.ray_a.as<rc_ray>());
-    RC_TRY(c->prof_end(ev, PK_OTHER));
-    FrameBuffers& FB = c->fb;
-    RC_TRY(rc_launch_trace(c, s, false, FB.ray_a.as<rc_ray>(), nullptr, npix, FB.hits.as<rc_hit>(), nullptr));
-    float4* rgba_d = FB.slotL.as<float4>();
-    // the hit indices and distances go to two device arrays (the queue
-    // buffers, free by now) as soon as the closest hits are known, and from
-    // there to the caller's arrays on the copy stream while the shadow rays
-    // are traced
-    int32_t* ids_d = hit_ids ? reinterpret_cast<int32_t*>(FB.st_a.p) : nullptr;
-    float* t_d = t ? reinterpret_cast<float*>(FB.st_b.p) : nullptr;
-    RC_TRY(c->prof_begin(&ev));
-    k_phong_prepare<<<grid, kBlock, 0, c->stream>>>(npix, Lp, FB.ray_a.as<rc_ray>(), FB.hits.as<rc_hit>(), s->shade,
-                                                    s->mats, FB.srays.as<rc_ray>(), FB.scontrib.as<float4>(), rgba_d,
-                                                    ids_d, t_d);
-    RC_TRY(c->prof_end(ev, PK_SHADE));
-    const bool side = hit_ids || t;
-    if (side) {
-        if (!c->copy_stream) RC_TRY_HIP(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
-        if (!c->copy_ev) RC_TRY_HIP(hipEventCreateWithFlags(&c->copy_ev, hipEventDisableTiming));
-        RC_TRY_HIP(hipEventRecord(c->copy_ev, c->stream));
-        RC_TRY_HIP(hipStreamWaitEvent(c->copy_stream, c->copy_ev, 0));
-        if (hit_ids)
-            RC_TRY_HIP(hipMemcpyAsync(hit_ids, ids_d, npix * sizeof(int32_t), hipMemcpyDeviceToHost, c->copy_stream));
-        if (t) RC_TRY_HIP(hipMemcpyAsync(t, t_d, npix * sizeof(float), hipMemcpyDeviceToHost, c->copy_stream));
+    const uint32_t grid = uint32_t(std::min<size_t>(size_t((w + 31) / 32) * ((h + 7) / 8), size_t(1) << 23));
+#define RC_PHONG(D, DEEP, GRID, BLOCK)                                                                            \
+    k_phong<D, DEEP><<<GRID, BLOCK, 0, c->stream>>>(B, w, h, seed, Lp, s->nodes, tri_array<D>(s), s->shade, s->mats, \
+                                                    rgba_d, ids_d, t_d, FB.ovf_list.as<uint32_t>(),               \
+                                                    FB.deep_stack.as<uint32_t>(), c->counters, rows)
+    if (c->hit_fp64) RC_PHONG(true, false, grid, kBlock);
+    else RC_PHONG(false, false, grid, kBlock);
+    if (rc_may_list(s, rows, npix)) {
+        if (c->hit_fp64) RC_PHONG(true, true, kDeepThreads / 64, 64);
+        else RC_PHONG(false, true, kDeepThreads / 64, 64);
     }
-    RC_TRY(rc_launch_trace(c, s, true, FB.srays.as<rc_ray>(), nullptr, npix, nullptr, FB.socc.as<uint8_t>()));
-    RC_TRY(c->prof_begin(&ev));
-    k_phong_finish<<<grid, kBlock, 0, c->stream>>>(npix, FB.socc.as<uint8_t>(), FB.scontrib.as<float4>(), rgba_d);
-    RC_TRY(c->prof_end(ev, PK_OTHER));
+#undef RC_PHONG
+    RC_TRY(c->prof_end(ev, PK_EXTEND));
     RC_TRY_HIP(hipGetLastError());
-    if (rgba) RC_TRY_HIP(hipMemcpyAsync(rgba, rgba_d, npix * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    if (side) {
-        // the ids and t buffers are the frame's queues: the next call on the
-        // main stream must not overwrite them before the copies are done
-        RC_TRY_HIP(hipEventRecord(c->copy_ev, c->copy_stream));
-        RC_TRY_HIP(hipStreamWaitEvent(c->stream, c->copy_ev, 0));
-        RC_TRY_HIP(hipStreamSynchronize(c->copy_stream));
-    }
+    if (ids_copy) RC_TRY(rc_download(c, hit_ids, ids_d, npix * sizeof(int32_t)));
+    if (t_copy) RC_TRY(rc_download(c, t, t_d, npix * sizeof(float)));
+    if (rgba_copy) RC_TRY(rc_download(c, rgba, rgba_d, npix * sizeof(float4)));
     RC_TRY_HIP(hipStreamSynchronize(c->stream));
     RC_TRY(c->prof_collect());
     c->stats.extension_rays = npix;
