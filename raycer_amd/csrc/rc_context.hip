@@ -181,8 +181,12 @@ int rc_download(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     return RC_OK;
 }
 
+void* rc_small_place(rc_ctx* c, SmallResult which) {
+    return c->stage + 2 * kStageChunk + size_t(which) * kSmallBytes;
+}
+
 int rc_small(rc_ctx* c, hipStream_t st, SmallResult which, const void* src, size_t bytes, const void** host) {
-    uint8_t* p = c->stage + 2 * kStageChunk + size_t(which) * kSmallBytes;
+    void* p = rc_small_place(c, which);
     RC_TRY_HIP(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, st));
     *host = p;
     return RC_OK;

@@ -269,6 +269,7 @@ int rc_download(rc_ctx* c, void* dst, const void* src, size_t bytes);
 // synchronisation of st.
 enum SmallResult { SMALL_COUNTERS, SMALL_TONEMAP, SMALL_TOTALS, SMALL_CACHE, SMALL_LOSS, SMALL_RESULTS };
 constexpr size_t kSmallBytes = 256, kStageChunk = size_t(2) << 20;
+void* rc_small_place(rc_ctx* c, SmallResult which);  // the place itself: kernels may write it
 int rc_small(rc_ctx* c, hipStream_t st, SmallResult which, const void* src, size_t bytes, const void** host);
 
 int rc_validate_cfg(const rc_render_cfg* cfg, const char* fn);

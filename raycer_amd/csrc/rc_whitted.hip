@@ -27,7 +27,6 @@
 // or shadow rays would outgrow their buffers is processed in halves (depth
 // first), so memory stays bounded for any glossy sample count.
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <chrono>
@@ -167,9 +166,9 @@ struct Counts {
 };
 constexpr uint32_t kDecReflect = 1u, kDecTransmit = 2u, kDecAO = 4u;
 struct Outs {
-    const uint32_t* oc;
-    const uint32_t* os;
-    const uint32_t* oa;
+    Counts cnt;              // the level's counts
+    const uint32_t* blocks;  // 3 x nblocks: where each block's children, shadow rays and AO rays start
+    uint32_t nblocks;
     rc_ray* crays;
     float4* cA;
     float4* cB;
@@ -324,6 +323,79 @@ __global__ __launch_bounds__(kBlock) void k_wt_count(WParams P, uint32_t level, 
     C.dec[i] = make_uint4(uint32_t(mask), uint32_t(mask >> 32), flags, 0u);
 }
 
+// Offsets of a range of nodes' rays, in node order: each block of kBlock nodes
+// sums its three counts (k_wt_sums), one block scans the sums and leaves the
+// totals where the host reads them (k_wt_scan), and k_wt_write adds the prefix
+// inside its block.  Two small launches where three device-wide scans and
+// three reads of their ends took nine, 57 us of a level of 2 M nodes (the frame
+// of 640 x 361, 4 samples and 2 x 2 of everything 8.75 ms with those, 8.3 with
+// these).  Bound by their launches and the 12 bytes per node.
+__global__ __launch_bounds__(kBlock) void k_wt_sums(uint32_t base, uint32_t n, Counts C, uint32_t* __restrict__ blocks) {
+    __shared__ uint32_t part[3][kBlock / 64];
+    const uint32_t r = blockIdx.x * kBlock + threadIdx.x, i = base + r;
+    uint32_t v[3] = {0u, 0u, 0u};
+    if (r < n) {
+        v[0] = C.nc[i];
+        v[1] = C.ns[i];
+        v[2] = C.na[i];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
+        if ((threadIdx.x & 63u) == 0) part[q][threadIdx.x >> 6] = v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        uint32_t t = 0;
+        for (int w = 0; w < kBlock / 64; ++w) t += part[threadIdx.x][w];
+        blocks[threadIdx.x * gridDim.x + blockIdx.x] = t;
+    }
+}
+
+// Exclusive scan of v over the BLOCK threads of a block; total: their sum.
+// scratch: BLOCK / 64 words, free again on return.
+template <int BLOCK>
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* scratch, uint32_t& total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+#pragma unroll
+    for (uint32_t o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) scratch[wave] = x;
+    __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+    for (uint32_t w = 0; w < BLOCK / 64; ++w) {
+        before += w < wave ? scratch[w] : 0u;
+        total += scratch[w];
+    }
+    __syncthreads();
+    return before + x - v;
+}
+
+constexpr int kScanBlock = 1024;
+__global__ __launch_bounds__(kScanBlock) void k_wt_scan(uint32_t nblocks, uint32_t* __restrict__ blocks,
+                                                        uint32_t* __restrict__ totals) {
+    __shared__ uint32_t scratch[kScanBlock / 64];
+    const uint32_t per = (nblocks + kScanBlock - 1) / kScanBlock;
+    const uint32_t lo = min(threadIdx.x * per, nblocks), hi = min(lo + per, nblocks);
+    for (int q = 0; q < 3; ++q) {
+        uint32_t* b = blocks + size_t(q) * nblocks;
+        uint32_t sum = 0, total;
+        for (uint32_t j = lo; j < hi; ++j) sum += b[j];
+        uint32_t off = block_scan<kScanBlock>(sum, scratch, total);
+        for (uint32_t j = lo; j < hi; ++j) {
+            const uint32_t c = b[j];
+            b[j] = off;
+            off += c;
+        }
+        if (threadIdx.x == 0) totals[q] = total;
+    }
+}
+
 // The node's terms, children, shadow rays and AO rays, placed at the scanned
 // offsets (relative to the first node of the range).
 __global__ __launch_bounds__(kBlock) void k_wt_write(WParams P, uint32_t level, uint32_t base, uint32_t n, LevelIn in,
@@ -331,9 +403,19 @@ __global__ __launch_bounds__(kBlock) void k_wt_write(WParams P, uint32_t level, 
                                                      const DevMaterial* __restrict__ mats,
                                                      const WMaterial* __restrict__ wm, const WLight* __restrict__ lights,
                                                      const uint4* __restrict__ dec, Outs O) {
+    __shared__ uint32_t scratch[kBlock / 64];
     const uint32_t r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n) return;
     const uint32_t i = base + r;
+    uint32_t off[3];  // of the node's children, shadow rays and AO rays
+    {
+        const uint32_t* cnt[3] = {O.cnt.nc, O.cnt.ns, O.cnt.na};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            uint32_t total;
+            off[q] = O.blocks[q * O.nblocks + blockIdx.x] + block_scan<kBlock>(r < n ? cnt[q][i] : 0u, scratch, total);
+        }
+    }
+    if (r >= n) return;
     const float4 A = in.A[i];
     const uint32_t slot = __float_as_uint(A.w);
     float3 w = f3(A);
@@ -395,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void k_wt_write(WParams P, uint32_t level, 
                 const uint32_t sb = __float_as_uint(M.b.w);
                 float R, T;
                 reflect_transmit(M, g, R, T);
-                uint32_t co = O.oc[i] - O.oc[base];
+                uint32_t co = off[0];
                 // calculateReflectedColor (Raytracer.cpp:160-226)
                 if (D.z & kDecReflect) {
                     float3 rd = normalize3(g.d + (2.0f * -dot3(g.d, g.n)) * g.n);
@@ -479,7 +561,7 @@ __global__ __launch_bounds__(kBlock) void k_wt_write(WParams P, uint32_t level, 
                     const uint64_t perm = node_perm(P, slot, g.key, kPurposeAO);
                     const uint32_t an = P.ao_n;
                     const float3 val = mul3(w, amb) * (1.0f / float(an * an));
-                    uint32_t ao = O.oa[i] - O.oa[base];
+                    uint32_t ao = off[2];
                     for (uint32_t y = 0; y < an; ++y)
                         for (uint32_t x = 0; x < an; ++x) {
                             const uint32_t s = y * an + x;
@@ -496,7 +578,7 @@ __global__ __launch_bounds__(kBlock) void k_wt_write(WParams P, uint32_t level, 
                 // directional, point and spot lights with their shadow rays
                 // (calculateShadowAmount, Raytracer.cpp:496-597)
                 const uint64_t mask = uint64_t(D.x) | (uint64_t(D.y) << 32);
-                uint32_t so = O.os[i] - O.os[base];
+                uint32_t so = off[1];
                 for (uint32_t li = 0; li < P.nlights; ++li) {
                     if (!((mask >> li) & 1ull)) continue;
                     const WLight L = lights[li];
@@ -563,11 +645,6 @@ __global__ __launch_bounds__(kBlock) void k_wt_sum(uint32_t n, const float4* __r
     L[s] = make_float4(l.x + acc.x, l.y + acc.y, l.z + acc.z, l.w);
 }
 
-__global__ void k_wt_total(const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ off, uint32_t last,
-                           uint32_t* __restrict__ out) {
-    *out = off[last] + cnt[last];
-}
-
 __global__ void k_wt_root(uint32_t n, uint32_t* __restrict__ keys, float4* __restrict__ B) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
@@ -580,11 +657,11 @@ __global__ void k_wt_root(uint32_t n, uint32_t* __restrict__ keys, float4* __res
 // ---------------------------------------------------------------- host side
 struct WhittedBufs {
     struct Level {
-        DevBuf rays, A, B, keys, hits, nc, ns, na, oc, os, oa, dec, contrib;
+        DevBuf rays, A, B, keys, hits, nc, ns, na, dec, contrib;
         size_t cap = 0;
     };
     std::vector<Level> levels;
-    DevBuf srays, sval, socc, arays, aval, ahits, scan_tmp, totals, lights, mats;
+    DevBuf srays, sval, socc, arays, aval, ahits, blocks, lights, mats;
     size_t scap = 0, acap = 0;
 };
 
@@ -592,10 +669,10 @@ void rc_whitted_release(rc_ctx* c) {
     if (!c || !c->whitted) return;
     WhittedBufs* W = c->whitted;
     for (auto& L : W->levels) {
-        DevBuf* b[] = {&L.rays, &L.A, &L.B, &L.keys, &L.hits, &L.nc, &L.ns, &L.na, &L.oc, &L.os, &L.oa, &L.dec, &L.contrib};
+        DevBuf* b[] = {&L.rays, &L.A, &L.B, &L.keys, &L.hits, &L.nc, &L.ns, &L.na, &L.dec, &L.contrib};
         for (DevBuf* d : b) d->release();
     }
-    DevBuf* b[] = {&W->srays, &W->sval, &W->socc, &W->arays, &W->aval, &W->ahits, &W->scan_tmp, &W->totals,
+    DevBuf* b[] = {&W->srays, &W->sval, &W->socc, &W->arays, &W->aval, &W->ahits, &W->blocks,
                    &W->lights, &W->mats};
     for (DevBuf* d : b) d->release();
     delete W;
@@ -613,9 +690,6 @@ int ensure_level(WhittedBufs::Level& L, size_t cap) {
     RC_TRY(L.nc.ensure(cap * sizeof(uint32_t)));
     RC_TRY(L.ns.ensure(cap * sizeof(uint32_t)));
     RC_TRY(L.na.ensure(cap * sizeof(uint32_t)));
-    RC_TRY(L.oc.ensure(cap * sizeof(uint32_t)));
-    RC_TRY(L.os.ensure(cap * sizeof(uint32_t)));
-    RC_TRY(L.oa.ensure(cap * sizeof(uint32_t)));
     RC_TRY(L.dec.ensure(cap * sizeof(uint4)));
     RC_TRY(L.contrib.ensure(cap * sizeof(float4)));
     L.cap = std::max(L.cap, cap);
@@ -633,14 +707,6 @@ struct Run {
     uint32_t nlev;  // levels in use: maxRayIterations + 1
     uint64_t ext_rays = 0, shadow_rays = 0;
 
-    int scan(const uint32_t* in, uint32_t* out, uint32_t n) {
-        size_t bytes = 0;
-        RC_TRY_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, in, out, n, c->stream));
-        RC_TRY(W->scan_tmp.ensure(std::max<size_t>(bytes, 256)));
-        RC_TRY_HIP(hipcub::DeviceScan::ExclusiveSum(W->scan_tmp.p, bytes, in, out, n, c->stream));
-        return RC_OK;
-    }
-
     LevelIn level_in(uint32_t k) {
         WhittedBufs::Level& Lv = W->levels[k];
         return LevelIn{Lv.rays.as<rc_ray>(), Lv.A.as<float4>(), Lv.B.as<float4>(), Lv.keys.as<uint32_t>(),
@@ -652,33 +718,32 @@ struct Run {
         WhittedBufs::Level& Lv = W->levels[k];
         RC_TRY(rc_launch_trace(c, s, false, Lv.rays.as<rc_ray>(), nullptr, n, Lv.hits.as<rc_hit>(), nullptr));
         ext_rays += n;
-        Counts C{Lv.nc.as<uint32_t>(), Lv.ns.as<uint32_t>(), Lv.na.as<uint32_t>(), Lv.dec.as<uint4>()};
+        const Counts C = level_counts(k);
         k_wt_count<<<(n + kBlock - 1) / kBlock, kBlock, 0, c->stream>>>(P, k, n, level_in(k), s->shade, s->mats, wm,
                                                                        wl, C);
         RC_TRY_HIP(hipGetLastError());
         return RC_OK;
     }
 
+    Counts level_counts(uint32_t k) {
+        WhittedBufs::Level& Lv = W->levels[k];
+        return Counts{Lv.nc.as<uint32_t>(), Lv.ns.as<uint32_t>(), Lv.na.as<uint32_t>(), Lv.dec.as<uint4>()};
+    }
+
     // children, shadow rays and AO rays of nodes [base, base + n) of level k
     int totals(uint32_t k, uint32_t base, uint32_t n, uint32_t out[3]) {
-        WhittedBufs::Level& Lv = W->levels[k];
-        const uint32_t* cnt[3] = {Lv.nc.as<uint32_t>(), Lv.ns.as<uint32_t>(), Lv.na.as<uint32_t>()};
-        uint32_t* off[3] = {Lv.oc.as<uint32_t>(), Lv.os.as<uint32_t>(), Lv.oa.as<uint32_t>()};
-        uint32_t* dev = W->totals.as<uint32_t>();
-        for (int q = 0; q < 3; ++q) {
-            RC_TRY(scan(cnt[q] + base, off[q] + base, n));
-            k_wt_total<<<1, 1, 0, c->stream>>>(cnt[q], off[q], base + n - 1, dev + q);
-        }
+        const uint32_t nb = (n + kBlock - 1) / kBlock;
+        RC_TRY(W->blocks.ensure(3 * size_t(nb) * sizeof(uint32_t)));
+        k_wt_sums<<<nb, kBlock, 0, c->stream>>>(base, n, level_counts(k), W->blocks.as<uint32_t>());
+        uint32_t* host = static_cast<uint32_t*>(rc_small_place(c, SMALL_TOTALS));
+        k_wt_scan<<<1, kScanBlock, 0, c->stream>>>(nb, W->blocks.as<uint32_t>(), host);
         RC_TRY_HIP(hipGetLastError());
-        const void* host = nullptr;
-        RC_TRY(rc_small(c, c->stream, SMALL_TOTALS, dev, 3 * sizeof(uint32_t), &host));
         RC_TRY_HIP(hipStreamSynchronize(c->stream));
         std::memcpy(out, host, 3 * sizeof(uint32_t));
         return RC_OK;
     }
 
-    // Offsets are scanned over [base, base + n) only, so the write kernel
-    // subtracts the range's first offset (zero by construction).
+    // The block offsets are those of [base, base + n), from zero.
     int process(uint32_t k, uint32_t base, uint32_t n) {
         if (n == 0) return RC_OK;
         uint32_t tot[3];
@@ -693,9 +758,9 @@ struct Run {
         }
         WhittedBufs::Level& Lv = W->levels[k];
         Outs O{};
-        O.oc = Lv.oc.as<uint32_t>();
-        O.os = Lv.os.as<uint32_t>();
-        O.oa = Lv.oa.as<uint32_t>();
+        O.cnt = level_counts(k);
+        O.blocks = W->blocks.as<uint32_t>();
+        O.nblocks = (n + kBlock - 1) / kBlock;
         if (k + 1 < nlev) {
             WhittedBufs::Level& Nx = W->levels[k + 1];
             O.crays = Nx.rays.as<rc_ray>();
@@ -849,7 +914,13 @@ extern "C" int rc_raytrace(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_ca
     const uint32_t spp_pass = pass_samples(c->tuning, P.npix, cfg->spp, kWhittedPassPaths);
     const size_t n0max = size_t(P.npix) * spp_pass;
     if (n0max > 0x7fffffffull) return rc_host_fail(RC_ERR_INVALID, "rc_raytrace: pass too large");
-    const size_t cap = std::max<size_t>(2 * n0max, size_t(1) << 20);
+    // Room for four rays of every kind per camera ray (2 x 2 samples) while
+    // that stays within what the largest pass gets anyway: a level that does
+    // not fit is traced in halves, each with launches and a tail of its own
+    // (640 x 361, 4 samples, 2 x 2 reflections, occlusion and light samples:
+    // 8.3 ms with room for two, 6.8 with this).
+    const size_t cap = std::max<size_t>(2 * n0max, std::min<size_t>(2 * kWhittedPassPaths,
+                                                                    std::max<size_t>(5 * n0max, size_t(1) << 20)));
     if (W->levels.size() < run.nlev) W->levels.resize(run.nlev);  // grow only: DevBuf frees nothing by itself
     RC_TRY(ensure_level(W->levels[0], n0max));
     for (uint32_t k = 1; k < run.nlev; ++k) RC_TRY(ensure_level(W->levels[k], cap));
@@ -860,7 +931,6 @@ extern "C" int rc_raytrace(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_ca
     RC_TRY(W->arays.ensure(cap * sizeof(rc_ray)));
     RC_TRY(W->aval.ensure(cap * sizeof(float4)));
     RC_TRY(W->ahits.ensure(cap * sizeof(rc_hit)));
-    RC_TRY(W->totals.ensure(4 * sizeof(uint32_t)));
     RC_TRY(c->fb.slotL.ensure(n0max * sizeof(float4)));
     RC_TRY(c->fb.slotW.ensure(n0max * sizeof(float)));
     RC_TRY(c->fb.ovf_list.ensure(cap * sizeof(uint32_t)));
