@@ -43,7 +43,7 @@ struct DevCounters {
     rcd::SpillCount spill;         // its total: rays whose stack outgrew its rows, over every launch since the last reset
     unsigned long long park_total; // traversals parked for the resume kernel since the last reset
     uint32_t ovf_count;            // rays listed for the next deep-stack launch
-    uint32_t queue_count[4];   // wavefront queue sizes (ping, pong, shadow, scratch)
+    uint32_t queue_count[5];   // sizes of the path queues (three, in turn) and the shadow queues (two, in turn)
     uint32_t park_count[2];    // traversals parked in the two park regions (ping-pong between phases)
     uint32_t error;
 };

@@ -215,17 +215,23 @@ __device__ __forceinline__ float camera_ray(const PassParams& P, uint32_t slot, 
     return w;
 }
 
+// Counters of the queues of vertex k: its paths', their continuations', and
+// its shadow rays'.  Those of vertex k + 1 that vertex k does not use are
+// cleared by its extension kernel, so no launch of its own clears them.
+__host__ __device__ __forceinline__ uint32_t path_queue(uint32_t k) { return k % 3u; }
+__host__ __device__ __forceinline__ uint32_t shadow_queue(uint32_t k) { return 3u + (k & 1u); }
+__device__ __forceinline__ void start_queues(DevCounters* ctr, uint32_t n) {
+    for (uint32_t q = 1; q < 5; ++q) ctr->queue_count[q] = 0;
+    ctr->queue_count[path_queue(0)] = n;
+}
+
 // The pass's camera rays, path states, zeroed slot radiance and weights.
 __global__ __launch_bounds__(kBlock) void k_camera(PassParams P, rc_ray* __restrict__ rays, float4* __restrict__ st,
                                                    float4* __restrict__ L, float* __restrict__ W,
                                                    DevCounters* __restrict__ ctr) {
     uint32_t n = P.npix * P.spp_pass;
     uint32_t slot = blockIdx.x * kBlock + threadIdx.x;
-    if (slot == 0) {
-        ctr->queue_count[0] = n;
-        ctr->queue_count[1] = 0;
-        ctr->queue_count[2] = 0;
-    }
+    if (slot == 0) start_queues(ctr, n);
     if (slot >= n) return;
     float4 r0, r1;
     const float w = camera_ray(P, slot, r0, r1);
@@ -253,11 +259,7 @@ __global__ __launch_bounds__(kBlock) void k_camera(PassParams P, rc_ray* __restr
 #endif
 // Start of a pass whose camera bounce makes its own rays (RC_FUSED_CAMERA):
 // the camera queue holds all n slots.
-__global__ void k_pass_start(DevCounters* ctr, uint32_t n) {
-    ctr->queue_count[0] = n;
-    ctr->queue_count[1] = 0;
-    ctr->queue_count[2] = 0;
-}
+__global__ void k_pass_start(DevCounters* ctr, uint32_t n) { start_queues(ctr, n); }
 
 // RC_PARK_KEEP > 0: a wave whose budget is spent keeps traversing while at
 // least RC_PARK_KEEP of its lanes still are (up to twice the budget), so
@@ -493,8 +495,8 @@ __device__ __forceinline__ void emit_vertex(const PassParams& P, uint32_t k, con
         st_stream(ro + 1, make_float4(O.newd.x, O.newd.y, O.newd.z, __builtin_inff()));
         st_stream(&st_out[pos], make_float4(O.thr.x, O.thr.y, O.thr.z, __uint_as_float(slot)));
     }
-    uint32_t spos = BLOCK ? block_append<BLOCK>(O.shadow, &ctr->queue_count[2], append_scratch)
-                          : wave_append(O.shadow, &ctr->queue_count[2]);
+    uint32_t spos = BLOCK ? block_append<BLOCK>(O.shadow, &ctr->queue_count[shadow_queue(k)], append_scratch)
+                          : wave_append(O.shadow, &ctr->queue_count[shadow_queue(k)]);
     if (O.shadow) {
         float4* ro = reinterpret_cast<float4*>(srays + spos);
         st_stream(ro, make_float4(O.so.x, O.so.y, O.so.z, 0.0f));
@@ -557,6 +559,10 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_extend_shade(
     __shared__ uint32_t append_scratch[BLOCK / 64 + 1];
     __shared__ uint4 top[4 * kTopNodes];
     const uint32_t n = ctr->queue_count[cin];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctr->queue_count[path_queue(k + 2)] = 0;
+        ctr->queue_count[shadow_queue(k + 1)] = 0;
+    }
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
     const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, P.stack_limit, gstack, &ctr->spill);
@@ -778,10 +784,10 @@ __global__ __launch_bounds__(BLOCK, kMinWaves<DEC64>) void k_shadow(const NodeT*
                                                        const float4* __restrict__ scontrib, float4* __restrict__ L,
                                                        uint32_t* __restrict__ ovf_list,
     uint32_t* __restrict__ gstack, DevCounters* __restrict__ ctr,
-                                                       uint8_t* __restrict__ occ_out, int stack_limit) {
+                                                       uint8_t* __restrict__ occ_out, int stack_limit, uint32_t queue) {
     __shared__ uint32_t stack[kLdsStack * BLOCK];
     __shared__ uint4 top[4 * kTopNodes];
-    const uint32_t n = ctr->queue_count[2];
+    const uint32_t n = ctr->queue_count[queue];
     if (blockIdx.x * uint32_t(BLOCK) >= n) return;
     const uint32_t ntop = load_top(nodes, top);
     const StackMem M = stack_mem(stack, threadIdx.x, BLOCK, stack_limit, gstack, &ctr->spill);
@@ -961,10 +967,10 @@ __global__ void k_cache_reset(uint32_t* counters, uint32_t which) {
     if (which) counters[kCcSamples] = 0;
 }
 
-// Zeroes the queue the next shade writes, the shadow queue and the overflow list.
-__global__ void k_prep(DevCounters* ctr, uint32_t cout) {
-    ctr->queue_count[cout] = 0;
-    ctr->queue_count[2] = 0;
+// Before an extension pass: the overflow list, the spill slots and both park
+// regions are free.  Not launched where a bounce can use none of them (4.6 us
+// each: 37 of the 520 us of a box frame's 256 x 256, 16 samples, 8 vertices).
+__global__ void k_prep(DevCounters* ctr) {
     ctr->ovf_count = 0;
     ctr->spill.claimed = 0;
     ctr->park_count[0] = 0;
@@ -1164,12 +1170,13 @@ struct ShadowArgs {
     DevCounters* ctr;
     uint8_t* occ_out;
     int stack_limit;
+    uint32_t queue;
 };
 
 template <bool COUNT, bool DEC64, int BLOCK>
 void shadow_t(const ShadowArgs& a, uint32_t n, hipStream_t st) {
     k_shadow<COUNT, DEC64, BLOCK><<<(n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(
-        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit);
+        a.s->nodes, tri_array<DEC64>(a.s), a.srays, a.scontrib, a.L, a.ovf, a.gstack, a.ctr, a.occ_out, a.stack_limit, a.queue);
 }
 
 template <bool COUNT, bool DEC64>
@@ -1438,12 +1445,13 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
         float4* sin_ = sa;
         float4* sout = sb;
         for (uint32_t k = 0; k < cfg->max_path_length; ++k) {
-            uint32_t cin = k & 1u, cout = cin ^ 1u;
-            k_prep<<<1, 1, 0, st>>>(ctr, cout);
+            const uint32_t cin = path_queue(k), cout = path_queue(k + 1);
             if (timed) RC_TRY(c->prof_begin(&ev));
             const bool camb = RC_FUSED_CAMERA && k == 0;
             ParkIO PK = regions[0];
             PK.steps = camb || n < min_rays ? 0u : c->tuning.park_steps;
+            const bool spills = rc_may_spill(s, P.stack_limit);
+            if (spills || PK.steps) k_prep<<<1, 1, 0, st>>>(ctr);
             ExtendArgs ea{P, k, s, rin, sin_, rout, sout, srays, scontrib, L, ovf, deep.deep_stack, ctr, cin, cout, CI, W, PK};
             launch_extend(ea, n, st, c->counting, camb, c->hit_fp64, shape.ext_block);
             if (PK.steps)
@@ -1463,9 +1471,9 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
                 // at the cache vertex the shadow results are kept for the training records
                 const bool nee_fix = CI.cache_vertex && k == CI.cache_vertex;
                 uint8_t* occ_out = nee_fix ? socc : nullptr;
-                k_reset_ovf<<<1, 1, 0, st>>>(ctr);
+                if (spills) k_reset_ovf<<<1, 1, 0, st>>>(ctr);
                 if (timed) RC_TRY(c->prof_begin(&ev));
-                ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit};
+                ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit, shadow_queue(k)};
                 launch_shadow(sa_, n, st, c->counting, c->hit_fp64, shape.shadow_block);
                 if (timed) RC_TRY(c->prof_end(ev, PK_SHADOW));
                 deep.any = true;
