@@ -324,8 +324,8 @@ __global__ __launch_bounds__(kBlock) void k_wt_count(WParams P, uint32_t level, 
 }
 
 // Offsets of a range of nodes' rays, in node order: each block of kBlock nodes
-// sums its three counts (k_wt_sums), one block scans the sums and leaves the
-// totals where the host reads them (k_wt_scan), and k_wt_write adds the prefix
+// sums its three counts (k_wt_sums), one block per count scans the sums and leaves
+// the total where the host reads it (k_wt_scan), and k_wt_write adds the prefix
 // inside its block.  Two small launches where three device-wide scans and
 // three reads of their ends took nine, 57 us of a level of 2 M nodes (the frame
 // of 640 x 361, 4 samples and 2 x 2 of everything 8.75 ms with those, 8.3 with
@@ -382,18 +382,17 @@ __global__ __launch_bounds__(kScanBlock) void k_wt_scan(uint32_t nblocks, uint32
     __shared__ uint32_t scratch[kScanBlock / 64];
     const uint32_t per = (nblocks + kScanBlock - 1) / kScanBlock;
     const uint32_t lo = min(threadIdx.x * per, nblocks), hi = min(lo + per, nblocks);
-    for (int q = 0; q < 3; ++q) {
-        uint32_t* b = blocks + size_t(q) * nblocks;
-        uint32_t sum = 0, total;
-        for (uint32_t j = lo; j < hi; ++j) sum += b[j];
-        uint32_t off = block_scan<kScanBlock>(sum, scratch, total);
-        for (uint32_t j = lo; j < hi; ++j) {
-            const uint32_t c = b[j];
-            b[j] = off;
-            off += c;
-        }
-        if (threadIdx.x == 0) totals[q] = total;
+    const uint32_t q = blockIdx.x;  // one block per count
+    uint32_t* b = blocks + size_t(q) * nblocks;
+    uint32_t sum = 0, total;
+    for (uint32_t j = lo; j < hi; ++j) sum += b[j];
+    uint32_t off = block_scan<kScanBlock>(sum, scratch, total);
+    for (uint32_t j = lo; j < hi; ++j) {
+        const uint32_t c = b[j];
+        b[j] = off;
+        off += c;
     }
+    if (threadIdx.x == 0) totals[q] = total;
 }
 
 // The node's terms, children, shadow rays and AO rays, placed at the scanned
@@ -736,7 +735,7 @@ struct Run {
         RC_TRY(W->blocks.ensure(3 * size_t(nb) * sizeof(uint32_t)));
         k_wt_sums<<<nb, kBlock, 0, c->stream>>>(base, n, level_counts(k), W->blocks.as<uint32_t>());
         uint32_t* host = static_cast<uint32_t*>(rc_small_place(c, SMALL_TOTALS));
-        k_wt_scan<<<1, kScanBlock, 0, c->stream>>>(nb, W->blocks.as<uint32_t>(), host);
+        k_wt_scan<<<3, kScanBlock, 0, c->stream>>>(nb, W->blocks.as<uint32_t>(), host);
         RC_TRY_HIP(hipGetLastError());
         RC_TRY_HIP(hipStreamSynchronize(c->stream));
         std::memcpy(out, host, 3 * sizeof(uint32_t));
