@@ -140,7 +140,7 @@ struct PassParams {
     float3 sky, sun, sun_e;
     uint64_t seed;
     uint32_t has_sun;
-    int stack_limit;  // on-chip traversal stack entries before the deep-stack kernel
+    int stack_limit;  // on-chip traversal stack entries before a stack goes on in global memory
 };
 
 // The pixel and sample a pass's queue slot traces.
@@ -507,8 +507,8 @@ __device__ __forceinline__ void emit_vertex(const PassParams& P, uint32_t k, con
 }
 
 // Extend + shade: closest-hit traversal of queue entry i and, in the same
-// thread, the shading of its hit.  A ray whose traversal stack outgrows LDS is
-// listed for the deep-stack kernel and shaded afterwards by k_shade_listed.
+// thread, the shading of its hit.  A ray whose stack outgrows its rows and the
+// spill slots is listed for the deep-stack kernel and shaded afterwards by k_shade_listed.
 // CAM: the camera bounce of a pass, whose entry i is camera slot i: the
 // thread makes the ray itself (k_camera's work) instead of loading it, writes
 // the slot's weight and zeroed radiance, and stores the ray and state only
