@@ -145,15 +145,17 @@ inline bool rc_may_spill(const rc_scene* s, int rows) {
     return int(s->stack_need) > rows - (rcd::kRegStack == 0 ? 1 : 0);  // row 0: the end marker
 }
 
-// Whether a launch over at most `rays` rays may list some for the deep-stack
-// kernel: one whose rays may outgrow their rows, unless each finds a spill slot
-// and its whole stack fits in it (a block of at least rows - 2 rows, end
-// markers among them, adds its length).  An empty launch costs about 5 us: it
-// and what follows it are left out of queries of few rays and of small scenes.
-inline bool rc_may_list(const rc_scene* s, int rows, size_t rays) {
+// Whether a launch that makes at most `walks` traversals may list some for the
+// deep-stack kernel: one whose rays may outgrow their rows, unless each finds a
+// spill slot and its whole stack fits in it (a block of at least rows - 2 rows,
+// end markers among them, adds its length).  Every traversal that spills claims
+// a slot of its own, also where one thread makes several.  An empty launch
+// costs about 5 us: it and what follows it are left out of queries of few rays
+// and of small scenes.
+inline bool rc_may_list(const rc_scene* s, int rows, size_t walks) {
     if (!rc_may_spill(s, rows)) return false;
     const int marks = std::max(1, rcd::kRegStack), held = rows - 2 - marks;
-    if (rays > size_t(rcd::kDeepThreads) || rows < rcd::kSpillRows || held < 1) return true;
+    if (walks > size_t(rcd::kDeepThreads) || rows < rcd::kSpillRows || held < 1) return true;
     const uint32_t need = s->stack_need, blocks = (need + uint32_t(held) - 1) / uint32_t(held);
     return need + blocks * uint32_t(marks + 1) > uint32_t(rcd::kDeepStack);
 }

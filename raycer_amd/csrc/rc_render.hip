@@ -1419,9 +1419,10 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
         const uint32_t n = npix * this_pass;
         const uint32_t grid_n = (n + kBlock - 1) / kBlock;
         deep.n_bound = n;
-        const bool listed = rc_may_list(s, P.stack_limit, n);
         hipEvent_t ev = nullptr;
         if (whole_paths) {
+            // a path's lane walks an extension and a shadow ray per vertex
+            const bool listed = rc_may_list(s, P.stack_limit, size_t(n) * cfg->max_path_length * (P.has_sun ? 2 : 1));
             if (rc_may_spill(s, P.stack_limit)) k_reset_ovf<<<1, 1, 0, st>>>(ctr);
             if (timed) RC_TRY(c->prof_begin(&ev));
             (c->hit_fp64 ? launch_paths<true> : launch_paths<false>)(P, s, L, W, ovf, deep.deep_stack, ctr, n, listed, st);
@@ -1432,6 +1433,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
             RC_TRY_HIP(hipGetLastError());
             continue;
         }
+        const bool listed = rc_may_list(s, P.stack_limit, n);
         if (CI.cache_vertex) k_cache_reset<<<1, 1, 0, st>>>(CI.counters, 0);
         if (RC_FUSED_CAMERA) {
             k_pass_start<<<1, 1, 0, st>>>(ctr, n);

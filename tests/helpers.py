@@ -3,6 +3,7 @@ import math
 
 import numpy as np
 
+import raycer_amd as ra
 from raycer_amd import api
 
 
@@ -167,3 +168,15 @@ def check_closest(gpu_hits, vertices, rays, diag, max_listed=0.01, rel_t=1e-5, f
         err = np.abs(gpu_hits["t"][agree] - t_o[agree]) / t_o[agree]
         assert err.max() <= rel_t
     return mismatch.sum(), listed.sum()
+
+
+def overlapping_scene(ntri=2000, seed=4):
+    """Triangles that each span a good part of the unit cube, seen from its
+    middle: every ray enters many boxes at once, so its traversal stack is
+    deep, and few paths leave the cube."""
+    sd = ra.generate_scene(ra.scene_params(api.RCH_SCENE_SOUP, seed=seed, tri_count=ntri))
+    r = np.random.default_rng(seed)
+    v = r.random((ntri, 1, 3)) + r.uniform(-0.3, 0.3, (ntri, 3, 3))
+    sd.vertices = np.ascontiguousarray(v.reshape(ntri, 9), np.float32)
+    sd.desc.camera = api.Camera((0.5, 0.5, 0.5), 10.0, 130.0, 0.0, 90.0)
+    return sd

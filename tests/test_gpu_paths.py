@@ -6,6 +6,7 @@ import pytest
 
 import raycer_amd as ra
 from raycer_amd import api
+from tests.helpers import overlapping_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +57,36 @@ def test_whole_paths_equal_the_queues(ctx, decision, scenes, name, width, height
         film.close()
     for r in results[1:]:
         assert r == results[0]
+
+
+# At most as many paths as there are spill slots (2,048), but many more
+# traversals that outgrow their rows than that: each claims a slot of its own,
+# so paths are listed and walked again.  A frame of other samples comes first,
+# so a path that is left out would show that frame's radiance.
+@pytest.mark.parametrize("width,height", [(45, 45), (32, 64)])
+@pytest.mark.parametrize("limit", [4, 5, 6, 7])
+def test_small_passes_lose_no_listed_path(ctx, decision, width, height, limit):
+    sd = overlapping_scene()
+    nodes, ordered, _, _ = ra.build_bvh(sd.vertices)
+    s = ctx.upload(sd, nodes, ordered)
+    cfg = api.RenderCfg.from_buffer_copy(sd.desc.cfg)
+    cfg.width, cfg.height, cfg.spp, cfg.max_path_length, cfg.rr_start = width, height, 1, 8, 0
+    other = api.RenderCfg.from_buffer_copy(cfg)
+    other.frame = cfg.frame + 5
+    film = ctx.film(width, height)
+    results = []
+    try:
+        for rows in (1, limit):
+            ctx.set_tuning(stack_limit=1)
+            ctx.render(s, film, sd.desc.camera, other)
+            film.clear()
+            ctx.set_tuning(stack_limit=rows)
+            ctx.render(s, film, sd.desc.camera, cfg)
+            st = ctx.stats()
+            results.append((film.sums().tobytes(), st.extension_rays, st.shadow_rays))
+    finally:
+        ctx.set_tuning()
+        film.close()
+        s.close()
+    assert results[1] == results[0]
+    assert st.overflow_rays > 2048
