@@ -1778,7 +1778,7 @@ extern "C" int rc_raycast_phong(rc_ctx* c, const rc_scene* s, const rc_camera* c
                                                     FB.deep_stack.as<uint32_t>(), c->counters, rows)
     if (c->hit_fp64) RC_PHONG(true, false, grid, kBlock);
     else RC_PHONG(false, false, grid, kBlock);
-    if (rc_may_list(s, rows, npix)) {
+    if (rc_may_list(s, rows, 2 * size_t(npix))) {  // a pixel's primary and shadow ray
         if (c->hit_fp64) RC_PHONG(true, true, kDeepThreads / 64, 64);
         else RC_PHONG(false, true, kDeepThreads / 64, 64);
     }

@@ -6,6 +6,7 @@ import pytest
 
 import raycer_amd as ra
 from raycer_amd import api
+from tests.helpers import overlapping_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,26 @@ def test_phong_variants_agree(ctx, decision, width, height):
         for b in blocks:
             b.close()
         s.close()
+
+
+# At most as many pixels as there are spill slots (2,048), but more traversals
+# than that outgrow their rows: a pixel's primary and shadow ray each claim a
+# slot, so pixels are listed and walked again.  The light is at the camera:
+# most shadow rays reach it, and a pixel left out would lack its light.
+@pytest.mark.parametrize("width,height", [(45, 45), (32, 64)])
+@pytest.mark.parametrize("limit", [4, 5])
+def test_phong_loses_no_listed_pixel(ctx, decision, width, height, limit):
+    sd = overlapping_scene()
+    nodes, ordered, _, _ = ra.build_bvh(sd.vertices)
+    s = ctx.upload(sd, nodes, ordered)
+    light = api.PointLight((0.5, 0.5, 0.5), (1.0, 1.0, 1.0), 1.0, 1000.0, 1.0, (1.0, 1.0, 1.0), 0.1)
+    args = (s, sd.desc.camera, width, height, 7, sd.desc.cfg.ray_start_offset, light)
+    try:
+        ctx.set_tuning(stack_limit=1)
+        ref = [x.tobytes() for x in ctx.raycast_phong(*args)]
+        ctx.set_tuning(stack_limit=limit)
+        assert [x.tobytes() for x in ctx.raycast_phong(*args)] == ref
+    finally:
+        ctx.set_tuning()
+        s.close()
+    assert (np.frombuffer(ref[2], np.float32)[::4] > 0.1).mean() > 0.5  # ambient alone gives less
