@@ -136,7 +136,7 @@ struct rc_scene {
     size_t nmat = 0;
     float bmin[3], bmax[3];
     uint32_t depth = 0;
-    uint32_t stack_need = 0;  // the most entries a traversal's stack can hold
+    uint32_t stack_need = 0;  // a bound of a traversal's stack: all of a node's slots but one, per level
     size_t bytes = 0;
 };
 

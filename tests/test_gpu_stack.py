@@ -78,3 +78,41 @@ def test_spilled_and_parked_traversals_give_the_same_image(ctx, decision, soup, 
         ctx.set_tuning()
         film.close()
     assert sums[1] == sums[0] and sums[2] == sums[0]
+
+
+@pytest.mark.parametrize("ntri", [3, 10, 50, 100])
+def test_unused_slots_seen_from_afar(ctx, decision, ntri):
+    """From afar a node's quantized bounds round together, so its unused slots
+    are entered and pushed too; a ray without numbers enters every box.  The
+    rows that only the used slots would need are not enough then.  The trees
+    have at most six levels, whose 18 entries the default 19 rows hold."""
+    sd = ra.generate_scene(ra.scene_params(api.RCH_SCENE_SOUP, seed=3, tri_count=ntri))
+    r = np.random.default_rng(ntri)
+    v = np.array([3.0, 2.0, 1.0]) + 1e-3 * (r.random((ntri, 1, 3)) + r.uniform(-0.2, 0.2, (ntri, 3, 3)))
+    sd.vertices = np.ascontiguousarray(v.reshape(ntri, 9), np.float32)
+    nodes, ordered, _, _ = ra.build_bvh(sd.vertices)
+    s = ctx.upload(sd, nodes, ordered)
+    n = 4096
+    target = v.reshape(-1, 3)[r.integers(0, 3 * ntri, n)]
+    d = r.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    rays = api.make_rays((target - d * r.uniform(1e2, 2e4, (n, 1))).astype(np.float32), d.astype(np.float32))
+    f = rays.view(np.float32).reshape(n, 8)
+    f[5::64, 0:3] = np.nan
+    f[6::64, 4:7] = np.nan
+    f[7::64, 0] = np.inf
+    try:
+        results = {}
+        for rows in (0, *range(1, 19), 1):
+            ctx.set_tuning(stack_limit=rows)
+            hits = ctx.trace_closest(s, rays)
+            outgrown = ctx.stats().overflow_rays
+            results[rows] = hits.tobytes(), np.asarray(ctx.trace_any(s, rays)).tobytes(), outgrown
+    finally:
+        ctx.set_tuning()
+        s.close()
+    assert results[0][2] == 0
+    for rows, got in results.items():
+        assert got[:2] == results[0][:2], rows
+    if ntri <= 10:  # one node with an unused slot: two entries if only the used ones counted
+        assert results[2][2] > 0
