@@ -637,6 +637,18 @@ __device__ __forceinline__ void order2(double& a, double& b) {
 #ifndef RC_LEAF_POSTPONE_ANY
 #define RC_LEAF_POSTPONE_ANY 32
 #endif
+// RC_PACKET_CAMERA = 1: the camera bounce's waves (one pixel's samples each,
+// with pixel-major slots) traverse as packets (traverse_packet); 0 (the
+// default): each lane on its own, as the other bounces.  On the 2M-triangle
+// terrain at 64 samples per pass the packets made the camera bounce 1.6 ms
+// slower (12.5 against 14.1 ms): the union of a pixel's 64 traversals costs
+// more visits than the per-lane traversal's leaf postponing and culling.
+#ifndef RC_PACKET_CAMERA
+#define RC_PACKET_CAMERA 0
+#endif
+// Whether every traversal of the build spills a stack that is full
+// (stack_spill); traverse_inline and traverse_packet list its ray instead.
+constexpr bool kSpillsInPlace = RC_QNODE ? !RC_PACKET_CAMERA : RC_TRAV_IFIF != 0;
 // Stack entries of the if-if traversal: an interior child's record index, or
 // a leaf tagged with kLeafTag, its triangle count (0..31) in bits 26..30 and
 // its first triangle (< 2^26) below.  The upload guarantees both: scenes hold
@@ -1142,8 +1154,7 @@ __device__ __forceinline__ TraceResult traverse(const NodeT* __restrict__ nodes,
 // of the extra visits, so the hits are those of traverse().  Children are
 // taken nearest first by the first active lane's entry distances.  The
 // stack entries are wave-uniform; each lane keeps its own copy in its LDS
-// row (entry k at stack[k * stride]), up to max_depth entries, beyond which
-// every lane of the wave reports an overflow.  Every active lane of the wave
+// rows, and when they are full every lane of the wave reports an overflow.  Every active lane of the wave
 // calls this (the loop and its exit are uniform).
 template <bool COUNT>
 __device__ __forceinline__ TraceResult traverse_packet(const QNode* __restrict__ nodes,

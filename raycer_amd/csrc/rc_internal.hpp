@@ -155,7 +155,7 @@ inline bool rc_may_spill(const rc_scene* s, int rows) {
 inline bool rc_may_list(const rc_scene* s, int rows, size_t walks) {
     if (!rc_may_spill(s, rows)) return false;
     const int marks = std::max(1, rcd::kRegStack), held = rows - 2 - marks;
-    if (walks > size_t(rcd::kDeepThreads) || rows < rcd::kSpillRows || held < 1) return true;
+    if (!rcd::kSpillsInPlace || walks > size_t(rcd::kDeepThreads) || rows < rcd::kSpillRows || held < 1) return true;
     const uint32_t need = s->stack_need, blocks = (need + uint32_t(held) - 1) / uint32_t(held);
     return need + blocks * uint32_t(marks + 1) > uint32_t(rcd::kDeepStack);
 }

@@ -245,15 +245,6 @@ __global__ __launch_bounds__(kBlock) void k_camera(PassParams P, rc_ray* __restr
 
 // 1: the camera bounce makes its camera rays in the extension kernel (no
 // k_camera pass over the queues).
-// RC_PACKET_CAMERA = 1: the camera bounce's waves (one pixel's samples each,
-// with pixel-major slots) traverse as packets (traverse_packet); 0 (the
-// default): each lane on its own, as the other bounces.  On the 2M-triangle
-// terrain at 64 samples per pass the packets made the camera bounce 1.6 ms
-// slower (12.5 against 14.1 ms): the union of a pixel's 64 traversals costs
-// more visits than the per-lane traversal's leaf postponing and culling.
-#ifndef RC_PACKET_CAMERA
-#define RC_PACKET_CAMERA 0
-#endif
 #ifndef RC_FUSED_CAMERA
 #define RC_FUSED_CAMERA 1
 #endif
