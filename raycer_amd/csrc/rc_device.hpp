@@ -888,6 +888,13 @@ __device__ __forceinline__ void node_hits(const Trav<DEC64>& S, const NodeT* __r
 #endif
 }
 
+// The sort key of a child not entered, above every entry distance that is.
+constexpr float kNotEntered = 2.0f;
+// A packet's distance of an entered child: its first lane's, or 1 (past
+// everything) where that lane's own ray enters later, not at all or has no
+// distance, so that the child still sorts before those no lane enters.
+__host__ __device__ inline float packet_entry(float t) { return fminf(t, 1.0f); }
+
 // The children of a visited node in H: the nearest (ANY without RC_ANY_SORT:
 // the first) becomes S.cur, the others go on the stack farthest first; with
 // none S.cur is popped.  False when the stack would outgrow its rows (SPILL:
@@ -900,11 +907,10 @@ __device__ __forceinline__ bool take_children(Trav<DEC64>& S, Hits& H, const Sta
     const bool two = b01 || b23 || (a01 && a23);
     const bool three = (b01 && a23) || (b23 && a01), four = b01 && b23;
     if (SORT) {
-        // a child not entered sorts last: 2.0f, above every entry distance
-        double k0 = __hiloint2double(h[0] ? __float_as_int(H.t[0]) : 0x40000000, int(e0));
-        double k1 = __hiloint2double(h[1] ? __float_as_int(H.t[1]) : 0x40000000, int(e1));
-        double k2 = __hiloint2double(h[2] ? __float_as_int(H.t[2]) : 0x40000000, int(e2));
-        double k3 = __hiloint2double(h[3] ? __float_as_int(H.t[3]) : 0x40000000, int(e3));
+        double k0 = __hiloint2double(__float_as_int(h[0] ? H.t[0] : kNotEntered), int(e0));
+        double k1 = __hiloint2double(__float_as_int(h[1] ? H.t[1] : kNotEntered), int(e1));
+        double k2 = __hiloint2double(__float_as_int(h[2] ? H.t[2] : kNotEntered), int(e2));
+        double k3 = __hiloint2double(__float_as_int(h[3] ? H.t[3] : kNotEntered), int(e3));
         order2(k0, k1);
         order2(k2, k3);
         order2(k0, k2);
@@ -1174,7 +1180,7 @@ __device__ __forceinline__ TraceResult traverse_packet(const QNode* __restrict__
 #pragma unroll
             for (int k = 0; k < kWidth; ++k) {
                 H.h[k] = __ballot(H.h[k]) != 0;
-                H.t[k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(H.t[k])));
+                H.t[k] = packet_entry(__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(H.t[k]))));
                 H.e[k] = __builtin_amdgcn_readfirstlane(H.e[k]);
             }
             if (!take_children<true, false>(S, H, M)) {
