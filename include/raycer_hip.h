@@ -174,8 +174,8 @@ typedef struct rc_point_light {
  * as keep a pass within 2^26 paths, 2^21 for rc_raytrace; else 1..64), grid
  * limit of the ray-query kernels in blocks per CU, the traversal stack
  * entries held on chip (registers and LDS) before a ray's stack goes on in
- * global memory: in one of a launch's 2048 spill slots or, when they are
- * taken or the limit is below 4, by a second walk in the deep-stack kernel
+ * global memory: in one of a launch's spill slots or, when they are taken
+ * or the limit is below 4, by a second walk in the deep-stack kernel
  * (0, the default: all the build holds, 19; 1..20: fewer, which sends more
  * rays that way and changes no result), and the
  * traversal steps a path tracer's extension ray takes in the first kernel

@@ -99,7 +99,7 @@ struct alignas(16) DevMaterial {
 
 constexpr uint32_t kNoHit = 0x7fffffffu;
 constexpr int kDeepStack = 256;  // words of a stack in global memory: a spill slot, a lane of the deep-stack kernel
-constexpr int kDeepThreads = 2048;  // such stacks of a launch
+constexpr int kDeepThreads = 2048;  // lanes of the deep-stack kernel
 
 // Traversal stack of one lane: the top kRegStack entries in registers, deeper
 // ones in LDS laid out [depth][lane] so a wave's accesses hit 64 distinct
@@ -387,12 +387,13 @@ constexpr float kTieWindow = 4.0f / 16777216.0f;
 // lanes, row r of the lane at byte offset base + r * stride (base = 4 * lane <
 // stride).  end is the offset past row `limit` of every lane (uniform), so a
 // lane whose next free row is at p may push m entries exactly when
-// p + m * stride < end.  spill: the launch's kDeepThreads stacks in global
+// p + m * stride < end.  spill: the launch's count->slots stacks in global
 // memory, handed out by count->claimed, for lanes whose rows are full; null:
 // none.
 struct SpillCount {
     unsigned long long total;  // rays whose stack outgrew its rows
     uint32_t claimed;          // stacks the launch's rays asked for
+    uint32_t slots;            // those there are, at most kMaxSpillSlots (here, not an argument: it costs no register)
 };
 struct StackMem {
     uint32_t* array;
@@ -410,6 +411,13 @@ __device__ __forceinline__ StackMem stack_mem(uint32_t* array, uint32_t lane, in
 // Rows the three entries of a node visit need above a stack just spilled: with
 // fewer nothing is spilled.
 constexpr int kSpillRows = 4;
+// A traversal's spilled stack in one word: 1 + its slot above, the blocks of
+// rows in it below.  A block takes the lane's rows and their number, so there
+// are at most kDeepStack / (kSpillRows + 1) of them.
+constexpr int kSpillBlockBits = 6;
+constexpr uint32_t kSpillMask = 0x007fffffu, kSpillBlocks = (1u << kSpillBlockBits) - 1u;
+constexpr uint32_t kMaxSpillSlots = kSpillMask >> kSpillBlockBits;  // 131,071
+static_assert(kDeepStack / (kSpillRows + 1) <= int(kSpillBlocks), "a slot's blocks do not fit their bits");
 
 // The stack's registers and the offset of its next free row.
 struct Stack {
@@ -699,7 +707,6 @@ __device__ __forceinline__ uint32_t load_top(const N* __restrict__ nodes, uint4*
     }
 }
 
-constexpr uint32_t kSpillMask = 0x007fffffu;
 template <bool DEC64>
 __device__ __forceinline__ float trav_scale(const Trav<DEC64>& S) {
     return __uint_as_float(S.scale_spill & ~kSpillMask);
@@ -713,35 +720,35 @@ __device__ __forceinline__ void trav_cull(Trav<DEC64>& S) {
 
 // A stack whose rows are full: they move to a slot of global memory and the
 // lane goes on with empty rows; when those are used up the rows come back
-// (stack_reload).  The word in scale_spill: 1 + the slot in bits 9.., the
-// slot's words in use below (each block of rows is followed by its length);
-// 0 while nothing was spilled.  False when the launch's slots are all taken,
-// the slot is full or the rows are too few: then the deep-stack kernel walks
-// the ray again.  Before, it walked all of them: the few rays that outgrow the
-// rows are a launch's longest, and walked twice, the second time alone on the
-// chip.  An any-hit query over 777,777 segments in 200,000 random triangles
-// takes 446 us against 514; the loop itself pays nothing (the word lies in
-// unused bits and is looked at where a traversal ends or finds no room).
+// (stack_reload).  The word in scale_spill names the slot and counts its
+// blocks; 0 while nothing was spilled.  False when the launch's slots are all
+// taken, the slot is full or the rows are too few: then the deep-stack kernel
+// walks the ray again.  Before, it walked all of them: the few rays that
+// outgrow the rows are a launch's longest, and walked twice, the second time
+// alone on the chip.  An any-hit query over 777,777 segments in 200,000 random
+// triangles takes 446 us against 514; the loop itself pays nothing (the word
+// lies in unused bits and is looked at where a traversal ends or finds no room).
 template <bool DEC64>
 __device__ __forceinline__ bool stack_spill(Trav<DEC64>& S, const StackMem& M) {
     if (!M.spill || M.end < (kSpillRows + 1) * M.stride) return false;
     uint32_t w = S.scale_spill & kSpillMask;
     if (w == 0) {
         const uint32_t slot = atomicAdd(&M.count->claimed, 1u);
-        if (slot >= uint32_t(kDeepThreads)) return false;
+        if (slot >= M.count->slots) return false;
         atomicAdd(&M.count->total, 1ull);
-        w = (slot + 1u) << 9;
+        w = (slot + 1u) << kSpillBlockBits;
     }
     const uint32_t rows = uint32_t(S.stack.p - M.base) / uint32_t(M.stride);
-    uint32_t used = w & 511u;
-    if (used + rows + 1u > uint32_t(kDeepStack)) {
+    const uint32_t words = uint32_t(M.end) / uint32_t(M.stride);  // of a block
+    const uint32_t at = (w & kSpillBlocks) * words;
+    if (at + words > uint32_t(kDeepStack)) {
         atomicAdd(&M.count->total, ~0ull);  // the deep-stack kernel counts it
         return false;
     }
-    uint32_t* q = M.spill + ((w >> 9) - 1u) * uint32_t(kDeepStack) + used;
+    uint32_t* q = M.spill + (((w >> kSpillBlockBits) - 1u) * uint32_t(kDeepStack) + at);
+    q[words - 1u] = rows;
     for (int p = M.base; p < S.stack.p; p += M.stride) *q++ = M.at(p);
-    *q = rows;
-    S.scale_spill = (S.scale_spill & ~kSpillMask) | (w + rows + 1u);
+    S.scale_spill = (S.scale_spill & ~kSpillMask) | (w + 1u);
     M.at(M.base) = kEmptyChild;  // below the register entries
     S.stack.p = M.base + M.stride;
     return true;
@@ -752,13 +759,14 @@ __device__ __forceinline__ bool stack_spill(Trav<DEC64>& S, const StackMem& M) {
 template <bool DEC64>
 __device__ __forceinline__ bool stack_reload(Trav<DEC64>& S, const StackMem& M) {
     const uint32_t w = S.scale_spill & kSpillMask;
-    if ((w & 511u) == 0) return false;
-    const uint32_t* q = M.spill + ((w >> 9) - 1u) * uint32_t(kDeepStack) + (w & 511u) - 1u;
-    const uint32_t rows = *q;
-    q -= rows;
+    if ((w & kSpillBlocks) == 0) return false;
+    const uint32_t words = uint32_t(M.end) / uint32_t(M.stride);
+    const uint32_t* q =
+        M.spill + (((w >> kSpillBlockBits) - 1u) * uint32_t(kDeepStack) + ((w & kSpillBlocks) - 1u) * words);
+    const uint32_t rows = q[words - 1u];
     S.stack.p = M.base;
     for (uint32_t r = 0; r < rows; ++r, S.stack.p += M.stride) M.at(S.stack.p) = q[r];
-    S.scale_spill -= rows + 1u;
+    S.scale_spill -= 1u;
 #pragma unroll
     for (int k = 0; k < kRegStack; ++k) stack_pop(S.stack, M);  // refills the registers
     S.cur = stack_pop(S.stack, M);

@@ -145,19 +145,32 @@ inline bool rc_may_spill(const rc_scene* s, int rows) {
     return int(s->stack_need) > rows - (rcd::kRegStack == 0 ? 1 : 0);  // row 0: the end marker
 }
 
+// Spill slots of a launch over at most `rays` rays (or paths): one for every 16
+// of them (64 bytes a ray), as many as a traversal's word can name.  Where
+// boxes overlap heavily one ray in 200 and more outgrows its rows, and a ray
+// (or whole path) without a slot is walked again by 2,048 lanes, alone on the
+// chip.  100,000 triangles within 0.05 of points of the unit cube, 2,048 slots
+// against these: 256 x 256 pixels, 4 samples, 5 vertices 3.0 and 1.2 ms, 64
+// vertices 85 and 22; 1280 x 720, 16 samples, 5 vertices 44.4 and 22.8 (40.5
+// with 16,383 slots); Whitted at 1080p 4.4 and 2.7.
+constexpr uint32_t kMinSpillSlots = 2048;
+inline uint32_t rc_spill_slots(size_t rays) {
+    return uint32_t(std::min<size_t>(std::max<size_t>(rays / 16, kMinSpillSlots), rcd::kMaxSpillSlots));
+}
+
 // Whether a launch that makes at most `walks` traversals may list some for the
-// deep-stack kernel: one whose rays may outgrow their rows, unless each finds a
-// spill slot and its whole stack fits in it (a block of at least rows - 2 rows,
-// end markers among them, adds its length).  Every traversal that spills claims
-// a slot of its own, also where one thread makes several.  An empty launch
-// costs about 5 us: it and what follows it are left out of queries of few rays
-// and of small scenes.
-inline bool rc_may_list(const rc_scene* s, int rows, size_t walks) {
+// deep-stack kernel: one whose rays may outgrow their rows, unless each finds
+// one of the `slots` spill slots and its whole stack fits in it (a block of
+// rows + 1 words holds at least rows - 2 rows, end markers among them).  Every
+// traversal that spills claims a slot of its own, also where one thread makes
+// several.  An empty launch costs about 5 us: it and what follows it are left
+// out of queries of few rays and of small scenes.
+inline bool rc_may_list(const rc_scene* s, int rows, size_t walks, uint32_t slots) {
     if (!rc_may_spill(s, rows)) return false;
     const int marks = std::max(1, rcd::kRegStack), held = rows - 2 - marks;
-    if (!rcd::kSpillsInPlace || walks > size_t(rcd::kDeepThreads) || rows < rcd::kSpillRows || held < 1) return true;
+    if (!rcd::kSpillsInPlace || walks > size_t(slots) || rows < rcd::kSpillRows || held < 1) return true;
     const uint32_t need = s->stack_need, blocks = (need + uint32_t(held) - 1) / uint32_t(held);
-    return need + blocks * uint32_t(marks + 1) > uint32_t(rcd::kDeepStack);
+    return blocks * uint32_t(rows + 1) > uint32_t(rcd::kDeepStack);
 }
 
 // The triangle records a traversal with the given decision reads.
@@ -195,6 +208,7 @@ struct TraceLaunch {
     uint8_t* occ = nullptr;
     uint32_t* ovf_list = nullptr;
     uint32_t* deep_stack = nullptr;
+    uint32_t spill_slots = 0;  // those deep_stack has room for
     DevCounters* ctr = nullptr;
     hipStream_t stream = nullptr;
     int max_depth = rcd::kLdsStack;  // on-chip stack entries
@@ -202,7 +216,8 @@ struct TraceLaunch {
     bool counting = false;
     bool dec64 = false;
 };
-size_t rc_deep_stack_bytes();
+// What the deep-stack kernel and `slots` spill slots need.
+size_t rc_deep_stack_bytes(uint32_t slots);
 // Clears the overflow count and launches the traversal kernel.
 int rc_launch_trace_with(const TraceLaunch& L);
 // The deep-stack kernel over the rays the last traversal launch (of at most

@@ -22,7 +22,7 @@ namespace {
 constexpr size_t kNoAllocMaxRays = size_t(1) << 20;  // rays per call
 constexpr size_t kCounterBytes = 256;                // DevCounters, padded
 constexpr size_t kOvfBytes = kNoAllocMaxRays * sizeof(uint32_t);
-constexpr size_t kDeepBytes = size_t(2048) * rcd::kDeepStack * sizeof(uint32_t);
+constexpr size_t kDeepBytes = size_t(kMinSpillSlots) * rcd::kDeepStack * sizeof(uint32_t);
 constexpr size_t kScratchBytes = kCounterBytes + kOvfBytes + kDeepBytes;  // 6.25 MiB
 static_assert(sizeof(DevCounters) <= kCounterBytes, "counters do not fit their slot");
 
@@ -37,7 +37,7 @@ static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 // Looks up this device's copy of the scratch array (the device is current).
 int rc_noalloc_setup(int device) {
     if (device < 0 || device >= kMaxDevices) return rc_host_fail(RC_ERR_INVALID, "rc_create: device index too large");
-    if (rc_deep_stack_bytes() > kDeepBytes)
+    if (rc_deep_stack_bytes(kMinSpillSlots) > kDeepBytes)
         return rc_host_fail(RC_ERR_INVALID, "rc_create: the deep stack outgrew the allocation-free scratch");
     std::lock_guard<std::mutex> lock(g_mu);
     if (g_scratch[device]) return RC_OK;
@@ -74,6 +74,7 @@ extern "C" int rc_trace_closest_device_noalloc(rc_ctx* c, const rc_scene* s, con
     L.ctr = reinterpret_cast<DevCounters*>(p);
     L.ovf_list = reinterpret_cast<uint32_t*>(p + kCounterBytes);
     L.deep_stack = reinterpret_cast<uint32_t*>(p + kCounterBytes + kOvfBytes);
+    L.spill_slots = kMinSpillSlots;
     L.stream = c->stream;
     L.max_depth = c->stack_depth();
     L.max_blocks = uint32_t(c->cu_count) * c->tuning.blocks_per_cu;

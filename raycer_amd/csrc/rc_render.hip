@@ -961,18 +961,20 @@ __global__ void k_cache_reset(uint32_t* counters, uint32_t which) {
 // Before an extension pass: the overflow list, the spill slots and both park
 // regions are free.  Not launched where a bounce can use none of them (4.6 us
 // each: 37 of the 520 us of a box frame's 256 x 256, 16 samples, 8 vertices).
-__global__ void k_prep(DevCounters* ctr) {
+__global__ void k_prep(DevCounters* ctr, uint32_t slots) {
     ctr->ovf_count = 0;
     ctr->spill.claimed = 0;
+    ctr->spill.slots = slots;
     ctr->park_count[0] = 0;
     ctr->park_count[1] = 0;
 }
 
 // Before a shadow pass, or whole paths: the overflow list and the spill slots
 // are free.
-__global__ void k_reset_ovf(DevCounters* ctr) {
+__global__ void k_reset_ovf(DevCounters* ctr, uint32_t slots) {
     ctr->ovf_count = 0;
     ctr->spill.claimed = 0;
+    ctr->spill.slots = slots;
 }
 
 __device__ __forceinline__ void kahan(float& s, float& c, float v) {
@@ -1225,7 +1227,7 @@ int FrameBuffers::ensure(size_t npaths) {
     RC_TRY(slotL.ensure(npaths * sizeof(float4)));
     RC_TRY(slotW.ensure(npaths * sizeof(float)));
     RC_TRY(ovf_list.ensure(npaths * sizeof(uint32_t)));
-    RC_TRY(deep_stack.ensure(rc_deep_stack_bytes()));
+    RC_TRY(deep_stack.ensure(rc_deep_stack_bytes(rc_spill_slots(npaths))));
     // parked traversals: 1 / RC_PARK_DIV of the pass's paths at most
     RC_TRY(park.ensure(std::max<size_t>(npaths / RC_PARK_DIV, 256) * kParkWords * sizeof(uint32_t)));
     return RC_OK;
@@ -1351,7 +1353,9 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
     const uint32_t spp_pass = std::max(1u, std::min(shape.spp_pass, cfg->spp));
     const size_t npaths = size_t(npix) * spp_pass;
     if (npaths > 0x7fffffffull) return rc_host_fail(RC_ERR_INVALID, "rc_render: pass too large");
-    if (B.slotW.bytes < npaths * sizeof(float) || B.ovf_list.bytes < npaths * sizeof(uint32_t) || !B.counters)
+    const uint32_t slots = rc_spill_slots(npaths);
+    if (B.slotW.bytes < npaths * sizeof(float) || B.ovf_list.bytes < npaths * sizeof(uint32_t) ||
+        B.deep_stack.bytes < rc_deep_stack_bytes(slots) || !B.counters)
         return rc_host_fail(RC_ERR_INVALID, "rc_render: frame buffers are smaller than the pass");
     // park regions, sized for this pass (the resume kernels' grids cover a
     // region, and a frame far smaller than the buffers must not launch grids
@@ -1392,6 +1396,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
     deep.counting = c->counting;
     deep.dec64 = c->hit_fp64;
     deep.max_depth = P.stack_limit;
+    deep.spill_slots = slots;
     // whole paths in one kernel: node and triangle counts stay those of the
     // queues' kernels, and a budget other than the default asks for parking;
     // frames beside each other fill the gaps and the tails with queues (eight
@@ -1413,8 +1418,9 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
         hipEvent_t ev = nullptr;
         if (whole_paths) {
             // a path's lane walks an extension and a shadow ray per vertex
-            const bool listed = rc_may_list(s, P.stack_limit, size_t(n) * cfg->max_path_length * (P.has_sun ? 2 : 1));
-            if (rc_may_spill(s, P.stack_limit)) k_reset_ovf<<<1, 1, 0, st>>>(ctr);
+            const bool listed = rc_may_list(s, P.stack_limit, size_t(n) * cfg->max_path_length * (P.has_sun ? 2 : 1),
+                                            slots);
+            if (rc_may_spill(s, P.stack_limit)) k_reset_ovf<<<1, 1, 0, st>>>(ctr, slots);
             if (timed) RC_TRY(c->prof_begin(&ev));
             (c->hit_fp64 ? launch_paths<true> : launch_paths<false>)(P, s, L, W, ovf, deep.deep_stack, ctr, n, listed, st);
             if (timed) RC_TRY(c->prof_end(ev, PK_EXTEND));
@@ -1424,7 +1430,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
             RC_TRY_HIP(hipGetLastError());
             continue;
         }
-        const bool listed = rc_may_list(s, P.stack_limit, n);
+        const bool listed = rc_may_list(s, P.stack_limit, n, slots);
         if (CI.cache_vertex) k_cache_reset<<<1, 1, 0, st>>>(CI.counters, 0);
         if (RC_FUSED_CAMERA) {
             k_pass_start<<<1, 1, 0, st>>>(ctr, n);
@@ -1444,7 +1450,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
             ParkIO PK = regions[0];
             PK.steps = camb || n < min_rays ? 0u : c->tuning.park_steps;
             const bool spills = rc_may_spill(s, P.stack_limit);
-            if (spills || PK.steps) k_prep<<<1, 1, 0, st>>>(ctr);
+            if (spills || PK.steps) k_prep<<<1, 1, 0, st>>>(ctr, slots);
             ExtendArgs ea{P, k, s, rin, sin_, rout, sout, srays, scontrib, L, ovf, deep.deep_stack, ctr, cin, cout, CI, W, PK};
             launch_extend(ea, n, st, c->counting, camb, c->hit_fp64, shape.ext_block);
             if (PK.steps)
@@ -1464,7 +1470,7 @@ int rc_enqueue_frame(rc_ctx* c, FrameBuffers& B, hipStream_t st, const rc_scene*
                 // at the cache vertex the shadow results are kept for the training records
                 const bool nee_fix = CI.cache_vertex && k == CI.cache_vertex;
                 uint8_t* occ_out = nee_fix ? socc : nullptr;
-                if (spills) k_reset_ovf<<<1, 1, 0, st>>>(ctr);
+                if (spills) k_reset_ovf<<<1, 1, 0, st>>>(ctr, slots);
                 if (timed) RC_TRY(c->prof_begin(&ev));
                 ShadowArgs sa_{s, srays, scontrib, L, ovf, deep.deep_stack, ctr, occ_out, P.stack_limit, shadow_queue(k)};
                 launch_shadow(sa_, n, st, c->counting, c->hit_fp64, shape.shadow_block);
@@ -1759,7 +1765,8 @@ extern "C" int rc_raycast_phong(rc_ctx* c, const rc_scene* s, const rc_camera* c
     if (t_copy) t_d = FB.st_b.as<float>();
     if (rgba_copy) rgba_d = FB.slotL.as<float4>();
     const int rows = c->stack_depth();
-    if (rc_may_spill(s, rows)) k_reset_ovf<<<1, 1, 0, c->stream>>>(c->counters);
+    const uint32_t slots = rc_spill_slots(npix);
+    if (rc_may_spill(s, rows)) k_reset_ovf<<<1, 1, 0, c->stream>>>(c->counters, slots);
     hipEvent_t ev;
     RC_TRY(c->prof_begin(&ev));
     const uint32_t grid = uint32_t(std::min<size_t>(size_t((w + 31) / 32) * ((h + 7) / 8), size_t(1) << 23));
@@ -1769,7 +1776,7 @@ extern "C" int rc_raycast_phong(rc_ctx* c, const rc_scene* s, const rc_camera* c
                                                     FB.deep_stack.as<uint32_t>(), c->counters, rows)
     if (c->hit_fp64) RC_PHONG(true, false, grid, kBlock);
     else RC_PHONG(false, false, grid, kBlock);
-    if (rc_may_list(s, rows, 2 * size_t(npix))) {  // a pixel's primary and shadow ray
+    if (rc_may_list(s, rows, 2 * size_t(npix), slots)) {  // a pixel's primary and shadow ray
         if (c->hit_fp64) RC_PHONG(true, true, kDeepThreads / 64, 64);
         else RC_PHONG(false, true, kDeepThreads / 64, 64);
     }

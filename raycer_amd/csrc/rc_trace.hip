@@ -100,9 +100,10 @@ __global__ __launch_bounds__(64) void k_trace_deep(const NodeT* __restrict__ nod
     }
 }
 
-__global__ void k_reset_overflow(DevCounters* ctr) {
+__global__ void k_reset_overflow(DevCounters* ctr, uint32_t slots) {
     ctr->ovf_count = 0;
     ctr->spill.claimed = 0;
+    ctr->spill.slots = slots;
 }
 
 template <bool ANY, bool COUNT, bool DEC64>
@@ -133,12 +134,14 @@ void dispatch_deep(const TraceLaunch& L) {
 
 }  // namespace
 
-size_t rc_deep_stack_bytes() { return size_t(kDeepThreads) * kDeepStack * sizeof(uint32_t); }
+size_t rc_deep_stack_bytes(uint32_t slots) {
+    return std::max(size_t(kDeepThreads), size_t(slots)) * kDeepStack * sizeof(uint32_t);
+}
 
 int rc_launch_trace_with(const TraceLaunch& L) {
     if (L.n_bound == 0) return RC_OK;
     const uint32_t blocks = std::max(1u, std::min((L.n_bound + kBlock - 1) / kBlock, L.max_blocks));
-    if (rc_may_spill(L.scene, L.max_depth)) k_reset_overflow<<<1, 1, 0, L.stream>>>(L.ctr);
+    if (rc_may_spill(L.scene, L.max_depth)) k_reset_overflow<<<1, 1, 0, L.stream>>>(L.ctr, L.spill_slots);
     if (L.counting) {
         if (L.dec64) dispatch_trace<true, true>(L, blocks);
         else dispatch_trace<true, false>(L, blocks);
@@ -150,7 +153,7 @@ int rc_launch_trace_with(const TraceLaunch& L) {
 }
 
 int rc_launch_deep_with(const TraceLaunch& L) {
-    if (!rc_may_list(L.scene, L.max_depth, L.n_bound)) return RC_OK;
+    if (!rc_may_list(L.scene, L.max_depth, L.n_bound, L.spill_slots)) return RC_OK;
     if (L.counting) {
         if (L.dec64) dispatch_deep<true, true>(L);
         else dispatch_deep<true, false>(L);
@@ -174,6 +177,7 @@ TraceLaunch context_launch(rc_ctx* c, const rc_scene* s, bool any, const rc_ray*
     L.occ = occ;
     L.ovf_list = c->fb.ovf_list.as<uint32_t>();
     L.deep_stack = c->fb.deep_stack.as<uint32_t>();
+    L.spill_slots = rc_spill_slots(n_bound);
     L.ctr = c->counters;
     L.stream = c->stream;
     L.max_depth = c->stack_depth();
@@ -188,7 +192,7 @@ int rc_launch_trace(rc_ctx* c, const rc_scene* s, bool any, const rc_ray* rays, 
                     uint32_t n_bound, rc_hit* hits, uint8_t* occ) {
     if (n_bound == 0) return RC_OK;
     RC_TRY(c->fb.ovf_list.ensure(size_t(n_bound) * sizeof(uint32_t)));
-    RC_TRY(c->fb.deep_stack.ensure(rc_deep_stack_bytes()));
+    RC_TRY(c->fb.deep_stack.ensure(rc_deep_stack_bytes(rc_spill_slots(n_bound))));
     // one lane per ray up to cu_count * blocks_per_cu blocks; beyond that the
     // kernel's grid-stride loop takes over
     const TraceLaunch L = context_launch(c, s, any, rays, n_dev, n_bound, hits, occ);

@@ -933,7 +933,7 @@ extern "C" int rc_raytrace(rc_ctx* c, const rc_scene* s, rc_film* f, const rc_ca
     RC_TRY(c->fb.slotL.ensure(n0max * sizeof(float4)));
     RC_TRY(c->fb.slotW.ensure(n0max * sizeof(float)));
     RC_TRY(c->fb.ovf_list.ensure(cap * sizeof(uint32_t)));
-    RC_TRY(c->fb.deep_stack.ensure(rc_deep_stack_bytes()));
+    RC_TRY(c->fb.deep_stack.ensure(rc_deep_stack_bytes(rc_spill_slots(cap))));
     run.L = c->fb.slotL.as<float4>();
 
     for (uint32_t s0 = 0; s0 < cfg->spp; s0 += spp_pass) {

@@ -1,7 +1,7 @@
 """Traversal stacks that outgrow their on-chip rows.
 
 A lane whose rows are full moves them to a spill slot in global memory and
-goes on; when the launch's 2048 slots are taken the ray is walked again by the
+goes on; when the launch's slots (2048, or one for 16 rays) are taken the ray is walked again by the
 deep-stack kernel.  A limit below four rows spills nothing, so one row sends
 every ray that needs more to the deep-stack kernel: the general path, against
 which the others are compared bit for bit (the hit does not depend on where a
@@ -54,7 +54,26 @@ def test_spilled_stacks_give_the_same_hits(ctx, decision, soup, n, limit):
     print(f"{n} rays, {limit} rows: {outgrown} outgrew them ({all_rays} one row)")
     assert outgrown <= all_rays
     if n == 60000 and limit in (3, 4):
-        assert outgrown > 2048  # more than there are slots: both ways are taken
+        assert outgrown > n // 16  # more than there are slots: both ways are taken
+
+
+# As many slots as a traversal's word can name (131,071), and fewer.
+@pytest.mark.parametrize("n", [600_001, 2_200_000])
+@pytest.mark.parametrize("limit", [4, 5])
+def test_many_slots(ctx, decision, soup, n, limit):
+    sd, s = soup
+    rays = query_rays(sd, n)
+    results = []
+    try:
+        for rows in (0, limit):
+            ctx.set_tuning(stack_limit=rows)
+            hits = ctx.trace_closest(s, rays)
+            outgrown = ctx.stats().overflow_rays
+            results.append((hits.tobytes(), np.asarray(ctx.trace_any(s, rays)).tobytes()))
+    finally:
+        ctx.set_tuning()
+    assert results[1] == results[0]
+    assert outgrown > min(n // 16, 131071)
 
 
 @pytest.mark.parametrize("limit", [4, 6])

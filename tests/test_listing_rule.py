@@ -1,5 +1,5 @@
 """When the deep-stack kernel may be left out (rc_may_list), in every build: a
-traversal that spills finds room for at most 2,048 walks of a launch, one that
+traversal that spills finds room for as many walks as there are slots, one that
 does not spill lists each ray whose stack outgrows its rows.  The rule is
 compiled for the host and asked (no GPU)."""
 import os
@@ -17,7 +17,7 @@ int main() {
     for (unsigned need : {18u, 20u, 60u})
         for (size_t walks : {size_t(1), size_t(2048), size_t(2049)}) {
             s.stack_need = need;
-            std::printf("%d", int(rc_may_list(&s, 19, walks)));
+            std::printf("%d", int(rc_may_list(&s, 19, walks, kMinSpillSlots)));
         }
     std::printf("\\n");
 }
