@@ -672,8 +672,11 @@ __device__ __forceinline__ bool is_leaf(uint32_t e) { return int32_t(e) < -1; }
 // of two (so every product and comparison is the unscaled one) that puts the
 // scene's end of the ray, or tmax when that is nearer, below 1: clamping an
 // entry plane's FMA to [0, 1], which is free (a modifier), then takes the place
-// of the maximum with 0, and 1 stays an entry past everything.  The distances
-// reported are the triangle tests', unscaled.
+// of the maximum with 0, and 1 stays an entry past everything.  Past 2^126 no
+// power of two is small enough: the last of a float's distances end at
+// kFarthest, and a clamped entry plane there only lets boxes in that are
+// further away.  The distances reported are the triangle tests', unscaled.
+constexpr float kFarthest = 3.9999998f;  // the largest float, scaled by 2^-126
 template <bool DEC64>
 struct Trav {
     float3 o, d;
@@ -681,7 +684,7 @@ struct Trav {
     uint32_t scale_spill;  // bits of the power of two (trav_scale); its mantissa's: the spilled stack (stack_spill)
     float tmin;
     bool late;    // wave-uniform: some ray of the wave has a tmin > 0, entries are held against it
-    float cull;   // boxes entered beyond it are skipped (scaled, below 1)
+    float cull;   // boxes entered beyond it are skipped (scaled)
     typename BestT<DEC64>::T best;  // DEC64: the best hit's FP64 distance; else unused (R.t is it)
     TraceResult R;
     uint32_t cur;
@@ -715,7 +718,7 @@ __device__ __forceinline__ float trav_scale(const Trav<DEC64>& S) {
 // The cull distance for R.t (the best hit's, or tmax).
 template <bool DEC64>
 __device__ __forceinline__ void trav_cull(Trav<DEC64>& S) {
-    S.cull = fminf(cull_at<DEC64>(S.R.t) * trav_scale(S), 0.99999994f);
+    S.cull = fminf(cull_at<DEC64>(S.R.t) * trav_scale(S), kFarthest);
 }
 
 // A stack whose rows are full: they move to a slot of global memory and the
@@ -808,7 +811,7 @@ __device__ __forceinline__ void trav_begin(Trav<DEC64>& S, const NodeT* __restri
     S.R = TraceResult{tmax, 0.0f, 0.0f, kNoHit, false, 1.0f};
     const float3 inv = safe_inv(d);
     const float T0 = cull_at<DEC64>(tmax), exit = scene_exit(nodes, o, inv);
-    const float T = fminf(fmaxf(exit < T0 ? exit : T0, 1e-12f), 3e37f);
+    const float T = fminf(fmaxf(exit < T0 ? exit : T0, 1e-12f), 8e37f);  // below 2^126, the smallest scale's
     S.scale_spill = (253u << 23) - (__float_as_uint(T) & 0x7f800000u);  // 2^-k, 2^(k-1) <= T < 2^k
     S.inv = inv * trav_scale(S);
     trav_cull(S);
@@ -897,7 +900,7 @@ __device__ __forceinline__ void node_hits(const Trav<DEC64>& S, const NodeT* __r
 }
 
 // The sort key of a child not entered, above every entry distance that is.
-constexpr float kNotEntered = 2.0f;
+constexpr float kNotEntered = 4.0f;
 // A packet's distance of an entered child: its first lane's, or 1 (past
 // everything) where that lane's own ray enters later, not at all or has no
 // distance, so that the child still sorts before those no lane enters.

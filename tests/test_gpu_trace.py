@@ -266,3 +266,27 @@ def test_full_size_sphere_ground_ray_set(ctx, decision):
                                  max_listed=0.005 if not decision else 0.02, fp32=decision)
     print(f"full C2 ray set: {mism} mismatches, {listed} listed of {w * h}")
     s.close()
+
+
+# Distances up to the largest float: a square at 1e18 and slow rays (a
+# direction component below 1e-20 counts as 1e-20, so these are the longest a
+# triangle can be hit at).  The FP64 decision, as the FP32 test overflows.
+@pytest.mark.parametrize("speed", [5e-20, 2.2e-20, 1.2e-20, 1.05e-20])
+def test_hits_at_the_longest_distances(ctx, speed):
+    sd = ra.generate_scene(ra.scene_params(api.RCH_SCENE_SOUP, seed=3, tri_count=2))
+    square = np.array([[-1, -1, 1, 1, -1, 1, -1, 1, 1], [1, 1, 1, 1, -1, 1, -1, 1, 1]])
+    sd.vertices = np.ascontiguousarray(1e18 * square, np.float32)
+    s = ctx.upload(sd)
+    d = speed * np.array([[0.5, 0.55, 1.0], [0.6, -0.7, 1.0], [-0.9, 0.95, 1.0], [0.5, 0.5, -1.0]])
+    d[:, :2] = np.where(np.abs(d[:, :2]) < 1e-20, 0.0, d[:, :2])
+    rays = api.make_rays(np.zeros(3, np.float32), d.astype(np.float32))
+    ctx.set_hit_decision("fp64")
+    try:
+        hits = ctx.trace_closest(s, rays)
+        occ = np.asarray(ctx.trace_any(s, rays))
+    finally:
+        ctx.set_hit_decision("fp32")
+        s.close()
+    np.testing.assert_allclose(hits["t"][:3], 1e18 / rays["dir"][:3, 2].astype(np.float64), rtol=1e-6)
+    assert np.isinf(hits["t"][3])
+    assert occ.tolist() == [1, 1, 1, 0]
