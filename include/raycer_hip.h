@@ -499,7 +499,8 @@ int rc_autotune_batch(rc_ctx* ctx, const rc_scene* const* scenes, const rc_camer
                       size_t nscenes, const char* cache_path, uint32_t* spp_per_pass);
 /* Autotuner for rc_render_batch_tuned: per size class, the samples per pass
  * as rc_autotune_batch chooses them, then the block shapes (extension 128 or
- * 256, shadow 64, 128 or 256 threads) timed at those samples per pass; then,
+ * 256, shadow 64, 128 or 256 threads) timed at those samples per pass (with two
+ * scenes and more, all with the kernels that frames beside each other run); then,
  * for the whole batch, the branch count (1, 2, 4, 8) timed as relaunches of
  * the captured graph.  A candidate replaces the default only when it is 2%
  * faster.  Choices are read from and added to the JSON cache (keys

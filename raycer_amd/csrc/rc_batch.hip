@@ -302,8 +302,10 @@ extern "C" int rc_render_batch_tuned(rc_ctx* c, const rc_scene* const* scenes, r
 // rendered in full: with 1, 2, 4, ... 64 samples per pass (at most the frame's
 // spp and 2^25 paths per pass), then at the best of those with every block
 // shape.  A candidate must beat the incumbent by 2% (larger queues and
-// non-default shapes have to earn their place).  Then the whole batch is
-// timed as relaunches of its graph with 1, 2, 4 and 8 branches.
+// non-default shapes have to earn their place).  A plan for several branches
+// is timed with the kernels frames beside each other run: a frame alone traces
+// small passes as whole paths, where every block shape is the same.  Then the
+// whole batch is timed as relaunches of its graph with 1, 2, 4 and 8 branches.
 namespace {
 constexpr uint64_t kMaxPassPaths = 1ull << 25;
 
@@ -371,6 +373,8 @@ int tune(rc_ctx* c, const rc_scene* const* scenes, const rc_camera* cams, const 
     std::map<std::string, uint32_t> table;
     if (cache_path && *cache_path) table = read_tuning(cache_path);
     bool changed = false;
+    const std::string bkey = c->name + "/branches/" + std::to_string(n);
+    const bool concurrent = branches && n > 1 && !(table.count(bkey) && table[bkey] == 1);
     std::map<uint32_t, rc_batch_plan> chosen;  // class -> plan
     for (size_t i = 0; i < n; ++i) {
         const uint32_t cls = size_class(cfgs[i]);
@@ -399,6 +403,7 @@ int tune(rc_ctx* c, const rc_scene* const* scenes, const rc_camera* cams, const 
             for (uint32_t sp = 1; sp <= 64 && rc == RC_OK; sp *= 2) {
                 if (sp > 1 && (sp > cfgs[i].spp || px * sp > kMaxPassPaths)) break;
                 FrameShape sh;
+                sh.concurrent = concurrent;
                 sh.spp_pass = sp;
                 double ms = 1e300;
                 rc = time_frame(c, scenes[i], film, &cams[i], &cfgs[i], sh, &ms);
@@ -410,6 +415,7 @@ int tune(rc_ctx* c, const rc_scene* const* scenes, const rc_camera* cams, const 
         }
         if (shapes && !have_shape && rc == RC_OK) {
             FrameShape sh;
+            sh.concurrent = concurrent;
             sh.spp_pass = p.spp_per_pass;
             double best_ms = 1e300;
             rc = time_frame(c, scenes[i], film, &cams[i], &cfgs[i], sh, &best_ms);  // the default shape
@@ -440,7 +446,6 @@ int tune(rc_ctx* c, const rc_scene* const* scenes, const rc_camera* cams, const 
     for (size_t i = 0; i < n; ++i) plans[i] = chosen[size_class(cfgs[i])];
     if (branches) {
         *branches = 1;
-        const std::string bkey = c->name + "/branches/" + std::to_string(n);
         auto it = table.find(bkey);
         if (it != table.end()) {
             *branches = std::max(1u, std::min(it->second, kMaxBranches));

@@ -155,3 +155,25 @@ def test_branches_and_block_shapes_do_not_change_the_images(ctx):
             ctx.render_batch_tuned(hs, films, cams, cfgs, plans, 9)
     finally:
         close(ctx, scenes, films)
+
+
+def test_plans_are_tuned_on_the_kernels_a_batch_runs(ctx, tmp_path):
+    """Frames of several branches run the queues' kernels, whose block shapes a
+    plan chooses; a small frame by itself is traced as whole paths, without a
+    shadow launch.  The last frame the tuner times by itself tells which."""
+    scenes = load(ctx, [1, 28])
+    hs = [s for _, s in scenes]
+    cams = [sd.desc.camera for sd, _ in scenes]
+    cfgs = [sd.desc.cfg for sd, _ in scenes]
+    for c in cfgs:
+        c.width = c.height = 64
+        c.spp = 4
+    ctx.set_profiling(True)
+    try:
+        ctx.autotune_batch_plan(hs, cams, cfgs, tmp_path / "plan.json")
+        assert ctx.stats().shadow_launches > 0
+        ctx.autotune_batch(hs, cams, cfgs, tmp_path / "alone.json")  # one branch
+        assert ctx.stats().shadow_launches == 0
+    finally:
+        ctx.set_profiling(False)
+        close(ctx, scenes, [])
