@@ -193,6 +193,11 @@ typedef struct rc_tuning {
     uint32_t park_steps;
 } rc_tuning;
 
+/* The times are of kernels (profiling on).  Where one kernel does all of a
+ * frame - rc_raycast_phong, and rc_render's passes of at most 1,024 paths per
+ * compute unit - its whole time, shading and shadow rays included, is in
+ * extend_ms, and shadow_ms, shade_ms and shadow_launches leave it out; the ray
+ * counts hold its rays of both kinds. */
 typedef struct rc_stats {
     uint64_t extension_rays;     /* closest-hit rays traced by the last render */
     uint64_t shadow_rays;        /* any-hit rays traced by the last render */
@@ -201,7 +206,7 @@ typedef struct rc_stats {
     uint64_t tri_tests;          /* 48-byte triangle records tested (counting runs only) */
     uint64_t overflow_rays;      /* rays whose stack outgrew the on-chip entries, summed over all launches of the call */
     uint64_t extend_launches;
-    double extend_ms;            /* sum of closest-hit kernel durations (profiling on) */
+    double extend_ms;            /* sum of closest-hit kernel durations */
     double shadow_ms;
     double shade_ms;
     double other_ms;
