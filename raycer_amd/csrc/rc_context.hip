@@ -136,17 +136,19 @@ void* rc_mapped(void* p, size_t bytes, size_t align) {
     return mapped ? a.devicePointer : nullptr;
 }
 
-int rc_upload(rc_ctx* c, void* dst, const void* src, size_t bytes) {
+int rc_upload(rc_ctx* c, void* dst, const void* src, size_t bytes, bool wait) {
     if (bytes == 0) return RC_OK;
     if (!src) return rc_host_fail(RC_ERR_INVALID, "copy to the device: null array");
     if (bytes > kStageUpload || rc_known_memory(src)) {
         RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        if (wait) RC_TRY_HIP(hipStreamSynchronize(c->stream));
         return RC_OK;
     }
     RC_TRY_HIP(hipEventSynchronize(c->stage_ev[0]));
     std::memcpy(c->stage, src, bytes);
     RC_TRY_HIP(hipMemcpyAsync(dst, c->stage, bytes, hipMemcpyHostToDevice, c->stream));
-    RC_TRY_HIP(hipEventRecord(c->stage_ev[0], c->stream));
+    if (wait) RC_TRY_HIP(hipStreamSynchronize(c->stream));
+    else RC_TRY_HIP(hipEventRecord(c->stage_ev[0], c->stream));
     return RC_OK;
 }
 
@@ -160,6 +162,12 @@ int rc_download(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     if (rc_known_memory(dst)) {
         RC_TRY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
         RC_TRY_HIP(hipStreamSynchronize(c->stream));
+        return RC_OK;
+    }
+    if (bytes <= kStageChunk) {
+        RC_TRY_HIP(hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        RC_TRY_HIP(hipStreamSynchronize(c->stream));
+        std::memcpy(dst, c->stage, bytes);
         return RC_OK;
     }
     uint8_t* d = static_cast<uint8_t*>(dst);
@@ -916,9 +924,7 @@ extern "C" int rc_host_free(rc_ctx* c, void* p) {
 }
 extern "C" int rc_memcpy_h2d(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     RC_TRY(rc_check_ctx(c, "rc_memcpy_h2d"));
-    RC_TRY(rc_upload(c, dst, src, bytes));
-    RC_TRY_HIP(hipStreamSynchronize(c->stream));
-    return RC_OK;
+    return rc_upload(c, dst, src, bytes, true);
 }
 extern "C" int rc_memcpy_d2h(rc_ctx* c, void* dst, const void* src, size_t bytes) {
     RC_TRY(rc_check_ctx(c, "rc_memcpy_d2h"));

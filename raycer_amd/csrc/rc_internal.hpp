@@ -271,15 +271,18 @@ void* rc_mapped(void* p, size_t bytes, size_t align);
 // Copies between host arrays and the device, ordered on the context's stream,
 // through the context's page-locked chunks unless the array is page-locked (or
 // device memory) itself.  The upload returns when src may be changed (page-locked: when the
-// copy is queued); the download when dst holds the bytes.
-// The runtime's own copies of pageable arrays reach 17 GB/s down and 37 up and
-// pin what is between 64 KiB and 1 MiB for each call.  Down, the chunks overlap
-// the host's copy with the transfer: 31.6 MiB take 940 us against 1885, 4 MiB
-// 160 against 236, 256 KiB 28 against 115.  Up, the host's copy alone is as
-// slow as the runtime: kStageUpload bytes and less are staged (256 KiB: 25 us
-// against 62).
+// copy is queued), or with wait when it has ended; the download when dst holds
+// the bytes.
+// The runtime's own copies of pageable arrays reach 17 GB/s down and 37 up, and
+// a process's first few hundred between 16 KiB and 1 MiB take 23 to 115 us
+// each.  Down, the chunks overlap the host's copy with the transfer: 31.6 MiB
+// take 940 us against 1885, 4 MiB 160 against 246; what fits one chunk costs
+// what the runtime's later copies do (64 KiB 12 us, 256 KiB 20, 1 MiB 60) from
+// the first on.  Up, the host's copy alone is as slow as the runtime:
+// kStageUpload bytes and less are staged (64 KiB 11 us, 256 KiB 16).  A copy
+// that ends in a wait waits for the stream: an event after it adds 7 us.
 constexpr size_t kStageUpload = size_t(512) << 10;
-int rc_upload(rc_ctx* c, void* dst, const void* src, size_t bytes);
+int rc_upload(rc_ctx* c, void* dst, const void* src, size_t bytes, bool wait = false);
 int rc_download(rc_ctx* c, void* dst, const void* src, size_t bytes);
 // Queues a copy of a small device result (bytes <= kSmallBytes) to place
 // `which` of the page-locked small results; *host is valid after the next
